@@ -152,13 +152,52 @@ __global__ __launch_bounds__(1024) void k_scan_tiles(const uint32_t* __restrict_
 // Workgroup t scans the counts of cell tile t (empty tiles only write their
 // prefix), clears the counts it read and the tile's occupied flag; the last
 // workgroup writes the deleted bucket: off[C] = live count, off[C+1] = n.
-// (CUB DeviceScan::ExclusiveSum in pbf_counting_sort.cu:62-71.)  When
-// `stat` is given, the occupied tiles are counted into its statistics
-// copies (CTR_SCANTILES).
+// (CUB DeviceScan::ExclusiveSum in pbf_counting_sort.cu:62-71.)
+//
+// With the offsets of its tile in LDS, the workgroup also lists the work
+// items of the tile's runs (kEmit, no run straddles a tile) with one atomic
+// on the item counter:
+//   EMIT_SEARCH  each run of uw cells along x.  A run whose estimated 27-cell
+//                neighbourhood (9 rows of W+2 cells at the run's mean density)
+//                exceeds `budget` particles is split into narrower units, and a
+//                unit with more than kChunk own particles into several items
+//                that share its neighbourhood (item = (first cell, W | chunk
+//                << 6)).  Also counts the occupied tiles (CTR_SCANTILES).
+//   EMIT_FINAL   each run of uw final cells (nc = 1 << lgnc counters) holding
+//                at least kSparse particles, one item per kChunk of them.
+// Listed here, the counter takes one atomic per occupied tile (128 on the 1M
+// dam).  Listed by the wave that meets a run's first particle, as the reorder
+// and the regrouping's scatter did, it takes thousands, which one address
+// serialises: k_reorder took 101 us on the 1M dam and 756 us on the 8M double
+// dam at uw = 16, now 14 and 148; k_cur_scatter 22 and 338 us, now 15 and 97;
+// the two scans 18 us together, now 23.
+enum EmitMode : int { EMIT_NONE = 0, EMIT_SEARCH, EMIT_FINAL };
+struct EmitArgs {
+    uint32_t uw, lguw, budget;
+    uint2* units;
+    uint32_t* nunits;
+};
+
+// Calls item(first cell, W | chunk << 6) for the items of the search run of uw
+// cells starting at tile cell r0 (key kb); off(c) gives a tile cell's offset.
+template <class OffF, class ItemF>
+__device__ __forceinline__ void search_items(uint32_t r0, uint32_t kb, uint32_t uw, uint32_t budget, OffF&& off,
+                                             ItemF&& item) {
+    const uint32_t nseg = off(r0 + uw) - off(r0);
+    if (nseg == 0u) return;
+    uint32_t W = uw;
+    while (W > 1u && 9ull * (W + 2u) * nseg > (unsigned long long)budget * uw) W >>= 1;
+    for (uint32_t q0 = 0; q0 < uw; q0 += W) {
+        const uint32_t nch = (off(r0 + q0 + W) - off(r0 + q0) + kChunk - 1u) / kChunk;
+        for (uint32_t c = 0; c < nch; ++c) item(kb + q0, W | (c << 6));
+    }
+}
+
+template <int kEmit>
 __global__ __launch_bounds__(256) void k_scan_cells(uint32_t* __restrict__ count, uint32_t* __restrict__ offset,
                                                     const uint32_t* __restrict__ tsum, uint32_t* __restrict__ tflag,
                                                     const uint32_t* __restrict__ tprefix, uint32_t nT,
-                                                    uint32_t lgT, uint32_t C, uint32_t lgnc,
+                                                    uint32_t lgT, uint32_t C, uint32_t lgnc, EmitArgs E,
                                                     uint32_t* __restrict__ stat) {
     __shared__ uint32_t wsum[kWaves];
     const uint32_t t = blockIdx.x;
@@ -179,11 +218,11 @@ __global__ __launch_bounds__(256) void k_scan_cells(uint32_t* __restrict__ count
         for (uint32_t i = threadIdx.x; i < T; i += blockDim.x) offset[c0 + i] = base;
         return;
     }
-    if (stat && threadIdx.x == 0) atomicAdd(&stat[CTR_NUM * (1u + (t & (kStatRep - 1u))) + CTR_SCANTILES], 1u);
+    if (kEmit == EMIT_SEARCH && threadIdx.x == 0) atomicAdd(&stat[CTR_NUM * (1u + (t & (kStatRep - 1u))) + CTR_SCANTILES], 1u);
     // The tile passes through LDS so that global reads and writes are
     // coalesced; thread t scans cells t*per .. t*per+per-1 there.  Word w is
     // kept at w + w/16, so the threads' 16-word strides hit distinct banks.
-    __shared__ uint32_t cell[kScanTile + kScanTile / 16];
+    __shared__ uint32_t cell[kScanTile + kScanTile / 16 + 1];
     auto at = [](uint32_t w) { return w + (w >> 4); };
     {
         uint32_t v[kScanPer];
@@ -211,12 +250,38 @@ __global__ __launch_bounds__(256) void k_scan_cells(uint32_t* __restrict__ count
         cell[at(my0 + j)] = run;
         run += c;
     }
+    if (kEmit != EMIT_NONE && threadIdx.x == 0) cell[at(T)] = base + tot;
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < T; i += blockDim.x) {
         offset[c0 + i] = cell[at(i)];
         count[count_slot(c0 + i, C, lgnc)] = 0;
     }
     if (threadIdx.x == 0) tflag[t] = 0;
+    if (kEmit == EMIT_NONE) return;
+    // thread t takes consecutive runs, so that the items stay in key order
+    __shared__ uint32_t ubase;
+    auto off = [&](uint32_t c) { return cell[at(c)]; };
+    const uint32_t lgrun = kEmit == EMIT_SEARCH ? E.lguw : lgnc;  // tile words per run
+    const uint32_t nrun = T >> lgrun, rper = (nrun + blockDim.x - 1) / blockDim.x;
+    const uint32_t r0 = threadIdx.x * rper, r1 = min(r0 + rper, nrun);
+    auto items = [&](auto&& item) {
+        for (uint32_t r = r0; r < r1; ++r) {
+            if (kEmit == EMIT_SEARCH) {
+                search_items(r << lgrun, c0 + (r << lgrun), E.uw, E.budget, off, item);
+            } else {
+                const uint32_t own = off((r + 1u) << lgrun) - off(r << lgrun);
+                const uint32_t nch = own >= kSparse ? (own + kChunk - 1u) / kChunk : 0u;
+                for (uint32_t c = 0; c < nch; ++c) item(((c0 >> lgrun) + r) << E.lguw, E.uw | (c << 6));
+            }
+        }
+    };
+    uint32_t mine = 0, all;
+    items([&](uint32_t, uint32_t) { ++mine; });
+    uint32_t u = block_excl_scan(mine, wsum, all);
+    if (threadIdx.x == 0 && all) ubase = atomicAdd(E.nunits, all);
+    __syncthreads();
+    u += ubase;
+    items([&](uint32_t k, uint32_t w) { E.units[u++] = make_uint2(k, w); });
 }
 
 // ------------------------------------------------- K4: scatter
@@ -328,68 +393,18 @@ __global__ __launch_bounds__(256) void k_merge_huge(const uint32_t* __restrict__
     }
 }
 
-// Work items of one sort: the particle at the first slot f of a run of `uw`
-// cells along x (cells kb .. kb+uw-1) appends the run's items.  A run whose
-// estimated 27-cell neighbourhood (9 rows of W+2 cells at the run's mean
-// density) exceeds `budget` particles is split into narrower units, and a
-// unit with more than kChunk own particles into several items that share its
-// neighbourhood (item = (first cell, W | chunk << 6)).
-// Called by all 64 lanes of the wave (k = kNoKey for lanes with nothing to
-// emit): the lanes' items are counted, scanned across the wave and placed
-// with one atomic per wave on the item counter, which every run of every
-// wave would otherwise hit in turn.
-constexpr uint32_t kNoKey = 0xFFFFFFFFu;
-__device__ __forceinline__ void emit_units(const uint32_t* __restrict__ offset, uint32_t k, uint32_t f, uint32_t uw,
-                                           uint32_t budget, uint2* __restrict__ units,
-                                           uint32_t* __restrict__ nunits) {
-    const uint32_t kb = (k != kNoKey ? k : 0u) & ~(uw - 1u);
-    const bool head = k != kNoKey && f == offset[kb];
-    uint32_t W = uw, total = 0;
-    if (head) {
-        const uint32_t nseg = offset[kb + uw] - offset[kb];
-        while (W > 1u && 9ull * (W + 2u) * nseg > (unsigned long long)budget * uw) W >>= 1;
-        for (uint32_t q0 = 0; q0 < uw; q0 += W) {
-            const uint32_t own = offset[kb + q0 + W] - offset[kb + q0];
-            total += (own + kChunk - 1u) / kChunk;
-        }
-    }
-    const uint32_t lane = lane_id();
-    uint32_t incl = total;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t y = (uint32_t)__shfl_up((int)incl, d, 64);
-        if (lane >= (uint32_t)d) incl += y;
-    }
-    const uint32_t wave_total = (uint32_t)__shfl((int)incl, 63, 64);
-    uint32_t base = 0;
-    if (lane == 0 && wave_total) base = atomicAdd(nunits, wave_total);
-    base = (uint32_t)__shfl((int)base, 0, 64);
-    if (head && total) {
-        uint32_t u = base + incl - total;
-        for (uint32_t q0 = 0; q0 < uw; q0 += W) {
-            const uint32_t kq = kb + q0;
-            const uint32_t nch = (offset[kq + W] - offset[kq] + kChunk - 1u) / kChunk;
-            for (uint32_t c = 0; c < nch; ++c) units[u++] = make_uint2(kq, W | (c << 6));
-        }
-    }
-}
-
 // ------------------------------------------------- K5: stable reorder
 // Makes the in-cell order ascending by original index (the stable order of
 // the reference's radix-sort paths, pbf_neighbor_search.cpp:112-131), gathers
-// x* (as float4) and x (SoA) (reorderDataCUDA, pbf_neighbor_search_util.cu:143-154)
-// and emits the work units: each run of up to `uw` cells along x is split into
-// narrower units where it is dense, so that a unit's 27-cell neighbourhood
-// fits the on-chip tile.
+// x* (as float4) and x (SoA) (reorderDataCUDA, pbf_neighbor_search_util.cu:143-154).
 template <bool kB>
 __global__ __launch_bounds__(256) void k_reorder(const float* __restrict__ x, const float* __restrict__ v, Bufs b, Scenes<kB> SC,
                                                  const uint32_t* __restrict__ key, const uint32_t* __restrict__ tmp,
-                                                 uint32_t n, uint32_t uw, uint32_t budget) {
+                                                 uint32_t n) {
     const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
     const bool active = s < (kB ? min(n, b.in_off[b.nscenes]) : n);
     const uint32_t i = active ? tmp[s] : 0u;
     const uint32_t si = (kB && active) ? b.isid[i] : 0u;
-    uint32_t ek = kNoKey, ef = 0;
     by_scene<kB>(si, active, [&](uint32_t sc) {
         const uint32_t k = key[i];
         const uint32_t o0 = b.offset[k], o1 = b.offset[k + 1];
@@ -415,12 +430,7 @@ __global__ __launch_bounds__(256) void k_reorder(const float* __restrict__ x, co
         }
         b.Pf[f] = make_float4(q[0], q[1], q[2], 0.f);
         st3(b.X, b.cap, f, mk3(xo[0], xo[1], xo[2]));
-        if (k < b.CT) {
-            ek = k;
-            ef = f;
-        }
     });
-    emit_units(b.offset, ek, ef, uw, budget, b.units, &b.ctr[CTR_UNITS]);  // all lanes
 }
 
 // ------------------------------------------------- K5b: groups of big cells
@@ -1330,33 +1340,18 @@ __global__ __launch_bounds__(256) void k_cur_hash(Bufs b, Scenes<kB> SC, uint32_
     }
 }
 
-// Places each particle at its run's position and emits the work items of
-// the runs holding at least kSparse particles (one per kChunk of them);
-// clears the overflow slots of the final-order blocks of 64.
+// Places each particle at its run's position; clears the overflow slots of
+// the final-order blocks of 64.
 __global__ __launch_bounds__(256) void k_cur_scatter(const uint32_t* __restrict__ offset, uint32_t CT,
                                                      const uint32_t* __restrict__ ckey,
                                                      const uint32_t* __restrict__ crank,
                                                      const uint32_t* __restrict__ coffset,
-                                                     uint32_t* __restrict__ cperm, uint32_t uw, uint32_t lguw,
-                                                     uint32_t lgnc, uint2* __restrict__ cunits,
-                                                     uint32_t* __restrict__ ctr, uint32_t* __restrict__ oslot) {
+                                                     uint32_t* __restrict__ cperm, uint32_t* __restrict__ oslot) {
     const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t nl = offset[CT];
     if (s >= nl) return;
     if (s <= (nl - 1u) / 64u) oslot[s] = kNoSlot;  // the final passes' blocks of 64 positions
-    const uint32_t k = ckey[s];
-    const uint32_t slot = coffset[k] + crank[s];
-    cperm[slot] = s;
-    const uint32_t run = k >> lgnc;
-    const uint32_t r0 = coffset[run << lgnc];
-    if (slot == r0) {
-        const uint32_t own = coffset[(run + 1u) << lgnc] - r0;
-        if (own >= kSparse) {
-            const uint32_t nch = (own + kChunk - 1u) / kChunk;
-            const uint32_t u = atomicAdd(&ctr[CTR_CUNITS], nch);
-            for (uint32_t c = 0; c < nch; ++c) cunits[u + c] = make_uint2(run << lguw, uw | (c << 6));
-        }
-    }
+    cperm[coffset[ckey[s]] + crank[s]] = s;
 }
 
 // The 27-cell neighbourhood of a particle's final cell, restated from
@@ -2338,6 +2333,8 @@ hipError_t step_seq(const Bufs& b, const Scenes<kB>& SC, const Tuning& T, float*
     const uint32_t nb = ceil_div(n > 0 ? n : 1, 256);
     const uint32_t CT = b.CT;
     const uint32_t budget = (T.tile_cap * 3u) / 4u > 0 ? (T.tile_cap * 3u) / 4u : 1u;
+    uint32_t lguw = 0;
+    while ((1u << lguw) < uw) ++lguw;
     auto grid = [&](int k) { return dim3(T.grid[k] ? T.grid[k] : T.grid_units); };
     const size_t smem = smem_of(T.tile_cap);
     if (n > 0) {
@@ -2352,8 +2349,9 @@ hipError_t step_seq(const Bufs& b, const Scenes<kB>& SC, const Tuning& T, float*
     }
     {
         Mark m(tm, s, K_SCAN_CELLS);
-        hipLaunchKernelGGL(k_scan_cells, dim3(b.nT + 1), dim3(kScanBlock), 0, s, b.count, b.offset, b.tsum, b.tflag,
-                           b.tprefix, b.nT, b.lgT, CT, 0u, b.ctr);
+        const EmitArgs E{uw, lguw, budget, b.units, &b.ctr[CTR_UNITS]};
+        hipLaunchKernelGGL(k_scan_cells<EMIT_SEARCH>, dim3(b.nT + 1), dim3(kScanBlock), 0, s, b.count, b.offset, b.tsum,
+                           b.tflag, b.tprefix, b.nT, b.lgT, CT, 0u, E, b.ctr);
     }
     if (n == 0) return hipGetLastError();
     {
@@ -2369,7 +2367,7 @@ hipError_t step_seq(const Bufs& b, const Scenes<kB>& SC, const Tuning& T, float*
     }
     {
         Mark m(tm, s, K_REORDER);
-        hipLaunchKernelGGL(k_reorder<kB>, dim3(nb), dim3(256), 0, s, x, v, b, SC, b.key, b.tmp, n, uw, budget);
+        hipLaunchKernelGGL(k_reorder<kB>, dim3(nb), dim3(256), 0, s, x, v, b, SC, b.key, b.tmp, n);
     }
     {
         Mark m(tm, s, K_BIG_SEG);
@@ -2401,8 +2399,6 @@ hipError_t step_seq(const Bufs& b, const Scenes<kB>& SC, const Tuning& T, float*
     }
     // runs of uw final cells, nc = min(8, uw) counters each: CR = CT / uw * nc
     // counters (never more than CT), scanned in tiles of up to 4096 that divide CR
-    uint32_t lguw = 0;
-    while ((1u << lguw) < uw) ++lguw;
     const uint32_t lgnc = lguw < 3u ? lguw : 3u;
     const uint32_t CR = (CT >> lguw) << lgnc;
     uint32_t lgTr = 0;
@@ -2414,10 +2410,11 @@ hipError_t step_seq(const Bufs& b, const Scenes<kB>& SC, const Tuning& T, float*
         hipLaunchKernelGGL(k_tile_reduce, dim3(nTr + 1), dim3(kScanBlock), 0, s, b.ccount, b.ctflag, b.ctsum, nTr, lgTr, CR,
                            lgnc);
         hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(1024), 0, s, b.ctsum, b.ctprefix, nTr + 1, b.ctr, 0u);
-        hipLaunchKernelGGL(k_scan_cells, dim3(nTr + 1), dim3(kScanBlock), 0, s, b.ccount, b.coffset, b.ctsum, b.ctflag,
-                           b.ctprefix, nTr, lgTr, CR, lgnc, (uint32_t*)nullptr);
-        hipLaunchKernelGGL(k_cur_scatter, dim3(nb), dim3(256), 0, s, b.offset, CT, b.ckey, b.crank, b.coffset,
-                           b.cperm, uw, lguw, lgnc, b.cunits, b.ctr, b.oslot);
+        const EmitArgs E{uw, lguw, 0u, b.cunits, &b.ctr[CTR_CUNITS]};
+        hipLaunchKernelGGL(k_scan_cells<EMIT_FINAL>, dim3(nTr + 1), dim3(kScanBlock), 0, s, b.ccount, b.coffset, b.ctsum,
+                           b.ctflag, b.ctprefix, nTr, lgTr, CR, lgnc, E, (uint32_t*)nullptr);
+        hipLaunchKernelGGL(k_cur_scatter, dim3(nb), dim3(256), 0, s, b.offset, CT, b.ckey, b.crank, b.coffset, b.cperm,
+                           b.oslot);
     }
     {
         Mark m(tm, s, K_FINAL_LIST);
@@ -2465,8 +2462,8 @@ hipError_t launch_count_scan(uint32_t* count, uint32_t* offset, uint32_t* tsum, 
                              uint32_t nT, uint32_t lgT, uint32_t C, hipStream_t s) {
     hipLaunchKernelGGL(k_tile_reduce, dim3(nT + 1), dim3(kScanBlock), 0, s, count, tflag, tsum, nT, lgT, C, 0u);
     hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(1024), 0, s, tsum, tprefix, nT + 1, (uint32_t*)nullptr, 0u);
-    hipLaunchKernelGGL(k_scan_cells, dim3(nT + 1), dim3(kScanBlock), 0, s, count, offset, tsum, tflag, tprefix, nT, lgT, C, 0u,
-                       (uint32_t*)nullptr);
+    hipLaunchKernelGGL(k_scan_cells<EMIT_NONE>, dim3(nT + 1), dim3(kScanBlock), 0, s, count, offset, tsum, tflag, tprefix, nT,
+                       lgT, C, 0u, EmitArgs{}, (uint32_t*)nullptr);
     return hipGetLastError();
 }
 
