@@ -258,37 +258,50 @@ __device__ __forceinline__ void walk_list(const uint32_t* __restrict__ nl, uint3
         for_list8(nl, cap, i, n, [&](uint32_t j) { return rec[j]; }, body);
 }
 
-// 1.f / sqrtf(r2) with both operations correctly rounded -- the IEEE
-// result -- in about a third of the instructions of the IEEE sequences.  On
-// [2^-96, FLT_MAX] (normal_r2): v_sqrt_f32, then the two-sided fma test of
-// its neighbours (s - 1 ulp is taken when fma(-(s - ulp), s, r2) <= 0, s + 1
-// ulp when fma(-(s + ulp), s, r2) > 0), then v_rcp_f32 and one Newton step
-// y + y * fma(-s, y, 1).  Outside that range (0, below 2^-96, inf, NaN) the
-// IEEE operations themselves.  pbfx_selftest_inv_sqrt compares this function
-// with the IEEE form on every float of the range.
+// sqrtf(r2) and 1.f / sqrtf(r2) with every operation correctly rounded -- the
+// IEEE results -- from one transcendental: with y = v_rsq_f32(r2), g = r2 y and
+// h = y / 2, s = g + h (r2 - g g) (the residual exact in one fma) is the
+// correctly rounded root, and y + y (e + 2 e^2), e = 1 - s y, the correctly
+// rounded reciprocal of s (for the root of all-ones significand y is a power of
+// two and y + y e a tie that rounds down, wrongly; e + e^2 rounds back to e).  On [2^-96, FLT_MAX] (normal_r2); outside it (0, below 2^-96, inf,
+// NaN) the IEEE operations themselves.  pbfx_selftest_inv_sqrt compares both
+// values with the IEEE operations on every float.  (v_sqrt_f32 with a
+// two-sided correction and v_rcp_f32 with a Newton step give the same values
+// in two transcendentals and two more operations: with them k_lambda took 51 us and
+// k_deltap 71 us on the 1M dam, with these 47 and 62.)
 __device__ __forceinline__ bool normal_r2(float r2) { return r2 >= 0x1p-96f && r2 <= 0x1.fffffep+127f; }
 
-__device__ __forceinline__ float inv_sqrt_normal(float r2) {
-    const float s0 = __builtin_amdgcn_sqrtf(r2);
-    const uint32_t si = __float_as_uint(s0);
-    const float sd = __uint_as_float(si - 1u), su = __uint_as_float(si + 1u);
-    const float vd = __builtin_fmaf(-sd, s0, r2), vu = __builtin_fmaf(-su, s0, r2);
-    float s = (vd <= 0.f) ? sd : s0;
-    s = (vu > 0.f) ? su : s;
-    const float y = __builtin_amdgcn_rcpf(s);
-    return __builtin_fmaf(__builtin_fmaf(-s, y, 1.f), y, y);
+struct RootInv {
+    float s, inv;  // sqrt(r2), 1 / sqrt(r2)
+};
+__device__ __forceinline__ RootInv sqrt_inv_normal(float r2) {
+    const float y = __builtin_amdgcn_rsqf(r2);
+    const float g = r2 * y, h = 0.5f * y;
+    const float s = __builtin_fmaf(__builtin_fmaf(-g, g, r2), h, g);
+    const float e = __builtin_fmaf(-s, y, 1.f);
+    return RootInv{s, __builtin_fmaf(__builtin_fmaf(e + e, e, e), y, y)};
 }
 
-__device__ __forceinline__ float inv_sqrt(float r2) {
-    if (__builtin_expect(normal_r2(r2), 1)) return inv_sqrt_normal(r2);
-    return 1.f / __builtin_sqrtf(r2);
+__device__ __forceinline__ RootInv sqrt_inv(float r2) {
+    if (__builtin_expect(normal_r2(r2), 1)) return sqrt_inv_normal(r2);
+    const float s = __builtin_sqrtf(r2);
+    return RootInv{s, 1.f / s};
+}
+
+// Whether every active lane's r2 is zero or in [2^-96, FLT_MAX]: every pair
+// but non-finite positions and separations below 2^-48.  A particle's list
+// holds the particle itself (r2 = 0) at a place that differs from lane to
+// lane, so that about half of a wave's pair steps have such a lane: the fast
+// forms below take it along instead of sending the wave to the general ones.
+__device__ __forceinline__ bool wave_plain_r2(float r2) {
+    return __builtin_amdgcn_ballot_w64(!normal_r2(r2) && r2 != 0.f) == 0ull;
 }
 
 // pbf/solver/cuda/pbf_kernel_memorization.cu:15-56 (memorizeKernelPair):
 // W and grad W of one listed pair from d = self - x_j and r2 = |d|^2
 // (rsqrtf restated as 1/sqrtf), for any r2.
 __device__ __forceinline__ void pair_core(F3 d, float r2, const Phys& P, float& W, F3& kg) {
-    float inv_r = inv_sqrt(r2);
+    float inv_r = sqrt_inv(r2).inv;
     float q2 = r2 * P.inv_h * P.inv_h;
     W = 0.f;
     if (q2 <= 1.f) {
@@ -303,11 +316,13 @@ __device__ __forceinline__ void pair_core(F3 d, float r2, const Phys& P, float& 
     if (r2 > 0.f) kg = mulsv(kd, mulvs(d, inv_r));
 }
 
-// pair_core for r2 in [2^-96, FLT_MAX], with the same results: the r2 > 0
-// test always holds there, and t = max(1 - q2, 0) is 1 - q2 when q2 <= 1 and
-// exactly 0 otherwise (q2 finite), so W = a t^3 needs no select.
-__device__ __forceinline__ void pair_core_normal(F3 d, float r2, const Phys& P, float& W, F3& kg) {
-    const float inv_r = inv_sqrt_normal(r2);
+// pair_core for r2 zero or in [2^-96, FLT_MAX], with the same results in the
+// sums: t = max(1 - q2, 0) is 1 - q2 when q2 <= 1 and exactly 0 otherwise (q2
+// finite), so W = a t^3 needs no select; and r2 = 0 takes the reciprocal root
+// of FLT_MAX, below 1/h, so that kd = 0 and kg is +-0 where pair_core's is +0,
+// which no sum that starts at +0 tells apart.
+__device__ __forceinline__ void pair_core_plain(F3 d, float r2, const Phys& P, float& W, F3& kg) {
+    const float inv_r = sqrt_inv_normal(r2 != 0.f ? r2 : 0x1.fffffep+127f).inv;
     const float q2 = r2 * P.inv_h * P.inv_h;
     const float t = __builtin_fmaxf(1.f - q2, 0.f);
     W = P.a * t * t * t;
@@ -318,16 +333,39 @@ __device__ __forceinline__ void pair_core_normal(F3 d, float r2, const Phys& P, 
     kg = mulsv(kd, mulvs(d, inv_r));
 }
 
-// W and grad W of the pair (self, pj).  A wave whose active lanes all have
-// r2 in [2^-96, FLT_MAX] -- every pair but coincident particles and
-// non-finite positions -- takes pair_core_normal.
+// W and grad W of the pair (self, pj): pair_core_plain in a wave whose active
+// lanes all qualify.
 __device__ __forceinline__ void pair_terms(F3 self, F3 pj, const Phys& P, float& W, F3& kg) {
     const F3 d = self - pj;
     const float r2 = __builtin_fmaf(d.z, d.z, __builtin_fmaf(d.y, d.y, d.x * d.x));
-    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!normal_r2(r2)) == 0ull, 1))
-        pair_core_normal(d, r2, P, W, kg);
+    if (__builtin_expect(wave_plain_r2(r2), 1))
+        pair_core_plain(d, r2, P, W, kg);
     else
         pair_core(d, r2, P, W, kg);
+}
+
+// a / s for the three components of a, correctly rounded, with inv the
+// correctly rounded reciprocal of s: q = a inv and one residual correction
+// each.  q lies within 1.5 units in the last place of the quotient, so the
+// corrected value is off by at most 4 * 2^-25 units before it is rounded; the
+// quotients that lie that close to a midpoint (a 2^k - (2Q+1) s = N with
+// |N| <= 16, all 93 million pairs of significands) were compared with the IEEE
+// division one by one.  Valid while nothing underflows: div3_plain.
+__device__ __forceinline__ F3 div3_inv(F3 a, float s, float inv) {
+    const F3 q = mk3(a.x * inv, a.y * inv, a.z * inv);
+    return mk3(__builtin_fmaf(__builtin_fmaf(-q.x, s, a.x), inv, q.x),
+               __builtin_fmaf(__builtin_fmaf(-q.y, s, a.y), inv, q.y),
+               __builtin_fmaf(__builtin_fmaf(-q.z, s, a.z), inv, q.z));
+}
+// Whether div3_inv holds for d with |d|^2 = r2 on every active lane: r2 zero or
+// in [2^-96, 2^60], the components zero or at least 2^-96 in magnitude.
+// (2 |x| - 1 as an unsigned word wraps to the largest value for x = 0.)
+__device__ __forceinline__ bool wave_plain_div(F3 d, float r2) {
+    const uint32_t lim = 2u * 0x0F800000u - 1u;  // the bits of 2^-96
+    const uint32_t x = 2u * __float_as_uint(d.x) - 1u, y = 2u * __float_as_uint(d.y) - 1u,
+                   z = 2u * __float_as_uint(d.z) - 1u;
+    const bool tiny = min(min(x, y), z) < lim;
+    return __builtin_amdgcn_ballot_w64(tiny || (!(r2 >= 0x1p-96f && r2 <= 0x1p60f) && r2 != 0.f)) == 0ull;
 }
 
 // pbf/solver/cuda/boundary/pbf_plane_boundary.cu:6-45

@@ -1925,12 +1925,24 @@ __device__ __forceinline__ void for_final(const Bufs& b, F&& body) {
     by_scene<kB>((kB && active) ? b.sid[g] : 0u, active, [&](uint32_t sc) { body(q, g, b.fcnt[q], sc); });
 }
 
+// The pair terms of the final passes.  Each takes its root (and the three
+// divisions by it) from sqrt_inv_normal and div3_inv in a wave whose active
+// lanes all qualify (the IEEE sequences otherwise): over the piles of the first
+// ten chained steps of the 1M dam k_ovf_part went from 1.72 to 1.41 ms a launch
+// (vorticity) and from 1.58 to 1.33 ms (confinement).
+
 // vorticity pair term (pbf_vorticity_confinement.cu:15-31)
 __device__ __forceinline__ F3 vort_pair(F3 self, F3 selfv, F3 pj, F3 vj, float warg) {
     const F3 pd = pj - self;
-    const float r = glm_length(pd);
     const F3 vd = vj - selfv;
+    const float r2 = glm_dot(pd, pd);
     F3 w = mk3(0.f, 0.f, 0.f);
+    if (__builtin_expect(wave_plain_div(pd, r2), 1)) {
+        const RootInv q = sqrt_inv_normal(r2);
+        if (r2 != 0.f) w = mulvs(glm_cross(vd, div3_inv(pd, q.s, q.inv)), wspiky_deriv(q.s, warg));
+        return w;
+    }
+    const float r = glm_length(pd);
     if (r > 0.f) w = mulvs(glm_cross(vd, divvs(pd, r)), wspiky_deriv(r, warg));
     return w;
 }
@@ -1938,8 +1950,14 @@ __device__ __forceinline__ F3 vort_pair(F3 self, F3 selfv, F3 pj, F3 vj, float w
 // confinement location-vector pair term (pbf_vorticity_confinement.cu:121-138)
 __device__ __forceinline__ F3 loc_pair(F3 self, F3 pj, float wj, float warg) {
     const F3 pd = pj - self;
-    const float r = glm_length(pd);
+    const float r2 = glm_dot(pd, pd);
     F3 l = mk3(0.f, 0.f, 0.f);
+    if (__builtin_expect(wave_plain_div(pd, r2), 1)) {
+        const RootInv q = sqrt_inv_normal(r2);
+        if (r2 != 0.f) l = mulvs(mulsv(wj, div3_inv(pd, q.s, q.inv)), wspiky_deriv(q.s, warg));
+        return l;
+    }
+    const float r = glm_length(pd);
     if (r > 0.f) l = mulvs(mulsv(wj, divvs(pd, r)), wspiky_deriv(r, warg));
     return l;
 }
@@ -1947,9 +1965,11 @@ __device__ __forceinline__ F3 loc_pair(F3 self, F3 pj, float wj, float warg) {
 // XSPH pair term (pbf_xsph.cu:15-29)
 __device__ __forceinline__ F3 xsph_pair(F3 self, F3 selfv, F3 pj, F3 vj, float inv_h) {
     const F3 pd = pj - self;
-    const float r = glm_length(pd);
     const F3 vd = vj - selfv;
-    return mulvs(vd, wpoly6(r, inv_h));
+    const float r2 = glm_dot(pd, pd);
+    if (__builtin_expect(wave_plain_r2(r2), 1))
+        return mulvs(vd, wpoly6(r2 != 0.f ? sqrt_inv_normal(r2).s : 0.f, inv_h));
+    return mulvs(vd, wpoly6(glm_length(pd), inv_h));
 }
 
 // The three final passes as (elements, pair term, support) for the particle
@@ -2233,8 +2253,8 @@ __global__ void k_selftest(const float* __restrict__ a, const float* __restrict_
     out[4 * i + 3] = floorf(x / y);
 }
 
-// inv_sqrt against 1.f / sqrtf on every bit pattern in [lo, hi] (grid-stride):
-// counts the mismatches and records the first one's input bits (any one, if
+// sqrt_inv against sqrtf and 1.f / sqrtf on every bit pattern in [lo, hi]
+// (grid-stride): counts the mismatches and records the first one's input bits (any one, if
 // several race).
 __global__ __launch_bounds__(256) void k_selftest_inv_sqrt(uint32_t lo, uint32_t hi,
                                                            unsigned long long* __restrict__ mismatches,
@@ -2243,7 +2263,9 @@ __global__ __launch_bounds__(256) void k_selftest_inv_sqrt(uint32_t lo, uint32_t
     uint32_t bad = 0, which = 0;
     for (uint64_t u = (uint64_t)lo + blockIdx.x * blockDim.x + threadIdx.x; u <= hi; u += stride) {
         const float r2 = __uint_as_float((uint32_t)u);
-        if (__float_as_uint(inv_sqrt(r2)) != __float_as_uint(1.f / __builtin_sqrtf(r2))) {
+        const RootInv q = sqrt_inv(r2);
+        const float s = __builtin_sqrtf(r2);
+        if (__float_as_uint(q.s) != __float_as_uint(s) || __float_as_uint(q.inv) != __float_as_uint(1.f / s)) {
             if (!bad) which = (uint32_t)u;
             ++bad;
         }
