@@ -261,10 +261,10 @@ typedef struct pbfx_stats {
     uint32_t max_sweeps_used;
     uint32_t xsph_nan;         /* particles whose XSPH sum was NaN (velocity kept) */
     uint32_t units;            /* work units (cell blocks) of the last step */
-    uint32_t slow_units;       /* units whose neighbourhood exceeded the on-chip tile */
-    uint32_t slow_particles;   /* final-pass particles filtered from global memory (sparse runs, large tiles) */
+    uint32_t slow_units;       /* units whose neighbourhood holds more than tile_cap particles */
+    uint32_t slow_particles;   /* final-pass particles of sparse final-cell runs, or of neighbourhoods above 2560 particles */
     uint32_t tile_overflow;    /* reserved, always 0 (neighbourhoods of any size are searched) */
-    uint32_t max_tile;         /* largest neighbourhood tile seen */
+    uint32_t max_tile;         /* particles of the largest neighbourhood of a work unit */
     uint32_t steps;            /* steps run by this context */
     uint32_t final_units;      /* work units of the final passes (final-cell runs) */
     uint32_t list_overflow;    /* particles with more than 64 in-range final pairs (summed cell by cell) */
@@ -276,9 +276,10 @@ typedef struct pbfx_stats {
 /* Statistics of the last step (synchronises `stream`). */
 pbfx_status pbfx_get_stats(pbfx_ctx* ctx, void* stream, pbfx_stats* out);
 
-/* Tuning knobs.  tile_cap: particles held on chip per work unit (0 forces
- * the global-memory path everywhere, for testing; default 2048, max 4096);
- * unit_width: max cells per work unit along x (power of two 1..32, default 16). */
+/* Tuning knobs.  tile_cap: particles of a work unit's neighbourhood above
+ * which a run of cells is split into narrower units, and a unit is counted as
+ * slow (statistics; default 2048, max 4096); unit_width: cells per run along x
+ * (power of two 1..32, default 16), by which the final passes group particles. */
 pbfx_status pbfx_set_tuning(pbfx_ctx* ctx, uint32_t tile_cap, uint32_t unit_width);
 
 /* Autotuner: times one step of the given state for every candidate

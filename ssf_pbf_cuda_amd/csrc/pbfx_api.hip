@@ -59,8 +59,6 @@ struct pbfx_ctx {
     uint32_t uw_max = kMaxW;             // narrowest grid row of any scene
     Bufs b{};
     Tuning T{};
-    int num_cu = 0;
-    int blocks_per_cu = 1;
     Scene* d_scenes = nullptr;           // scene table on the device
     Scene* h_scenes = nullptr;           // pinned staging of the table
     std::vector<Scene> last_table;       // what the device holds
@@ -272,11 +270,6 @@ pbfx_status alloc_list(pbfx_ctx* c, uint32_t stride) {
     if (e != hipSuccess) return hip_fail(c, e);
     c->list_stride = stride;
     return PBFX_OK;
-}
-
-void set_grid_units(pbfx_ctx* c) {
-    size_unit_grids(c->T, c->num_cu);
-    c->blocks_per_cu = (int)(c->T.grid_units / (uint32_t)(c->num_cu > 0 ? c->num_cu : 1));
 }
 
 pbfx_status make_grid(const pbfx_params& p, const float end[3], Grid& G);
@@ -525,7 +518,6 @@ pbfx_status create_common(pbfx_ctx* c) {
         const float4 sph = make_float4(3.f, 3.f, 3.f, 3.f);
         e = hipMemcpy(c->d_default_sphere, &sph, sizeof(sph), hipMemcpyHostToDevice);
     }
-    if (e == hipSuccess) e = hipDeviceGetAttribute(&c->num_cu, hipDeviceAttributeMultiprocessorCount, c->device);
     if (e != hipSuccess) return hip_fail(c, e);
     b.scenes = c->d_scenes;
     b.kbase = c->d_kbase;
@@ -539,7 +531,6 @@ pbfx_status create_common(pbfx_ctx* c) {
     if (st != PBFX_OK) return st;
     c->T.tile_cap = 2048;
     c->T.unit_width = 16;
-    set_grid_units(c);
     (void)hipDeviceSynchronize();
     return PBFX_OK;
 }
@@ -573,7 +564,6 @@ pbfx_status set_scene_params(pbfx_ctx* c, SceneHost& h, const pbfx_params* p) {
     st = alloc_list(c, (uint32_t)make_phys(*p).stride);
     if (st != PBFX_OK) return st;
     h.params = *p;
-    set_grid_units(c);
     return PBFX_OK;
 }
 
@@ -945,7 +935,6 @@ pbfx_status pbfx_set_tuning(pbfx_ctx* c, uint32_t tile_cap, uint32_t unit_width)
     DeviceGuard g(c->device);
     c->T.tile_cap = tile_cap;
     c->T.unit_width = unit_width;
-    set_grid_units(c);
     return PBFX_OK;
 }
 
@@ -986,7 +975,6 @@ pbfx_status pbfx_autotune(pbfx_ctx* c, const float* x, const float* v, uint32_t 
                 if (uw > c->uw_max && uw != widths[0]) continue;
                 c->T.tile_cap = tc;
                 c->T.unit_width = uw;
-                set_grid_units(c);
                 float& t = tbest[ti][wi];
                 for (int rep = 0; rep < 2 && e == hipSuccess && st == PBFX_OK; ++rep) {
                     e = hipMemcpyAsync(xs, x, (size_t)n * 3 * sizeof(float), hipMemcpyDeviceToDevice, s);
@@ -1015,7 +1003,6 @@ pbfx_status pbfx_autotune(pbfx_ctx* c, const float* x, const float* v, uint32_t 
     c->T = saved;
     c->T.tile_cap = best_tile;
     c->T.unit_width = best_uw;
-    set_grid_units(c);
     if (e != hipSuccess) return hip_fail(c, e);
     if (st != PBFX_OK) return st;
     if (tile_out) *tile_out = best_tile;
@@ -1416,8 +1403,6 @@ pbfx_status static_device(int dev, StaticDev** out, int* hip_err) {
     if (!d.ready) {
         void* p = nullptr;
         hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-        int ncu = 0;
-        if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
         if (e != hipSuccess) {
             *hip_err = (int)e;
             return PBFX_HIP_ERROR;
@@ -1425,7 +1410,6 @@ pbfx_status static_device(int dev, StaticDev** out, int* hip_err) {
         d.ptr = static_cast<unsigned char*>(p);
         d.T.tile_cap = 2048;
         d.T.unit_width = 16;
-        size_unit_grids(d.T, ncu);
         d.ready = true;
     }
     *out = &d;

@@ -41,6 +41,9 @@ __device__ __forceinline__ F3 glm_cross(F3 x, F3 y) {
 // the hand-fused dot of the solver kernels: fmaf(a.z,b.z, fmaf(a.y,b.y, a.x*b.x))
 __device__ __forceinline__ float fdot(F3 a, F3 b) { return __builtin_fmaf(a.z, b.z, __builtin_fmaf(a.y, b.y, a.x * b.x)); }
 
+__device__ __forceinline__ F3 f3of(float4 f) { return mk3(f.x, f.y, f.z); }
+__device__ __forceinline__ F3 f3of(F3 f) { return f; }
+
 __device__ __forceinline__ F3 ld3(const float* __restrict__ a, uint32_t cap, uint32_t i) {
     return mk3(a[i], a[cap + i], a[2 * cap + i]);
 }
@@ -247,17 +250,6 @@ __device__ __forceinline__ void for_list8_any(const uint32_t* __restrict__ nl, u
     }
 }
 
-// The Jacobi passes' walk over slot i's list: buffer gathers when the
-// records' byte offsets fit 32 bits, plain loads otherwise.
-template <class BodyF>
-__device__ __forceinline__ void walk_list(const uint32_t* __restrict__ nl, uint32_t cap, uint32_t i, uint32_t n,
-                                          const float4* __restrict__ rec, BodyF&& body) {
-    if (cap < kGatherMaxSlots)
-        for_list8_any(nl, cap, i, n, Gather16(rec, cap), body);
-    else
-        for_list8(nl, cap, i, n, [&](uint32_t j) { return rec[j]; }, body);
-}
-
 // sqrtf(r2) and 1.f / sqrtf(r2) with every operation correctly rounded -- the
 // IEEE results -- from one transcendental: with y = v_rsq_f32(r2), g = r2 y and
 // h = y / 2, s = g + h (r2 - g g) (the residual exact in one fma) is the
@@ -333,15 +325,83 @@ __device__ __forceinline__ void pair_core_plain(F3 d, float r2, const Phys& P, f
     kg = mulsv(kd, mulvs(d, inv_r));
 }
 
+__device__ __forceinline__ float pair_r2(F3 d) {
+    return __builtin_fmaf(d.z, d.z, __builtin_fmaf(d.y, d.y, d.x * d.x));
+}
+
 // W and grad W of the pair (self, pj): pair_core_plain in a wave whose active
 // lanes all qualify.
 __device__ __forceinline__ void pair_terms(F3 self, F3 pj, const Phys& P, float& W, F3& kg) {
     const F3 d = self - pj;
-    const float r2 = __builtin_fmaf(d.z, d.z, __builtin_fmaf(d.y, d.y, d.x * d.x));
+    const float r2 = pair_r2(d);
     if (__builtin_expect(wave_plain_r2(r2), 1))
         pair_core_plain(d, r2, P, W, kg);
     else
         pair_core(d, r2, P, W, kg);
+}
+
+// v of lane m of this lane's group of L (4: a quad; 16: a row), by DPP, which
+// the compiler folds into the instruction that uses it.
+template <int L, int m>
+__device__ __forceinline__ float lane_of(float v) {
+    static_assert(L == 4 || L == 16, "a quad or a row");
+    constexpr int ctrl = L == 4 ? m * 0x55 : 0x150 + m;  // quad_perm [m,m,m,m], row_newbcast:m
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), ctrl, 0xF, 0xF, true));
+}
+
+// acc += v of lane m for m = 0 .. L-1 in order, on every lane of the group.
+template <int L, int NC, int m = 0>
+__device__ __forceinline__ void add_lanes(float (&acc)[NC], const float (&v)[NC]) {
+    if constexpr (m < L) {
+#pragma unroll
+        for (int q = 0; q < NC; ++q) acc[q] += lane_of<L, m>(v[q]);
+        add_lanes<L, NC, m + 1>(acc, v);
+    }
+}
+
+// The Jacobi passes' sums over slot i's frozen list: term(W, grad W, record,
+// c) gives a pair's NC addends, added to acc in list order.
+//
+// L = 1: one thread walks the list, eight entries' records in flight (for_list8).
+// L > 1: the L lanes l of a group take one entry each of every L, and the
+// addends are then added in list order by every lane of the group (an entry
+// past n adds +0, which changes no sum that starts at +0), so the sums are the
+// same bit for bit.  Adding the addends on every lane makes a group of 16 cost
+// about three times one thread's work and a quad 1.4 times, which pays while the
+// chip is not full (the rule stands at by_lanes).
+template <int L, int NC, class TermF>
+__device__ __forceinline__ void sum_pairs(const uint32_t* __restrict__ nl, uint32_t cap, uint32_t i, uint32_t l,
+                                          uint32_t n, F3 self, const float4* __restrict__ rec, const Phys& P,
+                                          float (&acc)[NC], TermF&& term) {
+    if constexpr (L == 1) {
+        auto body = [&](uint32_t, float4 el) {
+            float W, c[NC];
+            F3 kg;
+            pair_terms(self, f3of(el), P, W, kg);
+            term(W, kg, el, c);
+#pragma unroll
+            for (int q = 0; q < NC; ++q) acc[q] += c[q];
+        };
+        // buffer gathers when the records' byte offsets fit 32 bits, plain loads otherwise
+        if (cap < kGatherMaxSlots)
+            for_list8_any(nl, cap, i, n, Gather16(rec, cap), body);
+        else
+            for_list8(nl, cap, i, n, [&](uint32_t j) { return rec[j]; }, body);
+    } else {
+        uint32_t j = l < n ? nl[list_at(cap, i, l)] : i;
+        for (uint32_t k = l; k - l < n; k += (uint32_t)L) {
+            const float4 el = rec[j];
+            const bool on = k < n;
+            j = k + (uint32_t)L < n ? nl[list_at(cap, i, k + (uint32_t)L)] : i;
+            float W, c[NC];
+            F3 kg;
+            pair_terms(self, f3of(el), P, W, kg);
+            term(W, kg, el, c);
+#pragma unroll
+            for (int q = 0; q < NC; ++q) c[q] = on ? c[q] : 0.f;
+            add_lanes<L, NC>(acc, c);
+        }
+    }
 }
 
 // a / s for the three components of a, correctly rounded, with inv the
@@ -583,9 +643,6 @@ __device__ __forceinline__ void mark_tile(uint32_t* __restrict__ tflag, uint32_t
     if (tflag[t] == 0u) tflag[t] = 1u;
 }
 
-__device__ __forceinline__ F3 f3of(float4 f) { return mk3(f.x, f.y, f.z); }
-__device__ __forceinline__ F3 f3of(F3 f) { return f; }
-
 // Whether the step sorts the segment of a cell of n particles.
 __device__ __forceinline__ bool sorted_cell(uint32_t n) { return n > kSmallCell; }
 
@@ -606,14 +663,15 @@ __device__ __forceinline__ void list_big_cell(const uint32_t* __restrict__ offse
     }
 }
 
-// Block -> index range, contiguous per XCD (workgroup b runs on XCD b % 8),
-// so that neighbouring slots share an L2.
-__device__ __forceinline__ uint32_t xcd_block() {
-    const uint32_t nb = gridDim.x, b = blockIdx.x, nx = 8;
+// Block b of nb -> index range, contiguous per XCD (workgroup b runs on XCD
+// b % 8), so that neighbouring slots share an L2.
+__device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t nb) {
+    const uint32_t nx = 8;
     if (nb < nx) return b;
     const uint32_t per = nb / nx, rem = nb % nx, x = b % nx;
     return x * per + min(x, rem) + b / nx;
 }
+__device__ __forceinline__ uint32_t xcd_block() { return xcd_block(blockIdx.x, gridDim.x); }
 
 }  // namespace
 }  // namespace pbfx

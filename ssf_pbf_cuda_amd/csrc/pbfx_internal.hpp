@@ -2,10 +2,11 @@
 //
 // Layout in HBM (capacity `cap` particles, C cells):
 //   key, rank, tmp, sorted_index   u32[cap]      hash / histogram rank / scatter / slot->index
-//   Pf                             f32x4[cap]    predicted positions x* (w unused)
+//   Pf                             f32x4[cap]    positions x*; w: after the sort, the bits of the cell key
 //   Q                              f32x4[cap]    (x*, s) of the current Jacobi iteration (s = -lambda)
 //   X                              f32[3*cap]    SoA sorted old positions
-//   R                              f32x4[2*cap]  per slot: (x*, 0), (v, 0) -- the final passes' own record
+//   R                              f32x4[2*cap]  per slot: (x*, bits of the final cell's key), (v, 0) --
+//                                                 the final passes' own record
 //   OM4                            f32x4[cap]    per slot: (omega, |omega|)
 //   nlist, ncnt                    u32[cap*stride], u32[cap]  frozen neighbour lists as sorted
 //                                                 slots in groups of four: entries 4q..4q+3 of slot
@@ -15,11 +16,7 @@
 //   tsum, tflag, tprefix           u32[nT+1]     per-4096-cell-tile totals, occupied flags, scan
 //   units                          uint2[cap+]   work items (first cell key, width | chunk << 5)
 //   ckey, crank, cperm, ccount, coffset, ctsum, ctprefix, cunits
-//                                                 the same sort keyed by each particle's final cell;
-//                                                 once placed, crank holds the queue of final-order
-//                                                 positions whose list build k_final_heavy does (and,
-//                                                 between the search and the regrouping, the slots
-//                                                 whose search list k_ns_heavy builds)
+//                                                 the same sort keyed by each particle's final cell
 //   flist, fcnt                    u32[64*cap], u32[cap]  in-range pairs of the final passes by
 //                                                 final-order position (groups of four, list_at), counts
 //   bslot, aux                     u32[cap]      big cell -> descriptor (at its first slot); its
@@ -39,15 +36,17 @@
 
 namespace pbfx {
 
-constexpr int kBlock = 256;               // threads per work-unit workgroup
+constexpr int kBlock = 256;               // threads per workgroup of the per-particle kernels
 constexpr int kWaves = kBlock / 64;
-constexpr uint32_t kMaxW = 32;            // widest work unit along x (cells)
-constexpr uint32_t kMaxCells = 9 * (kMaxW + 2);
-constexpr uint32_t kTileCapMax = 4096;
+// Work items: runs of cells along x with their particles.  The final-cell runs
+// are the unit of the regrouping; the items themselves (splits and chunks) are
+// only counted (item_stats).
+constexpr uint32_t kMaxW = 32;            // widest run along x (cells)
+constexpr uint32_t kTileCapMax = 4096;    // largest tile_cap accepted
 constexpr uint32_t kScanTile = 4096;      // cells per scan tile
 constexpr uint32_t kChunk = kBlock;       // own particles per work item
-constexpr uint32_t kFinalTileMax = 2560;  // LDS tile of the final-list units (particles)
-constexpr uint32_t kSparse = 64;          // final-cell runs below this go one thread per particle
+constexpr uint32_t kFinalTile = 2560;     // neighbourhood above which a final item counts as slow (particles)
+constexpr uint32_t kSparse = 64;          // a final-cell run below this is no item (its particles count as slow)
 // Cells above kSmallCell particles get their index segment sorted, so that a
 // particle's in-cell rank is its position rather than a count over the whole
 // cell: up to kSortMax in one LDS sort, above that ("huge" cells) in chunks of
@@ -91,13 +90,11 @@ constexpr uint32_t kOvfBlocks = 2048;
 constexpr uint32_t kNoSlot = 0xFFFFFFFFu;       // oslot: no particle of the block overflowed (yet)
 constexpr uint32_t kPendingSlot = 0xFFFFFFFEu;  // oslot: being allocated (never seen across kernels)
 constexpr uint32_t kFullSlot = 0xFFFFFFFDu;     // oslot: no slot was left
-// A final-list or search-list build from global memory whose next cell would
-// take it past kHeavyScan candidates (a particle beside a pile) is handed to
-// k_final_heavy / k_ns_heavy, which scan it with a whole wave (kHeavyBlocks
-// workgroups of 16 waves).
+// A list build whose next cell would take it past kHeavyScan candidates (a
+// particle beside a pile) is done by a whole wave instead of a group of eight
+// lanes.
 constexpr uint32_t kHeavyScan = 2048;
 static_assert(kHeavyScan >= 27u * kSmallCell, "a build without big cells never reaches the budget");
-constexpr uint32_t kHeavyBlocks = 256;
 
 enum Ctr : int {
     CTR_UNITS = 0,
@@ -107,7 +104,7 @@ enum Ctr : int {
     CTR_XSPHNAN,
     CTR_SLOWUNITS,
     CTR_SLOWPART,
-    CTR_HEAVY,      // final-list builds handed to k_final_heavy (allocation counter of the queue in crank)
+    CTR_HEAVY,      // final-list builds done by a whole wave (statistics)
     CTR_MAXTILE,
     CTR_CUNITS,
     CTR_LISTOVF,
@@ -115,7 +112,7 @@ enum Ctr : int {
     CTR_HUGECELLS,  // cells with more than kSortMax particles (chunk-sorted, then merged)
     CTR_SCANTILES,  // occupied tiles of the cell scan (statistics)
     CTR_OVF,        // final-pass positions whose list overflowed (allocation counter of ovf)
-    CTR_NSHEAVY,    // search lists handed to waves (allocation counter of the queue in crank)
+    CTR_NSHEAVY,    // search-list builds done by a whole wave (statistics)
     CTR_NUM = 16
 };
 constexpr uint32_t kStatRep = 64;                           // copies of the statistics counters
@@ -251,10 +248,8 @@ struct Timer {
 };
 
 struct Tuning {
-    uint32_t tile_cap;      // particles staged on chip per unit
-    uint32_t unit_width;    // max cells per unit along x
-    uint32_t grid_units;    // persistent workgroups for the unit kernels (the smallest of grid[])
-    uint32_t grid[K_NUM];   // persistent workgroups per unit kernel, from its own occupancy
+    uint32_t tile_cap;      // neighbourhood above which a search item counts as slow, and is split below (particles)
+    uint32_t unit_width;    // cells per run along x
 };
 
 // ---------------------------------------------------------- differentiable form
@@ -353,8 +348,6 @@ hipError_t launch_sort_cells(const uint32_t* offset, const uint32_t* cells, cons
 hipError_t launch_restore(const Bufs& b, const float* xs, const float* vs, float* xo, float* vo, hipStream_t s);
 // p[0..n) = value by a kernel (no memset node when the caller captures a graph).
 hipError_t launch_fill_u32(uint32_t* p, size_t n, uint32_t value, hipStream_t s);
-// Fills T.grid[] (and T.grid_units) for num_cu compute units.
-void size_unit_grids(Tuning& T, int num_cu);
 
 // Adjoint launchers (pbfx_adjoint.hip).  launch_adj_step: dL/d(step input)
 // into a.axin / a.avin from a.ax / a.av, and the step's dL/dc, dL/d eps into

@@ -19,7 +19,9 @@
 // on the host.
 #include "pbfx_device.hpp"
 
+#include <algorithm>
 #include <climits>
+#include <type_traits>
 
 namespace pbfx {
 namespace {
@@ -428,7 +430,7 @@ __global__ __launch_bounds__(256) void k_reorder(const float* __restrict__ x, co
             float vs = __builtin_fmaf(P.g[c], dt, vv[c]);
             q[c] = __builtin_fmaf(vs, dt, xo[c]);
         }
-        b.Pf[f] = make_float4(q[0], q[1], q[2], 0.f);
+        b.Pf[f] = make_float4(q[0], q[1], q[2], __uint_as_float(k));
         st3(b.X, b.cap, f, mk3(xo[0], xo[1], xo[2]));
     });
 }
@@ -736,33 +738,12 @@ __device__ __forceinline__ CellView cell_view(const Bufs& b) { return CellView{b
 // grid-uniform value: the scans without them keep their plain loops).
 __device__ __forceinline__ bool big_cells(const Bufs& b) { return (b.ctr[CTR_BIGCELLS] | b.ctr[CTR_HUGECELLS]) != 0u; }
 
-// a[i] by selects (i in 0..3, not known at compile time): no array in
-// scratch memory
-__device__ __forceinline__ uint32_t pick4(const uint32_t (&a)[4], uint32_t i) {
-    const uint32_t lo = (i & 1u) ? a[1] : a[0], hi = (i & 1u) ? a[3] : a[2];
-    return (i & 2u) ? hi : lo;
-}
-
 // Whether visiting one group through aux beats scanning the whole cell (the
 // indirection costs a load per candidate): when it skips a quarter or more.
 __device__ __forceinline__ bool aux_pays(const BigPart& bp, uint32_t n) {
     return bp.how == 2u && 4u * (bp.p1 - bp.p0) <= 3u * n;
 }
 
-
-// ------------------------------------------------- work units
-struct UnitShared {
-    uint32_t tstart[kMaxCells + 1];  // tile start of each neighbourhood cell (row-major 9 x (W+2))
-    uint32_t gstart[kMaxCells];      // sorted slot of each neighbourhood cell's first particle
-    uint32_t cnt[kMaxCells];
-    uint32_t run_e[kMaxCells + 1];   // first cell of each run of cells contiguous in memory
-    uint32_t wsum[kWaves];
-};
-
-struct UnitInfo {
-    uint32_t W, ncell, xb, y, z, total, own_t0, own_g0, n_own, nruns;
-    bool staged;  // the neighbourhood fits the LDS tile; otherwise it is read from global memory
-};
 
 // Per-thread event tallies, summed per wave and added once at kernel end.
 struct Tally {
@@ -802,113 +783,277 @@ __device__ void flush_tally(uint32_t* __restrict__ ctr_base, const Tally& t) {
     }
 }
 
-// XCD-aware split: workgroup b runs on XCD b % 8; each XCD takes a contiguous
-// share of the (roughly key-ordered) unit list so neighbouring units share an L2.
-__device__ __forceinline__ void unit_range(uint32_t nU, uint32_t& u0, uint32_t& u1, uint32_t& step) {
-    const uint32_t nx = 8, b = blockIdx.x, Gd = gridDim.x;
-    if (Gd < nx) {
-        u0 = b;
-        u1 = nU;
-        step = Gd;
-        return;
-    }
-    const uint32_t xcd = b % nx, lb = b / nx;
-    const uint32_t nbx = (Gd - xcd + nx - 1) / nx;
-    const uint32_t chunk = (nU + nx - 1) / nx;
-    u0 = xcd * chunk + lb;
-    u1 = min(nU, (xcd + 1) * chunk);
-    step = nbx;
+constexpr uint32_t kDeferred = 0xFFFFFFFFu;  // a group's count when it left its list to a wave
+
+// ------------------------------------------------- lists by groups of eight
+// Key of cell c (0..26, in z,y,x order) of the 27 around grid position gp.
+__device__ __forceinline__ uint32_t cell27(const int gp[3], uint32_t c, const Grid& G) {
+    const int dz = (int)(c / 9u) - 1, q = (int)(c % 9u);
+    return scene_key(gp[0] + (q % 3) - 1, gp[1] + (q / 3) - 1, gp[2] + dz, G);
 }
 
-// Builds the neighbourhood table of a unit: 9 rows (dz outer, dy inner -- the
-// reference's z,y order) of W+2 cells (x0-1 .. x0+W, wrapped), their tile
-// starts and sorted slots, and the runs of cells whose particles are
-// contiguous in memory (one per row unless the row wraps).  Thread t owns
-// cells 2t and 2t+1 (up to 2 * kBlock cells).  Contains barriers: call
-// uniformly.
-static_assert(kMaxCells <= 2u * kBlock, "unit_setup gives each thread two neighbourhood cells");
-__device__ UnitInfo unit_setup(const Grid& G, const uint32_t* __restrict__ offset, uint2 unit, uint32_t tile_cap,
-                               UnitShared& S, Tally& tl) {
-    UnitInfo I;
-    I.W = unit.y & 63u;
-    const uint32_t chunk = unit.y >> 6;
-    I.ncell = 9u * (I.W + 2u);
-    const uint32_t kb = unit.x - G.base;  // key within the scene's grid
-    I.xb = kb & (G.gx - 1u);
-    I.y = (kb >> G.lgx) & (G.gy - 1u);
-    I.z = kb >> (G.lgx + G.lgy);
-    const uint32_t e0 = 2u * threadIdx.x;
-    uint32_t cnt[2] = {0u, 0u};
+constexpr uint32_t kGroup = 8;
+constexpr uint32_t kGroups = kBlock / kGroup;  // groups of a workgroup
+constexpr uint32_t kMaxPair = 64;              // the largest max_pair accepted
+constexpr uint32_t kGroupList = 96;            // entries held on chip: the longest list kept, and a row's hits past it
+static_assert(kGroupList >= kFinalK + 4u * kGroup && kGroupList >= kMaxPair - 1u + 4u * kGroup,
+              "room for the hits past a full list");
+// A group's cells (first slot and particles of each of the 27) and its list.
+struct GroupShared {
+    uint2 cell[kGroups][27];
+    uint4 list[kGroups][kGroupList / 4];
+};
+
+// The list of one particle (slot `slot`, in the cell of key `key`), at list
+// position i, built by a group of eight lanes from global memory: the 27 cells
+// around its cell in z,y,x order, slots ascending, eight candidates x*_j = Pf[j]
+// at a time (a cell of the lattice is one step).  A ballot ranks a step's hits,
+// which go to the list on chip; the list is written out whole at the end, 16
+// bytes a lane.  A row's three cells are tested together, and the next row's
+// candidates are loaded before their hits are ranked.
+//   search (kFinal false): pairs by pair_test<false>, the first lim kept; the
+//     return value exceeds lim when there are more.
+//   final (kFinal true): pairs by pair_test<true>, the first pair of each cell
+//     marked by bit 31; past lim pairs the list overflows (returns more than
+//     lim) and is not written.
+// kBig (the step has cells of more than kSmallCell particles): in a big cell
+// groups out of range are skipped, a group wholly in range is listed without
+// tests (the final lists stop at once when such groups alone take them past
+// lim), and a single group left is scanned through aux when that skips a
+// quarter of the cell or more.  Returns kDeferred, leaving the list unfinished,
+// before a range that would take the candidates tested past `budget` (only a
+// neighbourhood holding a big cell can: 27 * kSmallCell < kHeavyScan).
+// kWide: more than 2^28 slots, whose records' byte offsets pass 32 bits.
+// Called by all eight lanes; every value but the candidates is the same on them.
+//
+// Bound by VALU issue at large sizes (0.95 of one wave64 instruction per SIMD
+// every 4 cycles, about 95 instructions a particle; 177 us for the search and
+// 184 us for the final lists of the 1M dam) and by the latency of nine dependent
+// rows at small ones (4 us).  A thread per particle walks a serial chain of 54
+// groups of four candidates instead, whose latency set the time: from tiles of
+// cells staged in LDS 202 and 340 us on the 1M dam, 27 and 33 us for 960
+// particles, and 576 us a launch for the final lists beside the piles of the
+// chained 32k dam (now 40).  Taking a row's 24 particles as one range (fewer
+// partial steps in the lattice) measured slower wherever cells hold more than
+// eight or a row wraps: 521 against 247 us at 16 particles a cell (1M).
+template <bool kFinal, bool kBig, bool kWide>
+__device__ __forceinline__ uint32_t group_list(GroupShared& S, const Grid& G, CellView b,
+                                               const float4* __restrict__ Pf, F3 self, uint32_t key, float thr,
+                                               uint32_t lim, uint32_t* __restrict__ lst, uint32_t cap, uint32_t i,
+                                               uint32_t slot, uint32_t budget) {
+    const uint32_t lane = lane_id(), l = lane & (kGroup - 1u), sh = lane & 56u;
+    uint2* __restrict__ cells = S.cell[threadIdx.x / kGroup];
+    uint32_t* __restrict__ keep = reinterpret_cast<uint32_t*>(S.list[threadIdx.x / kGroup]);
+    {
+        // lane l finds the cells of row l (dz outer, dy inner), and lane 0 those of row 8
+        const uint32_t k0 = key - G.base;
+        const uint32_t x = k0 & (G.gx - 1u), y = (k0 >> G.lgx) & (G.gy - 1u), z = k0 >> (G.lgx + G.lgy);
+        auto find_row = [&](uint32_t r) {
+            const uint32_t dz = r / 3u, dy = r - 3u * dz;
+            const uint32_t row = G.base + (((((z + dz - 1u) & (G.gz - 1u)) << G.lgy) + ((y + dy - 1u) & (G.gy - 1u))) << G.lgx);
 #pragma unroll
-    for (uint32_t h = 0; h < 2u; ++h) {
-        const uint32_t e = e0 + h;
-        if (e < I.ncell) {
-            const uint32_t r = e / (I.W + 2u), kk = e - r * (I.W + 2u);
-            const uint32_t cx = (I.xb + kk - 1u) & (G.gx - 1u);
-            const uint32_t cy = (I.y + (r % 3u) - 1u) & (G.gy - 1u);
-            const uint32_t cz = (I.z + (r / 3u) - 1u) & (G.gz - 1u);
-            const uint32_t key = G.base + (cz * G.gy + cy) * G.gx + cx;
-            const uint32_t gs = offset[key];
-            cnt[h] = offset[key + 1] - gs;
-            S.gstart[e] = gs;
-            S.cnt[e] = cnt[h];
+            for (uint32_t dx = 0; dx < 3u; ++dx) {
+                const uint32_t k = row + ((x + dx - 1u) & (G.gx - 1u));
+                const uint32_t o = b.offset[k];
+                cells[3u * r + dx] = make_uint2(o, b.offset[k + 1] - o);
+            }
+        };
+        find_row(l);
+        if (l == 0u) find_row(8u);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the group's own lanes wrote what it reads
+    // A lane past its row's end loads some other record, which is not looked at.
+    const Gather16 buf(Pf, cap);
+    auto load = [&](uint32_t j) { return f3of(kWide ? Pf[min(j, cap - 1u)] : buf(j)); };
+    auto test = [&](F3 pj) { return pair_test<kFinal>(kFinal ? pj - self : self - pj, thr); };
+    uint32_t n = 0;
+    const uint32_t under = (1u << l) - 1u;
+    // a step's hits, this group's byte of the wave's
+    auto byte_of = [&](bool in, bool ok) {
+        return (uint32_t)((__builtin_amdgcn_ballot_w64(in) & __builtin_amdgcn_ballot_w64(ok)) >> sh) & 0xFFu;
+    };
+    // Appends a step's hits in lane order; first: none of this cell's came before.
+    auto append = [&](uint32_t bits, bool hit, uint32_t j, bool first) {
+        if (hit) {
+            const uint32_t k = (uint32_t)__builtin_popcount(bits & under);
+            // k - 1 has bit 31 set when no lane below hits
+            (keep + n)[k] = (kFinal && first) ? (((k - 1u) & 0x80000000u) | j) : j;
+        }
+        n += (uint32_t)__builtin_popcount(bits);
+    };
+    uint2 c[3];
+    F3 p[3], q[3];  // the cells' first and second steps
+    bool two;       // some group's row has a cell of more than one step
+    auto fetch = [&](uint32_t r) {
+#pragma unroll
+        for (uint32_t d = 0; d < 3u; ++d) c[d] = cells[3u * r + d];
+#pragma unroll
+        for (uint32_t d = 0; d < 3u; ++d) p[d] = load(c[d].x + l);
+        two = __builtin_amdgcn_ballot_w64(max(max(c[0].y, c[1].y), c[2].y) > kGroup) != 0ull;
+        if (two) {
+#pragma unroll
+            for (uint32_t d = 0; d < 3u; ++d) q[d] = load(c[d].x + l + kGroup);
+        }
+    };
+    q[0] = q[1] = q[2] = self;
+    fetch(0u);
+    for (uint32_t r = 0; r < 9u; ++r) {
+        const uint2 C[3] = {c[0], c[1], c[2]};
+        const uint32_t most = max(max(C[0].y, C[1].y), C[2].y);
+        uint32_t m[3], m2[3] = {0u, 0u, 0u};
+        bool h[3], h2[3] = {false, false, false};
+#pragma unroll
+        for (uint32_t d = 0; d < 3u; ++d) {
+            const bool in = l < C[d].y, ok = test(p[d]);
+            m[d] = byte_of(in, ok);
+            h[d] = in && ok;
+        }
+        const bool second = two;
+        if (second) {
+#pragma unroll
+            for (uint32_t d = 0; d < 3u; ++d) {
+                const bool in = l + kGroup < C[d].y, ok = test(q[d]);
+                m2[d] = byte_of(in, ok);
+                h2[d] = in && ok;
+            }
+        }
+        if (r < 8u) fetch(r + 1u);
+        if (!second) {  // every cell of every group's row is one step
+            if (kBig) {
+                const uint32_t all = C[0].y + C[1].y + C[2].y;
+                if (all > budget) return kDeferred;
+                budget -= all;
+            }
+#pragma unroll
+            for (uint32_t d = 0; d < 3u; ++d) append(m[d], h[d], C[d].x + l, true);
+        } else if (!kBig || most <= kSmallCell) {
+            if (kBig) {
+                const uint32_t all = C[0].y + C[1].y + C[2].y;
+                if (all > budget) return kDeferred;
+                budget -= all;
+            }
+#pragma unroll
+            for (uint32_t d = 0; d < 3u; ++d) {
+                const uint32_t n0 = n;
+                append(m[d], h[d], C[d].x + l, true);
+                if (n <= lim) append(m2[d], h2[d], C[d].x + l + kGroup, n == n0);
+                for (uint32_t t = 2u * kGroup; t < C[d].y && n <= lim; t += kGroup) {
+                    const bool in = t + l < C[d].y, ok = test(load(C[d].x + t + l));
+                    const uint32_t bits = byte_of(in, ok);
+                    append(bits, in && ok, C[d].x + t + l, n == n0);
+                }
+            }
+        } else {
+#pragma unroll 1
+            for (uint32_t d = 0; d < 3u; ++d) {
+                const uint32_t o0 = d == 0u ? C[0].x : (d == 1u ? C[1].x : C[2].x);
+                const uint32_t ncell = d == 0u ? C[0].y : (d == 1u ? C[1].y : C[2].y);
+                uint32_t p0 = 0, p1 = ncell;
+                bool via = false;
+                if (ncell > kSmallCell) {
+                    const BigPart bp = big_part<kFinal>(b.bseg + b.bslot[o0], self, thr, ncell);
+                    if (bp.how == 0u) continue;
+                    if (kFinal && n + bp.inside > lim) return lim + 1u;
+                    if (bp.all_in) {  // every member of the group is a pair: its first slots, ascending
+                        const uint32_t size = bp.p1 - bp.p0;
+                        for (uint32_t t = l; t < size && n + t < lim; t += kGroup) {
+                            const uint32_t j = bp.how == 2u ? b.aux[o0 + bp.p0 + t] : o0 + bp.p0 + t;
+                            keep[n + t] = (kFinal && t == 0u) ? (j | 0x80000000u) : j;
+                        }
+                        n += size;
+                        if (n > lim) break;
+                        continue;
+                    }
+                    if (aux_pays(bp, ncell)) {
+                        p0 = bp.p0;
+                        p1 = bp.p1;
+                        via = true;
+                    }
+                }
+                if (p1 - p0 > budget) return kDeferred;
+                budget -= p1 - p0;
+                const uint32_t n0 = n;
+                // 32 candidates' records loaded together
+                for (uint32_t t0 = p0; t0 < p1 && n <= lim; t0 += 4u * kGroup) {
+                    uint32_t j[4];
+                    F3 pj[4];
+#pragma unroll
+                    for (uint32_t u = 0; u < 4u; ++u) {
+                        const uint32_t t = t0 + l + u * kGroup;
+                        j[u] = via ? b.aux[o0 + min(t, p1 - 1u)] : o0 + t;
+                    }
+#pragma unroll
+                    for (uint32_t u = 0; u < 4u; ++u) pj[u] = load(j[u]);
+#pragma unroll
+                    for (uint32_t u = 0; u < 4u; ++u) {
+                        const bool in = t0 + l + u * kGroup < p1, ok = test(pj[u]);
+                        const uint32_t bits = byte_of(in, ok);
+                        append(bits, in && ok, j[u], n == n0);
+                    }
+                }
+                if (n > lim) break;
+            }
+        }
+        if (n > lim) break;
+    }
+    if (kFinal && n > lim) return n;
+    // the rest of the last word, which the walks load and do not use: a record at hand
+    if (l < 3u) keep[min(n, lim) + l] = slot;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const uint32_t nw = (min(n, lim) + 3u) / 4u;
+    for (uint32_t w = l; w < nw; w += kGroup)
+        reinterpret_cast<uint4*>(lst)[(size_t)w * cap + i] = S.list[threadIdx.x / kGroup][w];
+    return n;
+}
+
+// The search list of slot g by its group, and its count; true when the list
+// is left to a whole wave instead (kDeferred).
+template <bool kBig, bool kWide>
+__device__ __forceinline__ bool group_search(GroupShared& S, const Bufs& b, const Scene& sc, uint32_t g, Tally& tl) {
+    const Grid G = sc.G;
+    const uint32_t ncap = (uint32_t)sc.P.cap;
+    const float4 pk = b.Pf[g];
+    const uint32_t n = group_list<false, kBig, kWide>(S, G, cell_view(b), b.Pf, f3of(pk), __float_as_uint(pk.w),
+                                                      sc.P.h2, ncap, b.nlist, b.cap, g, g, kHeavyScan);
+    if (kBig && n == kDeferred) return true;
+    if ((lane_id() & (kGroup - 1u)) == 0u) {
+        b.ncnt[g] = min(n, ncap);
+        tl.trunc += n > ncap ? 1u : 0u;
+    }
+    return false;
+}
+
+// Statistics of the work items, one thread each (thread t of nt): the largest
+// neighbourhood, and the items whose neighbourhood passes tile_cap particles;
+// big(item) for each of those.
+template <bool kB, class BigF>
+__device__ __forceinline__ void item_stats(const Bufs& b, const Scenes<kB>& SC, const uint2* __restrict__ units,
+                                           uint32_t nU, uint32_t tile_cap, uint32_t t, uint32_t nt, Tally& tl,
+                                           BigF&& big) {
+    for (uint32_t u = t; u < nU; u += nt) {
+        const uint2 unit = units[u];
+        const Grid G = SC[scene_index<kB>(b.kbase, b.nscenes, unit.x)].G;
+        const uint32_t kb = unit.x - G.base;
+        const uint32_t x = (kb - 1u) & (G.gx - 1u), y = (kb >> G.lgx) & (G.gy - 1u), z = kb >> (G.lgx + G.lgy);
+        uint32_t total = 0;
+        for (uint32_t r = 0; r < 9u; ++r) {
+            const uint32_t cy = (y + r % 3u - 1u) & (G.gy - 1u), cz = (z + r / 3u - 1u) & (G.gz - 1u);
+            const uint32_t row = G.base + (((cz << G.lgy) + cy) << G.lgx);
+            // W + 2 cells from x on, wrapping
+            uint32_t left = (unit.y & 63u) + 2u, at = x;
+            while (left) {
+                const uint32_t k = min(left, G.gx - at);
+                total += b.offset[row + at + k] - b.offset[row + at];
+                left -= k;
+                at = 0;
+            }
+        }
+        tl.maxtile = max(tl.maxtile, total);
+        if (total > tile_cap) {
+            tl.slowunits++;
+            big(unit);
         }
     }
-    uint32_t total;
-    const uint32_t ex = block_excl_scan(cnt[0] + cnt[1], S.wsum, total);
-    if (e0 < I.ncell) S.tstart[e0] = ex;
-    if (e0 + 1u < I.ncell) S.tstart[e0 + 1u] = ex + cnt[0];
-    if (threadIdx.x == 0) S.tstart[I.ncell] = total;
-    uint32_t flag[2] = {0u, 0u};
-#pragma unroll
-    for (uint32_t h = 0; h < 2u; ++h) {
-        const uint32_t e = e0 + h;
-        if (e < I.ncell) flag[h] = (e == 0 || S.gstart[e] != S.gstart[e - 1] + S.cnt[e - 1]) ? 1u : 0u;
-    }
-    uint32_t nruns;
-    const uint32_t ri = block_excl_scan(flag[0] + flag[1], S.wsum, nruns);
-    if (flag[0]) S.run_e[ri] = e0;
-    if (flag[1]) S.run_e[ri + flag[0]] = e0 + 1u;
-    if (threadIdx.x == 0) S.run_e[nruns] = I.ncell;
-    __syncthreads();
-    const uint32_t base = 4u * (I.W + 2u);
-    I.total = total;
-    I.nruns = nruns;
-    const uint32_t skip = chunk * kChunk;
-    I.own_t0 = S.tstart[base + 1] + skip;
-    I.own_g0 = S.gstart[base + 1] + skip;
-    I.n_own = min(kChunk, S.tstart[base + I.W + 1] - I.own_t0);
-    I.staged = total <= tile_cap;
-    if (threadIdx.x == 0) {
-        tl.maxtile = max(tl.maxtile, total);
-        if (!I.staged) tl.slowunits++;
-    }
-    return I;
-}
-
-// Copies the unit's neighbourhood into the tile, one run per wave at a time
-// (coalesced): put(tile index, sorted slot).
-template <class F>
-__device__ __forceinline__ void load_runs(const UnitShared& S, const UnitInfo& I, F&& put) {
-    const uint32_t lane = lane_id(), wid = threadIdx.x >> 6;
-    for (uint32_t ri = wid; ri < I.nruns; ri += kWaves) {
-        const uint32_t e0 = S.run_e[ri], e1 = S.run_e[ri + 1];
-        const uint32_t t0 = S.tstart[e0], len = S.tstart[e1] - t0, g0 = S.gstart[e0];
-#pragma unroll 4
-        for (uint32_t i = lane; i < len; i += 64) put(t0 + i, g0 + i);
-    }
-}
-
-// cell column (1..W) of an own particle's tile index
-__device__ __forceinline__ uint32_t own_column(const UnitShared& S, uint32_t W, uint32_t t) {
-    const uint32_t base = 4u * (W + 2u);
-    uint32_t lo = base + 1u, hi = base + W;
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi + 1u) >> 1;
-        if (S.tstart[mid] <= t) lo = mid;
-        else hi = mid - 1u;
-    }
-    return lo - base;
 }
 
 // ------------------------------------------------- K6: neighbour lists
@@ -916,210 +1061,29 @@ __device__ __forceinline__ uint32_t own_column(const UnitShared& S, uint32_t W, 
 // 27 cells in z,y,x order, slots ascending, keep r2 < h^2 while fewer than
 // cap are kept; the list is frozen for all Jacobi iterations.  Stored as
 // sorted slots in groups of four (list_at), with the count in
-// ncnt[slot].  Candidates come from the unit's staged tile, four at a time.
-
-// Appends v to the queue of long list builds counted by ctr[which], a
-// wave-aggregated append to crank (dead from the final passes to the next
-// regrouping: the search's queue is read before it, the final lists' queue
-// after its placement).  A slot or position is queued at most once per step,
-// so a queue never exceeds cap.
-constexpr uint32_t kDeferred = 0xFFFFFFFFu;  // a filter's count when it left its list to a wave
-__device__ __forceinline__ void queue_push(const Bufs& b, uint32_t which, uint32_t v) {
-    const uint64_t m = __ballot(true);
-    const uint32_t lane = lane_id(), leader = (uint32_t)(__ffsll((unsigned long long)m) - 1);
-    uint32_t base = 0;
-    if (lane == leader) base = atomicAdd(&b.ctr[which], (uint32_t)__popcll(m));
-    base = (uint32_t)__shfl((int)base, (int)leader, 64);
-    const uint32_t k = base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-    if (k < b.cap) b.crank[k] = v;
-}
-
-// The filter of one own particle (column kc of the unit, slot g): candidate
-// tile index t is read at src[sb + t] -- the tile itself (kStaged) or the
-// sorted positions, with sb the cell's slot base.  Returns the number kept
-// (at most ncap); trunc is set when an (ncap+1)-th pair exists.  Each group
-// of four candidates gives a 4-bit hit mask whose pairs are stored in order.
-template <bool kStaged, class E>
-__device__ __forceinline__ uint32_t ns_filter(const UnitShared& S, uint32_t W, uint32_t kc, F3 self, float h2,
-                                              uint32_t ncap, const E* __restrict__ src,
-                                              uint32_t* __restrict__ nl, uint32_t cap, uint32_t g, bool& trunc) {
-    uint32_t* __restrict__ dst = nl + list_at(cap, g, 0u);  // where entry cnt goes
-    const size_t jump = (size_t)4u * cap - 3u;              // from entry 4q+3 to 4q+4
-    uint32_t cnt = 0;
-    for (uint32_t c = 0; c < 27u; ++c) {
-        const uint32_t e = (c / 3u) * (W + 2u) + kc - 1u + (c % 3u);
-        const uint32_t lo = S.tstart[e], hi = S.tstart[e + 1];
-        const uint32_t gb = S.gstart[e] - lo;  // slot = gb + tile index
-        const uint32_t sb = kStaged ? 0u : gb;
-        for (uint32_t t = lo; t < hi; t += 4u) {
-            F3 pj[4];
-#pragma unroll
-            for (uint32_t i = 0; i < 4u; ++i)  // the tile is padded: no clamp
-                pj[i] = f3of(kStaged ? src[t + i] : src[sb + min(t + i, hi - 1u)]);
-            uint32_t m = 0;
-#pragma unroll
-            for (uint32_t i = 0; i < 4u; ++i) {
-                const F3 d = self - pj[i];
-                const float r2 = __builtin_fmaf(d.z, d.z, __builtin_fmaf(d.y, d.y, d.x * d.x));
-                m |= (r2 < h2) ? (1u << i) : 0u;
-            }
-            m &= (hi - t >= 4u) ? 0xFu : ((1u << (hi - t)) - 1u);
-            // keep the first ncap - cnt hits of the group; any beyond them
-            // truncate the list
-            const uint32_t room = ncap - cnt;
-            bool full = false;
-            while ((uint32_t)__builtin_popcount(m) > room) {
-                m &= ~(0x80000000u >> __builtin_clz(m));
-                full = true;
-            }
-            while (m) {
-                const uint32_t i = (uint32_t)__builtin_ctz(m);
-                m &= m - 1u;
-                *dst = gb + t + i;
-                ++cnt;
-                dst += ((cnt & 3u) == 0u) ? jump : 1u;
-            }
-            if (full) {
-                trunc = true;
-                return cnt;
-            }
-        }
-    }
-    return cnt;
-}
-
-// The same filter from global memory, for units whose neighbourhood exceeds
-// the tile: candidate x*_j = Pf[j] by slot.  In a big cell, groups out of
-// range are skipped, a group wholly in range is listed without tests, and a
-// single group left is scanned through aux when that skips a quarter of the
-// cell or more.  Every scan is one loop whose slots come, per lane, from aux
-// or from the cell's own run, the next group's slots in flight.  Returns
-// kDeferred, leaving the list unfinished, before a range that would take the
-// candidates tested past `budget` (only a neighbourhood holding a cell of
-// more than kSmallCell particles can: 27 * kSmallCell < kHeavyScan).
-__device__ __forceinline__ uint32_t ns_filter_global(const UnitShared& S, uint32_t W, uint32_t kc, F3 self,
-                                                     float h2, uint32_t ncap, const float4* __restrict__ Pf,
-                                                     CellView b, uint32_t* __restrict__ nl, uint32_t cap,
-                                                     uint32_t g, uint32_t budget, bool& trunc) {
-    uint32_t* __restrict__ dst = nl + list_at(cap, g, 0u);  // where entry cnt goes
-    const size_t jump = (size_t)4u * cap - 3u;              // from entry 4q+3 to 4q+4
-    uint32_t cnt = 0;
-    for (uint32_t c = 0; c < 27u; ++c) {
-        const uint32_t e = (c / 3u) * (W + 2u) + kc - 1u + (c % 3u);
-        const uint32_t o0 = S.gstart[e], ncell = S.tstart[e + 1] - S.tstart[e];
-        uint32_t p0 = 0, p1 = ncell;
-        bool via = false;
-        if (ncell > kSmallCell) {
-            const BigPart bp = big_part<false>(b.bseg + b.bslot[o0], self, h2, ncell);
-            if (bp.how == 0u) continue;
-            if (bp.all_in) {
-                // every member of the group is a pair: its first slots, ascending
-                const uint32_t room = ncap - cnt, size = bp.p1 - bp.p0, take = min(room, size);
-                for (uint32_t q = 0; q < take; ++q) {
-                    *dst = bp.how == 2u ? b.aux[o0 + bp.p0 + q] : o0 + bp.p0 + q;
-                    ++cnt;
-                    dst += ((cnt & 3u) == 0u) ? jump : 1u;
-                }
-                if (size > room) {
-                    trunc = true;
-                    return cnt;
-                }
-                continue;
-            }
-            if (aux_pays(bp, ncell)) {
-                p0 = bp.p0;
-                p1 = bp.p1;
-                via = true;
-            }
-        }
-        if (p1 == p0) continue;
-        if (p1 - p0 > budget) return kDeferred;
-        budget -= p1 - p0;
-        const uint32_t* __restrict__ ax = b.aux + o0;
-        uint32_t jn[4];
-#pragma unroll
-        for (uint32_t i = 0; i < 4u; ++i) jn[i] = via ? ax[min(p0 + i, p1 - 1u)] : o0 + min(p0 + i, p1 - 1u);
-        for (uint32_t p = p0; p < p1; p += 4u) {
-            const uint32_t j[4] = {jn[0], jn[1], jn[2], jn[3]};
-            F3 pj[4];
-#pragma unroll
-            for (uint32_t i = 0; i < 4u; ++i) pj[i] = f3of(Pf[j[i]]);
-#pragma unroll
-            for (uint32_t i = 0; i < 4u; ++i)
-                jn[i] = via ? ax[min(p + 4u + i, p1 - 1u)] : o0 + min(p + 4u + i, p1 - 1u);
-            uint32_t m = 0;
-#pragma unroll
-            for (uint32_t i = 0; i < 4u; ++i) m |= pair_test<false>(self - pj[i], h2) ? (1u << i) : 0u;
-            m &= (p1 - p >= 4u) ? 0xFu : ((1u << (p1 - p)) - 1u);
-            // keep the first ncap - cnt hits of the group; any beyond them
-            // truncate the list
-            const uint32_t room = ncap - cnt;
-            bool full = false;
-            while ((uint32_t)__builtin_popcount(m) > room) {
-                m &= ~(0x80000000u >> __builtin_clz(m));
-                full = true;
-            }
-            while (m) {
-                const uint32_t i = (uint32_t)__builtin_ctz(m);
-                m &= m - 1u;
-                *dst = pick4(j, i);
-                ++cnt;
-                dst += ((cnt & 3u) == 0u) ? jump : 1u;
-            }
-            if (full) {
-                trunc = true;
-                return cnt;
-            }
-        }
-    }
-    return cnt;
-}
-
-template <bool kB>
-__global__ __launch_bounds__(kBlock) void k_ns(Bufs b, Scenes<kB> SC, uint32_t tile_cap) {
-    __shared__ UnitShared S;
-    extern __shared__ float4 smem[];
-    F3* tile = reinterpret_cast<F3*>(smem);  // x*, 12 bytes a candidate
-    const float4* __restrict__ Pf = b.Pf;
-    uint32_t* __restrict__ nl = b.nlist;
-    const uint32_t cap = b.cap;
-    const uint32_t nU = b.ctr[CTR_UNITS];
-    uint32_t u0, u1, us;
-    unit_range(nU, u0, u1, us);
+// ncnt[slot].  Every slot by a group of eight lanes (the first ngroup
+// workgroups, unless the step has big cells: k_ns_big); the rest of the grid
+// walks the work items for their statistics.
+template <bool kB, bool kWide>
+__global__ __launch_bounds__(kBlock) void k_ns_groups(Bufs b, Scenes<kB> SC, uint32_t tile_cap, uint32_t ngroup) {
+    __shared__ GroupShared GS;
     Tally tl;
-    for (uint32_t u = u0; u < u1; u += us) {
-        const uint2 unit = b.units[u];
-        const uint32_t sc = scene_index<kB>(b.kbase, b.nscenes, unit.x);
-        const Grid G = SC[sc].G;
-        const float h2 = SC[sc].P.h2;
-        const uint32_t ncap = (uint32_t)SC[sc].P.cap;
-        const UnitInfo I = unit_setup(G, b.offset, unit, tile_cap, S, tl);
-        // a neighbourhood larger than the tile (any size) is filtered from global memory
-        if (I.staged) load_runs(S, I, [&](uint32_t t, uint32_t g) { tile[t] = f3of(Pf[g]); });
-        __syncthreads();
-        for (uint32_t q = threadIdx.x; q < I.n_own; q += kBlock) {
-            const uint32_t ts = I.own_t0 + q, g = I.own_g0 + q;
-            const uint32_t kc = own_column(S, I.W, ts);
-            bool trunc = false;
-            const uint32_t cnt =
-                I.staged ? ns_filter<true>(S, I.W, kc, tile[ts], h2, ncap, tile, nl, cap, g, trunc)
-                         : ns_filter_global(S, I.W, kc, f3of(Pf[g]), h2, ncap, Pf, cell_view(b), nl, cap, g,
-                                            kHeavyScan, trunc);
-            if (cnt == kDeferred) {  // a long scan: k_ns_heavy builds this list with a whole wave
-                queue_push(b, CTR_NSHEAVY, g);
-            } else {
-                b.ncnt[g] = cnt;
-                tl.trunc += trunc ? 1u : 0u;
-            }
-        }
-        __syncthreads();
+    if (blockIdx.x < ngroup) {
+        if (big_cells(b)) return;
+        const uint32_t g = xcd_block(blockIdx.x, ngroup) * kGroups + threadIdx.x / kGroup;
+        const bool active = g < b.offset[b.CT];
+        by_scene<kB>((kB && active) ? b.sid[g] : 0u, active,
+                     [&](uint32_t sc) { group_search<false, kWide>(GS, b, SC[sc], g, tl); });
+    } else {
+        item_stats<kB>(b, SC, b.units, b.ctr[CTR_UNITS], tile_cap, (blockIdx.x - ngroup) * kBlock + threadIdx.x,
+                       (gridDim.x - ngroup) * kBlock, tl, [](uint2) {});
     }
     flush_tally(b.ctr, tl);
 }
 
-// The search list of one queued slot g (x* = self), built by a whole wave:
+// The search list of slot g (x* = self), built by a whole wave:
 // the 27 cells around its cell in z,y,x order with the same ranges and group
-// skips as ns_filter_global, 64 candidates at a time, lane l testing the
+// skips as group_list, 64 candidates at a time, lane l testing the
 // l-th, the hits appended in slot order through a ballot; the first ncap
 // are kept and trunc is set when there are more.  Called by all lanes of the
 // wave; every value it depends on is the same on every lane.
@@ -1178,31 +1142,38 @@ __device__ uint32_t ns_heavy_list(const Grid& G, CellView b, const float4* __res
     return n;
 }
 
-// The search lists k_ns queued (global-memory filters that would test more
-// than kHeavyScan candidates): one wave per slot, then its count and
-// truncation tally as k_ns would have written them.
-template <bool kB>
-__global__ __launch_bounds__(1024) void k_ns_heavy(Bufs b, Scenes<kB> SC) {
-    const uint32_t nh = min(b.ctr[CTR_NSHEAVY], b.cap);
-    if (nh == 0u) return;  // uniform over the grid
-    const uint32_t waves = (gridDim.x * blockDim.x) >> 6;
-    const uint32_t w0 = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-    const CellView cv = cell_view(b);
-    const bool any_big = big_cells(b);
+// The search lists of a step with big cells (a step without them has its lists
+// from k_ns_groups): 32 slots a workgroup at a time by groups of eight lanes;
+// a list of more than kHeavyScan candidates is then built by its group's whole
+// wave.
+template <bool kB, bool kWide>
+__global__ __launch_bounds__(kBlock) void k_ns_big(Bufs b, Scenes<kB> SC) {
+    if (!big_cells(b)) return;  // uniform over the grid
+    __shared__ GroupShared GS;
     Tally tl;
-    for (uint32_t h = w0; h < nh; h += waves) {
-        const uint32_t g = __builtin_amdgcn_readfirstlane(b.crank[h]);
-        const uint32_t sc = kB ? __builtin_amdgcn_readfirstlane(b.sid[g]) : 0u;
-        const Grid G = SC[sc].G;
-        const float h2 = SC[sc].P.h2;
-        const uint32_t ncap = (uint32_t)SC[sc].P.cap;
-        const F3 self = f3of(b.Pf[g]);
-        bool trunc = false;
-        const uint32_t n = any_big ? ns_heavy_list<true>(G, cv, b.Pf, self, h2, ncap, b.nlist, b.cap, g, trunc)
-                                   : ns_heavy_list<false>(G, cv, b.Pf, self, h2, ncap, b.nlist, b.cap, g, trunc);
-        if (lane_id() == 0u) {
-            b.ncnt[g] = n;
-            tl.trunc += trunc ? 1u : 0u;
+    const uint32_t nl = b.offset[b.CT], nblk = (nl + kGroups - 1u) / kGroups;
+    for (uint32_t c = blockIdx.x; c < nblk; c += gridDim.x) {
+        const uint32_t g = c * kGroups + threadIdx.x / kGroup;
+        const bool active = g < nl;
+        bool left = false;
+        by_scene<kB>((kB && active) ? b.sid[g] : 0u, active,
+                     [&](uint32_t sc) { left = group_search<true, kWide>(GS, b, SC[sc], g, tl); });
+        uint64_t todo = __ballot(left && (lane_id() & (kGroup - 1u)) == 0u);
+        if (todo && lane_id() == 0u) atomicAdd(&b.ctr[CTR_NSHEAVY], (uint32_t)__popcll(todo));
+        while (todo) {
+            const int src = __ffsll((unsigned long long)todo) - 1;
+            todo &= todo - 1ull;
+            const uint32_t gw = (uint32_t)__builtin_amdgcn_readlane((int)g, src);
+            const uint32_t sc = kB ? __builtin_amdgcn_readfirstlane(b.sid[gw]) : 0u;
+            const Grid G = SC[sc].G;
+            const uint32_t ncap = (uint32_t)SC[sc].P.cap;
+            bool trunc = false;
+            const uint32_t n = ns_heavy_list<true>(G, cell_view(b), b.Pf, f3of(b.Pf[gw]), SC[sc].P.h2, ncap, b.nlist,
+                                                   b.cap, gw, trunc);
+            if (lane_id() == 0u) {
+                b.ncnt[gw] = n;
+                tl.trunc += trunc ? 1u : 0u;
+            }
         }
     }
     flush_tally(b.ctr, tl);
@@ -1211,33 +1182,26 @@ __global__ __launch_bounds__(1024) void k_ns_heavy(Bufs b, Scenes<kB> SC) {
 // ------------------------------------------------- K7: lambda
 // calcScalingFactorCUDA, memo form (pbf_constraint.cu:168-209): over the
 // frozen list, s = C / (m^2 inv_rho0^2 G + eps) with the reference's fma
-// order; writes (x*, s).  One thread per slot.
-template <bool kB>
+// order; writes (x*, s).  L lanes per slot (sum_pairs).
+template <bool kB, int L>
 __global__ __launch_bounds__(256) void k_lambda(Bufs b, Scenes<kB> SC) {
-    const uint32_t i = xcd_block() * blockDim.x + threadIdx.x;
+    const uint32_t t = xcd_block() * blockDim.x + threadIdx.x;
+    const uint32_t i = t / L, l = t % L;
     const bool active = i < b.offset[b.CT];
     by_scene<kB>((kB && active) ? b.sid[i] : 0u, active, [&](uint32_t sc) {
         const Phys P = SC[sc].P;
-        const float4* __restrict__ Pf = b.Pf;
-        const uint32_t* __restrict__ nl = b.nlist;
-        const uint32_t cap = b.cap;
-        const F3 self = f3of(Pf[i]);
-        const uint32_t n = b.ncnt[i];
-        float ks = 0.f, kg2s = 0.f;
-        F3 kgs = mk3(0.f, 0.f, 0.f);
-        walk_list(nl, cap, i, n, Pf, [&](uint32_t, float4 pj) {
-            float W;
-            F3 kg;
-            pair_terms(self, f3of(pj), P, W, kg);
-            const float kg2 = fdot(kg, kg);
-            ks += W;
-            acc(kgs, kg);
-            kg2s += kg2;
+        const F3 self = f3of(b.Pf[i]);
+        float a[5] = {0.f, 0.f, 0.f, 0.f, 0.f};  // sum W, sum kg, sum |kg|^2
+        sum_pairs<L>(b.nlist, b.cap, i, l, b.ncnt[i], self, b.Pf, P, a, [&](float W, F3 kg, float4, float(&c)[5]) {
+            c[0] = W;
+            c[1] = kg.x;
+            c[2] = kg.y;
+            c[3] = kg.z;
+            c[4] = fdot(kg, kg);
         });
-        const float Cc = __builtin_fmaf(ks * P.m, P.inv_rho0, -1.f);
-        const float Gs =
-            __builtin_fmaf(kgs.x, kgs.x, __builtin_fmaf(kgs.z, kgs.z, __builtin_fmaf(kgs.y, kgs.y, kg2s)));
-        b.Q[i] = make_float4(self.x, self.y, self.z, Cc / __builtin_fmaf(P.m2r2, Gs, P.relax));
+        const float Cc = __builtin_fmaf(a[0] * P.m, P.inv_rho0, -1.f);
+        const float Gs = __builtin_fmaf(a[1], a[1], __builtin_fmaf(a[3], a[3], __builtin_fmaf(a[2], a[2], a[4])));
+        if (l == 0u) b.Q[i] = make_float4(self.x, self.y, self.z, Cc / __builtin_fmaf(P.m2r2, Gs, P.relax));
     });
 }
 
@@ -1245,29 +1209,23 @@ __global__ __launch_bounds__(256) void k_lambda(Bufs b, Scenes<kB> SC) {
 // calcPositionUpdateCUDA (memo form, pbf_position_update.cu:131-188),
 // responseCollisionCUDA (pbf_response_collision.cu:12-66) and
 // updateInterimPositionCUDA (pbf_constraint.cu:335-345).  Reads (x*, s),
-// writes the new x*.  One thread per slot.  kPow4: every scene's s_corr
-// exponent is 4, so powi unrolls to its two squarings at compile time.
-template <bool kB, bool kPow4>
+// writes the new x*.  L lanes per slot (sum_pairs).  kPow4: every scene's
+// s_corr exponent is 4, so powi unrolls to its two squarings at compile time.
+template <bool kB, bool kPow4, int L>
 __global__ __launch_bounds__(256) void k_deltap(Bufs b, Scenes<kB> SC) {
-    const uint32_t i = xcd_block() * blockDim.x + threadIdx.x;
+    const uint32_t t = xcd_block() * blockDim.x + threadIdx.x;
+    const uint32_t i = t / L, l = t % L;
     const bool active = i < b.offset[b.CT];
     Tally tl;
     by_scene<kB>((kB && active) ? b.sid[i] : 0u, active, [&](uint32_t sc) {
         const Phys P = SC[sc].P;
         const Boundary B = SC[sc].B;
-        const float4* __restrict__ Q = b.Q;
-        const uint32_t* __restrict__ nl = b.nlist;
-        const uint32_t cap = b.cap;
-        const float4 se = Q[i];
+        const float4 se = b.Q[i];
         const F3 self = f3of(se);
         const float si = se.w;
         const float self_cl = (si < 0.f) ? -si : 0.f;
-        const uint32_t n = b.ncnt[i];
-        F3 sum = mk3(0.f, 0.f, 0.f);
-        walk_list(nl, cap, i, n, Q, [&](uint32_t, float4 pe) {
-            float W;
-            F3 kg;
-            pair_terms(self, f3of(pe), P, W, kg);
+        float sum[3] = {0.f, 0.f, 0.f};
+        sum_pairs<L>(b.nlist, b.cap, i, l, b.ncnt[i], self, b.Q, P, sum, [&](float W, F3 kg, float4 pe, float(&c)[3]) {
             const float sj = pe.w;
             float corr;
             if (P.mode == 0) {
@@ -1280,18 +1238,22 @@ __global__ __launch_bounds__(256) void k_deltap(Bufs b, Scenes<kB> SC) {
             } else {
                 corr = P.sk * powi(W * P.inv_wdq, kPow4 ? 4 : P.sn);
             }
-            const float a = -(si + sj + corr);
-            acc(sum, mulsv(a, kg));
+            const F3 ak = mulsv(-(si + sj + corr), kg);
+            c[0] = ak.x;
+            c[1] = ak.y;
+            c[2] = ak.z;
         });
-        F3 dp = mk3(sum.x * P.m * P.inv_rho0, sum.y * P.m * P.inv_rho0, sum.z * P.m * P.inv_rho0);
+        F3 dp = mk3(sum[0] * P.m * P.inv_rho0, sum[1] * P.m * P.inv_rho0, sum[2] * P.m * P.inv_rho0);
         bool capped = false;
         const int sw = (B.n_planes == 6 && B.n_inner == 0 && B.n_outer == 0)
                            ? collide_planes<6>(P, B, dp, self, capped)
                            : collide(P, B, dp, self, capped);
         const F3 np = self + dp;
-        b.Pf[i] = make_float4(np.x, np.y, np.z, 0.f);
-        tl.sweepcap = capped ? 1u : 0u;
-        tl.maxsweep = (uint32_t)sw;
+        if (l == 0u) {
+            b.Pf[i] = make_float4(np.x, np.y, np.z, 0.f);
+            tl.sweepcap = capped ? 1u : 0u;
+            tl.maxsweep = (uint32_t)sw;
+        }
     });
     flush_tally(b.ctr, tl);
 }
@@ -1322,12 +1284,13 @@ __global__ __launch_bounds__(256) void k_cur_hash(Bufs b, Scenes<kB> SC, uint32_
         const Scene& S = SC[sc];
         const F3 p = f3of(b.Pf[s]);
         const F3 vv = mulsv(S.P.inv_dt, p - ld3(b.X, b.cap, s));
-        b.R[2 * s] = make_float4(p.x, p.y, p.z, 0.f);
-        b.R[2 * s + 1] = make_float4(vv.x, vv.y, vv.z, 0.f);
         const Grid G = S.G;
         int gp[3];
         grid_pos(p, G.cw, gp);
-        k = ((scene_key(gp[0], gp[1], gp[2], G) >> lguw) << lgnc) | (blockIdx.x & ((1u << lgnc) - 1u));
+        k = scene_key(gp[0], gp[1], gp[2], G);
+        b.R[2 * s] = make_float4(p.x, p.y, p.z, __uint_as_float(k));
+        b.R[2 * s + 1] = make_float4(vv.x, vv.y, vv.z, 0.f);
+        k = ((k >> lguw) << lgnc) | (blockIdx.x & ((1u << lgnc) - 1u));
     });
     // the final boxes of the big cells' groups (the marks k_big_seg left)
     const uint32_t bm = active ? b.rank[s] : 0u;
@@ -1366,177 +1329,12 @@ __global__ __launch_bounds__(256) void k_cur_scatter(const uint32_t* __restrict_
 // lists with every lane busy.  Adding only the cells that have pairs gives
 // the same sums: the skipped cells add +0.
 
-// Keeps the first `room` set bits of a group's hit mask; returns whether any
-// were dropped.
-__device__ __forceinline__ bool clip_hits(uint32_t& m, uint32_t room) {
-    bool full = false;
-    while ((uint32_t)__builtin_popcount(m) > room) {
-        m &= ~(0x80000000u >> __builtin_clz(m));
-        full = true;
-    }
-    return full;
-}
-
-// Emits the in-range tile elements of the staged neighbourhood around own
-// column kc, in order: emit(slot, first pair of its cell), which counts them
-// in n; stops once n reaches lim.
-template <class EmitF>
-__device__ __forceinline__ void list_tile(const UnitInfo& I, const UnitShared& S, const F3* __restrict__ tp,
-                                          uint32_t kc, F3 self, float cut2, const uint32_t& n, uint32_t lim,
-                                          EmitF&& emit) {
-    for (uint32_t q = 0; q < 27u; ++q) {
-        const uint32_t e = (q / 3u) * (I.W + 2u) + kc - 1u + (q % 3u);
-        const uint32_t lo = S.tstart[e], hi = S.tstart[e + 1];
-        const uint32_t gb = S.gstart[e] - lo;  // slot = gb + tile index
-        bool first = true;
-        for (uint32_t t = lo; t < hi; t += 4u) {
-            F3 el[4];
-#pragma unroll
-            for (uint32_t i = 0; i < 4u; ++i) el[i] = tp[t + i];  // the tile is padded: no clamp
-            uint32_t m = 0;
-#pragma unroll
-            for (uint32_t i = 0; i < 4u; ++i) {
-                const F3 d = el[i] - self;
-                m |= !(glm_dot(d, d) > cut2) ? (1u << i) : 0u;
-            }
-            m &= (hi - t >= 4u) ? 0xFu : ((1u << (hi - t)) - 1u);
-            const bool full = clip_hits(m, lim - n);
-            while (m) {
-                const uint32_t i = (uint32_t)__builtin_ctz(m);
-                m &= m - 1u;
-                emit(gb + t + i, first);
-                first = false;
-            }
-            if (full || n == lim) return;
-        }
-    }
-}
-
-// The same from global memory, row by row (dz outer, dy inner), the next
-// row's three cell ranges loaded while the current row is filtered; pos(j)
-// gives x*_j.  kBig (the step has big cells): a big cell's groups out of
-// range are skipped by their final boxes, one wholly in range is listed
-// without tests, and the scan stops at once when such groups alone take the
-// list to lim.  Stops once n reaches lim.  kBig: returns false, leaving the
-// list unfinished, before a cell that would take the candidates tested past
-// `budget` (at least 27 * kSmallCell).
-template <bool kBig, class PosF, class EmitF>
-__device__ __forceinline__ bool list_global(const Grid& G, CellView b, F3 self, float cut2, uint32_t& n,
-                                            uint32_t lim, uint32_t budget, PosF&& pos, EmitF&& emit) {
-    const uint32_t* __restrict__ offset = b.offset;
-    int gp[3];
-    grid_pos(self, G.cw, gp);
-    auto row = [&](int r, uint32_t* st, uint32_t* en) {
-#pragma unroll
-        for (int dx = 0; dx < 3; ++dx) {
-            const uint32_t c = scene_key(gp[0] + dx - 1, gp[1] + (r % 3) - 1, gp[2] + (r / 3) - 1, G);
-            st[dx] = offset[c];
-            en[dx] = offset[c + 1];
-        }
-    };
-    uint32_t st[3], en[3];
-    row(0, st, en);
-    for (int r = 0; r < 9; ++r) {
-        uint32_t ns[3] = {0, 0, 0}, ne[3] = {0, 0, 0};
-        if (r < 8) row(r + 1, ns, ne);
-#pragma unroll
-        for (int dx = 0; dx < 3; ++dx) {
-            bool first = true;
-            if (!kBig) {
-                // a step without big cells: the plain scan (27 cells of at
-                // most kSmallCell particles stay within any budget)
-                for (uint32_t j = st[dx]; j < en[dx]; j += 4u) {
-                    F3 pj[4];
-#pragma unroll
-                    for (uint32_t i = 0; i < 4u; ++i) pj[i] = pos(min(j + i, en[dx] - 1u));
-                    uint32_t m = 0;
-#pragma unroll
-                    for (uint32_t i = 0; i < 4u; ++i) m |= pair_test<true>(pj[i] - self, cut2) ? (1u << i) : 0u;
-                    m &= (en[dx] - j >= 4u) ? 0xFu : ((1u << (en[dx] - j)) - 1u);
-                    const bool full = clip_hits(m, lim - n);
-                    while (m) {
-                        const uint32_t i = (uint32_t)__builtin_ctz(m);
-                        m &= m - 1u;
-                        emit(j + i, first);
-                        first = false;
-                    }
-                    if (full || n == lim) return true;
-                }
-                continue;
-            }
-            const uint32_t o0 = st[dx], ncell = en[dx] - st[dx];
-            uint32_t p0 = 0, p1 = ncell;
-            bool via = false;
-            if (ncell > kSmallCell) {
-                const BigPart bp = big_part<true>(b.bseg + b.bslot[o0], self, cut2, ncell);
-                if (bp.how == 0u) continue;
-                if (n + bp.inside >= lim) {  // the list reaches lim here: no need to store it
-                    n = lim;
-                    return true;
-                }
-                if (bp.all_in) {  // fewer than lim - n members, all pairs
-                    for (uint32_t q = bp.p0; q < bp.p1; ++q) {
-                        emit(bp.how == 2u ? b.aux[o0 + q] : o0 + q, first);
-                        first = false;
-                    }
-                    continue;
-                }
-                if (aux_pays(bp, ncell)) {
-                    p0 = bp.p0;
-                    p1 = bp.p1;
-                    via = true;
-                }
-            }
-            if (p1 == p0) continue;
-            if (p1 - p0 > budget) return false;
-            budget -= p1 - p0;
-            const uint32_t* __restrict__ ax = b.aux + o0;
-            uint32_t jn[4];
-#pragma unroll
-            for (uint32_t i = 0; i < 4u; ++i) jn[i] = via ? ax[min(p0 + i, p1 - 1u)] : o0 + min(p0 + i, p1 - 1u);
-            for (uint32_t p = p0; p < p1; p += 4u) {
-                const uint32_t jj[4] = {jn[0], jn[1], jn[2], jn[3]};
-                F3 pj[4];
-#pragma unroll
-                for (uint32_t i = 0; i < 4u; ++i) pj[i] = pos(jj[i]);
-#pragma unroll
-                for (uint32_t i = 0; i < 4u; ++i)
-                    jn[i] = via ? ax[min(p + 4u + i, p1 - 1u)] : o0 + min(p + 4u + i, p1 - 1u);
-                uint32_t m = 0;
-#pragma unroll
-                for (uint32_t i = 0; i < 4u; ++i) m |= pair_test<true>(pj[i] - self, cut2) ? (1u << i) : 0u;
-                m &= (p1 - p >= 4u) ? 0xFu : ((1u << (p1 - p)) - 1u);
-                const bool full = clip_hits(m, lim - n);
-                while (m) {
-                    const uint32_t i = (uint32_t)__builtin_ctz(m);
-                    m &= m - 1u;
-                    emit(pick4(jj, i), first);
-                    first = false;
-                }
-                if (full || n == lim) return true;
-            }
-        }
-#pragma unroll
-        for (int dx = 0; dx < 3; ++dx) {
-            st[dx] = ns[dx];
-            en[dx] = ne[dx];
-        }
-    }
-    return true;
-}
-
 // A candidate's records for a pass's term: p = (x*_j, pass-specific w),
 // q = the second record the pass needs (the velocity, or unused).  Loaded
 // together by the sums, so no load waits on another.
 struct El2 {
     float4 p, q;
 };
-
-// Key of cell c (0..26, in z,y,x order) of the 27 around grid position gp.
-__device__ __forceinline__ uint32_t cell27(const int gp[3], uint32_t c, const Grid& G) {
-    const int dz = (int)(c / 9u) - 1, q = (int)(c % 9u);
-    return scene_key(gp[0] + (q % 3) - 1, gp[1] + (q / 3) - 1, gp[2] + dz, G);
-}
 
 // Partial sum of one cell (key) in slot order: the per-cell sum of
 // calcContribution; elem(j) builds the pass's element of slot j.  A big
@@ -1605,23 +1403,11 @@ __device__ __forceinline__ F3 sum27_global(const Grid& G, CellView b, F3 self, f
     return sum;
 }
 
-// Particles of final-cell runs too sparse for a unit (fewer than kSparse
-// particles in their run of uw cells): one thread each, in final-cell order
-// so that the lanes of a wave share their neighbourhoods' cache lines, with
-// a contiguous share of that order per XCD.  Sparse runs are contiguous
-// stretches of the order.  body(q, g): position q in that order, slot g.
-template <class F>
-__device__ __forceinline__ void for_sparse(const Bufs& b, uint32_t lgnc, F&& body) {
-    const uint32_t nl = b.offset[b.CT];
-    uint32_t c0, c1, cs;
-    unit_range((nl + kBlock - 1) / kBlock, c0, c1, cs);
-    for (uint32_t c = c0; c < c1; c += cs) {
-        const uint32_t q = c * kBlock + threadIdx.x;
-        if (q >= nl) continue;
-        const uint32_t g = b.cperm[q];
-        const uint32_t run = b.ckey[g] >> lgnc;
-        if (b.coffset[(run + 1u) << lgnc] - b.coffset[run << lgnc] < kSparse) body(q, g);
-    }
+// Whether the final-cell run of slot g is too sparse for a unit (fewer than
+// kSparse particles).
+__device__ __forceinline__ bool sparse_run(const Bufs& b, uint32_t lgnc, uint32_t g) {
+    const uint32_t run = b.ckey[g] >> lgnc;
+    return b.coffset[(run + 1u) << lgnc] - b.coffset[run << lgnc] < kSparse;
 }
 
 // Own particles of a final-run work item: positions coffset[run] + chunk*kChunk .. of the run order.
@@ -1634,13 +1420,6 @@ __device__ __forceinline__ OwnCur own_cur(const Bufs& b, uint2 unit, uint32_t lg
     o.c0 = b.coffset[run << lgnc] + skip;
     o.n = min(kChunk, b.coffset[(run + 1u) << lgnc] - o.c0);
     return o;
-}
-
-// Own column (1..W) of a final-cell unit's particle at position p.
-__device__ __forceinline__ uint32_t final_column(const Grid& G, const UnitInfo& I, F3 p) {
-    int gp[3];
-    grid_pos(p, G.cw, gp);
-    return (((uint32_t)gp[0] & (G.gx - 1u)) - I.xb) + 1u;
 }
 
 // ------------------------------------------------- overflow slots
@@ -1671,108 +1450,52 @@ __device__ __forceinline__ uint32_t ovf_mark(const Bufs& b, uint32_t q) {
 // their count, or kFinalK + 1 when there are more (the passes then fall back
 // to the direct sum, so the filter stops at the (kFinalK+1)-th pair: a
 // particle in a pile of thousands does not scan its whole neighbourhood).
-template <bool kB>
-__global__ __launch_bounds__(kBlock) void k_final_list(Bufs b, Scenes<kB> SC, uint32_t tile_cap, uint32_t lguw, uint32_t lgnc) {
-    static_assert(kChunk <= kBlock, "one own particle per thread");
-    __shared__ UnitShared S;
-    __shared__ uint32_t colpos[kMaxW + 2];  // own particles per final column, then each column's first position
-    __shared__ uint32_t corder[kChunk];     // the item's own slots in final-column order
-    extern __shared__ float4 smem[];
-    F3* tp = reinterpret_cast<F3*>(smem);  // x*, 12 bytes a candidate
-    // the final x*, packed: the same values as the passes' records R (built
-    // from Pf), at half the bytes per candidate
-    const float4* __restrict__ Pf = b.Pf;
-    const uint32_t cap = b.cap;
-    uint32_t* __restrict__ fl = b.flist;
-    const CellView cv = cell_view(b);
-    const bool any_big = big_cells(b);
-    Tally tl;
-    UnitInfo I;
-    // inlined at both call sites: a call would copy the kernel arguments to scratch memory
-    auto build = [&](uint32_t q, uint32_t g, bool tiled, const Grid& G, float cut2) __attribute__((always_inline)) {
-        const F3 self = f3of(Pf[g]);
-        uint32_t n = 0;
-        uint32_t* __restrict__ dst = fl + list_at(cap, q, 0u);  // where entry n goes
-        const size_t jump = (size_t)4u * cap - 3u;              // from entry 4q+3 to 4q+4
-        // the (kFinalK+1)-th pair is counted, not stored: it marks the overflow
-        auto emit = [&](uint32_t j, bool first) {
-            if (n < kFinalK) {
-                *dst = j | (first ? 0x80000000u : 0u);
-                dst += (((n + 1u) & 3u) == 0u) ? jump : 1u;
-            }
-            ++n;
-        };
-        if (tiled) {
-            list_tile(I, S, tp, final_column(G, I, self), self, cut2, n, kFinalK + 1u, emit);
-        } else if (any_big) {
-            if (!list_global<true>(G, cv, self, cut2, n, kFinalK + 1u, kHeavyScan,
-                                   [&](uint32_t j) { return f3of(Pf[j]); }, emit)) {
-                queue_push(b, CTR_HEAVY, q);  // a long scan: k_final_heavy builds this list with a whole wave
-                return;
-            }
-        } else {
-            list_global<false>(G, cv, self, cut2, n, kFinalK + 1u, kHeavyScan, [&](uint32_t j) { return f3of(Pf[j]); },
-                               emit);
-        }
-        if (n > kFinalK) n = ovf_mark(b, q);
-        b.fcnt[q] = n;
+__device__ __forceinline__ float final_cut2(const Phys& P) { return fmaxf(P.cut2_w, P.cut2_wd); }
+
+// The final list of position q (slot g) by its group of eight lanes, and its
+// count or overflow entry; true when the list is left to a whole wave instead.
+template <bool kBig, bool kWide>
+__device__ __forceinline__ bool group_final(GroupShared& S, const Bufs& b, const Scene& sc, uint32_t q, uint32_t g,
+                                            Tally& tl) {
+    const Grid G = sc.G;
+    const float4 pk = b.R[2 * g];
+    const uint32_t n = group_list<true, kBig, kWide>(S, G, cell_view(b), b.Pf, f3of(pk), __float_as_uint(pk.w),
+                                                     final_cut2(sc.P), kFinalK, b.flist, b.cap, q, g, kHeavyScan);
+    if (kBig && n == kDeferred) return true;
+    if ((lane_id() & (kGroup - 1u)) == 0u) {
+        b.fcnt[q] = n > kFinalK ? ovf_mark(b, q) : n;
         tl.listovf += n > kFinalK ? 1u : 0u;
-    };
-    auto cut2_of = [&](uint32_t sc) { return fmaxf(SC[sc].P.cut2_w, SC[sc].P.cut2_wd); };
-    const uint32_t nU = b.ctr[CTR_CUNITS];
-    uint32_t u0, u1, us;
-    unit_range(nU, u0, u1, us);
-    for (uint32_t u = u0; u < u1; u += us) {
-        const uint2 unit = b.cunits[u];
-        const uint32_t sc = scene_index<kB>(b.kbase, b.nscenes, unit.x);
-        const Grid G = SC[sc].G;
-        const float cut2 = cut2_of(sc);
-        for (uint32_t c = threadIdx.x; c < kMaxW + 2u; c += kBlock) colpos[c] = 0u;
-        I = unit_setup(G, b.offset, unit, tile_cap, S, tl);  // barriers order the clearing above
-        // The item's own particles are put in final-column order (a
-        // counting sort in LDS), written back to cperm, so that the lanes
-        // of a wave share their candidate cells here and their pairs in
-        // the passes; the order of the particles changes no sum.
-        const OwnCur o = own_cur(b, unit, lguw, lgnc);
-        const bool mine = threadIdx.x < o.n;
-        uint32_t kc = 0, rk = 0, gm = 0;
-        if (mine) {
-            gm = b.cperm[o.c0 + threadIdx.x];
-            kc = min(final_column(G, I, f3of(Pf[gm])), I.W + 1u);
-            rk = atomicAdd(&colpos[kc], 1u);
-        }
-        if (I.staged)
-            load_runs(S, I, [&](uint32_t t, uint32_t j) { tp[t] = f3of(Pf[j]); });
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            uint32_t run = 0;
-            for (uint32_t c = 0; c <= I.W + 1u; ++c) {
-                const uint32_t k = colpos[c];
-                colpos[c] = run;
-                run += k;
-            }
-        }
-        __syncthreads();
-        if (mine) corder[colpos[kc] + rk] = gm;
-        __syncthreads();
-        if (mine) {
-            const uint32_t g = corder[threadIdx.x];
-            b.cperm[o.c0 + threadIdx.x] = g;
-            if (!I.staged) tl.slowpart++;
-            build(o.c0 + threadIdx.x, g, I.staged, G, cut2);
-        }
-        __syncthreads();
     }
-    for_sparse(b, lgnc, [&](uint32_t q, uint32_t g) {
-        tl.slowpart++;
-        by_scene<kB>(kB ? b.sid[g] : 0u, true, [&](uint32_t sc) { build(q, g, false, SC[sc].G, cut2_of(sc)); });
-    });
+    return false;
+}
+
+// Every position by a group of eight lanes (the first ngroup workgroups, unless
+// the step has big cells: k_final_big); the rest of the grid walks the work
+// items for their statistics.
+template <bool kB, bool kWide>
+__global__ __launch_bounds__(kBlock) void k_final_groups(Bufs b, Scenes<kB> SC, uint32_t tile_cap, uint32_t lguw,
+                                                         uint32_t lgnc, uint32_t ngroup) {
+    __shared__ GroupShared GS;
+    Tally tl;
+    if (blockIdx.x < ngroup) {
+        const bool any_big = big_cells(b);
+        const uint32_t q = xcd_block(blockIdx.x, ngroup) * kGroups + threadIdx.x / kGroup;
+        const bool active = q < b.offset[b.CT];
+        const uint32_t g = active ? b.cperm[q] : 0u;
+        if (active && (threadIdx.x & (kGroup - 1u)) == 0u && sparse_run(b, lgnc, g)) tl.slowpart++;
+        by_scene<kB>((kB && active) ? b.sid[g] : 0u, active && !any_big,
+                     [&](uint32_t sc) { group_final<false, kWide>(GS, b, SC[sc], q, g, tl); });
+    } else {
+        item_stats<kB>(b, SC, b.cunits, b.ctr[CTR_CUNITS], tile_cap, (blockIdx.x - ngroup) * kBlock + threadIdx.x,
+                       (gridDim.x - ngroup) * kBlock, tl,
+                       [&](uint2 unit) { tl.slowpart += own_cur(b, unit, lguw, lgnc).n; });
+    }
     flush_tally(b.ctr, tl);
 }
 
-// The final list of one queued particle (x* = self, final-order position q),
+// The final list of one particle (x* = self, final-order position q),
 // built by a whole wave: each cell's candidates (the same ranges and group
-// skips as list_global) 64 at a time, lane l testing the l-th; the hits are
+// skips as group_list) 64 at a time, lane l testing the l-th; the hits are
 // appended in slot order through a ballot.  Returns the pair count, or lim
 // once it reaches lim = kFinalK + 1 (the list then overflows and is not
 // read).  Called by all lanes of the wave; every value it depends on is the
@@ -1831,30 +1554,35 @@ __device__ uint32_t heavy_list(const Grid& G, CellView b, const float4* __restri
     return n;
 }
 
-// The final lists k_final_list queued (builds of more than kHeavyScan
-// candidates): one wave per particle, then its count or
-// overflow entry as k_final_list would have written them.
-template <bool kB>
-__global__ __launch_bounds__(1024) void k_final_heavy(Bufs b, Scenes<kB> SC) {
-    const uint32_t nh = min(b.ctr[CTR_HEAVY], b.cap);
-    if (nh == 0u) return;  // uniform over the grid
-    const uint32_t waves = (gridDim.x * blockDim.x) >> 6;
-    const uint32_t w0 = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-    const CellView cv = cell_view(b);
-    const bool any_big = big_cells(b);
+// The final lists of a step with big cells, as k_ns_big builds the search's.
+template <bool kB, bool kWide>
+__global__ __launch_bounds__(kBlock) void k_final_big(Bufs b, Scenes<kB> SC) {
+    if (!big_cells(b)) return;  // uniform over the grid
+    __shared__ GroupShared GS;
     Tally tl;
-    for (uint32_t h = w0; h < nh; h += waves) {
-        const uint32_t q = __builtin_amdgcn_readfirstlane(b.crank[h]);
-        const uint32_t g = __builtin_amdgcn_readfirstlane(b.cperm[q]);
-        const uint32_t sc = kB ? b.sid[g] : 0u;
-        const Grid G = SC[sc].G;
-        const float cut2 = fmaxf(SC[sc].P.cut2_w, SC[sc].P.cut2_wd);
-        const F3 self = f3of(b.Pf[g]);
-        const uint32_t n = any_big ? heavy_list<true>(G, cv, b.Pf, self, cut2, b.flist, b.cap, q)
-                                   : heavy_list<false>(G, cv, b.Pf, self, cut2, b.flist, b.cap, q);
-        if (lane_id() == 0u) {
-            b.fcnt[q] = n > kFinalK ? ovf_mark(b, q) : n;
-            tl.listovf += n > kFinalK ? 1u : 0u;
+    const uint32_t nl = b.offset[b.CT], nblk = (nl + kGroups - 1u) / kGroups;
+    for (uint32_t c = blockIdx.x; c < nblk; c += gridDim.x) {
+        const uint32_t q = c * kGroups + threadIdx.x / kGroup;
+        const bool active = q < nl;
+        const uint32_t g = active ? b.cperm[q] : 0u;
+        bool left = false;
+        by_scene<kB>((kB && active) ? b.sid[g] : 0u, active,
+                     [&](uint32_t sc) { left = group_final<true, kWide>(GS, b, SC[sc], q, g, tl); });
+        uint64_t todo = __ballot(left && (lane_id() & (kGroup - 1u)) == 0u);
+        if (todo && lane_id() == 0u) atomicAdd(&b.ctr[CTR_HEAVY], (uint32_t)__popcll(todo));
+        while (todo) {
+            const int src = __ffsll((unsigned long long)todo) - 1;
+            todo &= todo - 1ull;
+            const uint32_t qw = (uint32_t)__builtin_amdgcn_readlane((int)q, src);
+            const uint32_t gw = (uint32_t)__builtin_amdgcn_readlane((int)g, src);
+            const uint32_t sc = kB ? __builtin_amdgcn_readfirstlane(b.sid[gw]) : 0u;
+            const Grid G = SC[sc].G;
+            const uint32_t n = heavy_list<true>(G, cell_view(b), b.Pf, f3of(b.Pf[gw]), final_cut2(SC[sc].P), b.flist,
+                                                b.cap, qw);
+            if (lane_id() == 0u) {
+                b.fcnt[qw] = n > kFinalK ? ovf_mark(b, qw) : n;
+                tl.listovf += n > kFinalK ? 1u : 0u;
+            }
         }
     }
     flush_tally(b.ctr, tl);
@@ -1915,14 +1643,48 @@ __device__ __forceinline__ F3 sum_list_any(const uint32_t* __restrict__ fl, uint
     return sum;
 }
 
-// Visits position q of the final-cell order: body(q, slot, stored pair
-// count, scene), grouped by scene (no wave-wide operations inside).
-template <bool kB, class F>
+// sum_list by a group of L lanes (l: this lane), one entry each of every L: the
+// entries' terms and first-of-cell marks are then taken in list order by every
+// lane, which forms the same partial sums bit for bit (an entry past n adds a
+// zero term).
+template <int L, int m = 0>
+__device__ __forceinline__ void add_cell_lanes(F3& sum, F3& cs, float first, F3 t) {
+    if constexpr (m < L) {
+        if (lane_of<L, m>(first) != 0.f) {
+            acc(sum, cs);
+            cs = mk3(0.f, 0.f, 0.f);
+        }
+        acc(cs, mk3(lane_of<L, m>(t.x), lane_of<L, m>(t.y), lane_of<L, m>(t.z)));
+        add_cell_lanes<L, m + 1>(sum, cs, first, t);
+    }
+}
+template <int L, class ElemF, class TermF>
+__device__ __forceinline__ F3 sum_list_lanes(const uint32_t* __restrict__ fl, uint32_t cap, uint32_t q, uint32_t l,
+                                             uint32_t n, ElemF&& elem, TermF&& term) {
+    F3 sum = mk3(0.f, 0.f, 0.f), cs = mk3(0.f, 0.f, 0.f);
+    uint32_t e = l < n ? fl[list_at(cap, q, l)] : 0u;
+    for (uint32_t k = l; k - l < n; k += (uint32_t)L) {
+        const El2 el = elem(e & 0x7FFFFFFFu);
+        const float first = (e >> 31) ? 1.f : 0.f;
+        const bool on = k < n;
+        e = k + (uint32_t)L < n ? fl[list_at(cap, q, k + (uint32_t)L)] : 0u;
+        const F3 t = term(el);
+        add_cell_lanes<L>(sum, cs, first, on ? t : mk3(0.f, 0.f, 0.f));
+    }
+    acc(sum, cs);
+    return sum;
+}
+
+// Visits position q of the final-cell order, L lanes each (l: this lane):
+// body(q, slot, stored pair count, scene, l), grouped by scene (no operations
+// across groups inside).
+template <bool kB, int L, class F>
 __device__ __forceinline__ void for_final(const Bufs& b, F&& body) {
-    const uint32_t q = xcd_block() * blockDim.x + threadIdx.x;
+    const uint32_t t = xcd_block() * blockDim.x + threadIdx.x;
+    const uint32_t q = t / L, l = t % L;
     const bool active = q < b.offset[b.CT];
     const uint32_t g = active ? b.cperm[q] : 0u;
-    by_scene<kB>((kB && active) ? b.sid[g] : 0u, active, [&](uint32_t sc) { body(q, g, b.fcnt[q], sc); });
+    by_scene<kB>((kB && active) ? b.sid[g] : 0u, active, [&](uint32_t sc) { body(q, g, b.fcnt[q], sc, l); });
 }
 
 // The pair terms of the final passes.  Each takes its root (and the three
@@ -2026,11 +1788,13 @@ __device__ __forceinline__ F3 pass_cell(const Bufs& b, const Grid& G, const Pass
 // k_ovf_part left in its block's overflow slot, added in the same z,y,x order
 // as the direct 27-cell sum adds its cells (which it does when the block has
 // no slot).
-template <class Pass>
-__device__ __forceinline__ F3 pass_sum(const Bufs& b, const Grid& G, const Pass& ps, uint32_t q, uint32_t n) {
+template <int L, class Pass>
+__device__ __forceinline__ F3 pass_sum(const Bufs& b, const Grid& G, const Pass& ps, uint32_t q, uint32_t n,
+                                       uint32_t l) {
     auto elem = [&](uint32_t j) { return ps.elem(j); };
     auto term = [&](const El2& e) { return ps.term(e); };
     if (n <= kFinalK) {
+        if constexpr (L > 1) return sum_list_lanes<L>(b.flist, b.cap, q, l, n, elem, term);
         if (b.cap < kGatherMaxSlots / 2u) {
             const Gather16 gr(b.R, 2u * b.cap), go(b.OM4, b.cap);
             return sum_list_any(b.flist, b.cap, q, n, [&](uint32_t j) { return ps.elem_buf(gr, go, j); }, term);
@@ -2078,33 +1842,33 @@ __global__ __launch_bounds__(256) void k_ovf_part(Bufs b, Scenes<kB> SC) {
 // calcVorticityCUDA (pbf_vorticity_confinement.cu:87-115) with inv_h in the
 // spiky derivative (or h, when reproducing the reference's argument);
 // writes (omega, |omega|).  Elements: (x*_j, slot j).
-template <bool kB>
+template <bool kB, int L>
 __global__ __launch_bounds__(kBlock) void k_vort(Bufs b, Scenes<kB> SC) {
-    for_final<kB>(b, [&](uint32_t q, uint32_t g, uint32_t n, uint32_t sc) {
+    for_final<kB, L>(b, [&](uint32_t q, uint32_t g, uint32_t n, uint32_t sc, uint32_t l) {
         const Phys P = SC[sc].P;
         if (!P.vort_on) {
-            b.OM4[g] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (l == 0u) b.OM4[g] = make_float4(0.f, 0.f, 0.f, 0.f);
             return;
         }
         const float mr = P.m * P.inv_rho0;
-        const F3 w = pass_sum(b, SC[sc].G, PassTerms<PASS_VORT>(b, P, g), q, n);
+        const F3 w = pass_sum<L>(b, SC[sc].G, PassTerms<PASS_VORT>(b, P, g), q, n, l);
         const F3 om = mulsv(mr, w);
-        b.OM4[g] = make_float4(om.x, om.y, om.z, glm_length(om));
+        if (l == 0u) b.OM4[g] = make_float4(om.x, om.y, om.z, glm_length(om));
     });
 }
 
 // ------------------------------------------------- K11: vorticity confinement
 // addVorticityConfinementCUDA (pbf_vorticity_confinement.cu:192-222), in place
 // on the record's velocity.  Elements: (x*_j, |omega_j|).
-template <bool kB>
+template <bool kB, int L>
 __global__ __launch_bounds__(kBlock) void k_confine(Bufs b, Scenes<kB> SC) {
     float4* __restrict__ R = b.R;
     const float4* __restrict__ OM4 = b.OM4;
-    for_final<kB>(b, [&](uint32_t q, uint32_t g, uint32_t n, uint32_t sc) {
+    for_final<kB, L>(b, [&](uint32_t q, uint32_t g, uint32_t n, uint32_t sc, uint32_t l) {
         const Phys P = SC[sc].P;
         if (!P.vort_on) return;
-        F3 N = pass_sum(b, SC[sc].G, PassTerms<PASS_CONF>(b, P, g), q, n);
-        if (glm_length(N) > 0.f) {
+        F3 N = pass_sum<L>(b, SC[sc].G, PassTerms<PASS_CONF>(b, P, g), q, n, l);
+        if (l == 0u && glm_length(N) > 0.f) {
             N = mulvs(mulvs(N, P.m), P.inv_rho0);
             N = divvs(N, glm_length(N));
             const F3 add = mulvs(divvs(mulsv(P.vc, glm_cross(N, f3of(OM4[g]))), P.inv_rho0), P.dtc);
@@ -2118,20 +1882,23 @@ __global__ __launch_bounds__(kBlock) void k_confine(Bufs b, Scenes<kB> SC) {
 // calcXSPHCUDA (pbf_xsph.cu:84-113) and updatePosition (pbf_update.cu:16-23):
 // x_out = x*, v_out = v + c*m*inv_rho0*sum unless the sum is NaN, with v the
 // record's velocity (after confinement when that ran).
-template <bool kB>
+template <bool kB, int L>
 __global__ __launch_bounds__(kBlock) void k_xsph_out(Bufs b, Scenes<kB> SC, float* __restrict__ xo, float* __restrict__ vo) {
     const float4* __restrict__ R = b.R;
     Tally tl;
-    for_final<kB>(b, [&](uint32_t q, uint32_t g, uint32_t n, uint32_t sc) {
+    for_final<kB, L>(b, [&](uint32_t q, uint32_t g, uint32_t n, uint32_t sc, uint32_t l) {
         const Phys P = SC[sc].P;
         const F3 self = f3of(R[2 * g]);
         const F3 selfv = f3of(R[2 * g + 1]);
         if (!P.xsph_on) {
-            reinterpret_cast<F3*>(xo)[g] = self;
-            reinterpret_cast<F3*>(vo)[g] = selfv;
+            if (l == 0u) {
+                reinterpret_cast<F3*>(xo)[g] = self;
+                reinterpret_cast<F3*>(vo)[g] = selfv;
+            }
             return;
         }
-        const F3 a = pass_sum(b, SC[sc].G, PassTerms<PASS_XSPH>(b, P, g), q, n);
+        const F3 a = pass_sum<L>(b, SC[sc].G, PassTerms<PASS_XSPH>(b, P, g), q, n, l);
+        if (l != 0u) return;
         F3 out;
         if (isnan(a.x) || isnan(a.y) || isnan(a.z)) {
             out = selfv;
@@ -2279,48 +2046,7 @@ __global__ __launch_bounds__(256) void k_selftest_inv_sqrt(uint32_t lo, uint32_t
 
 inline uint32_t ceil_div(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
 
-// Dynamic LDS of each unit kernel: the tile of 12-byte positions, plus
-// kTilePad entries so that the filters read candidates four at a time past a
-// cell's last one without clamping (those reads are masked out).
-constexpr uint32_t kTilePad = 4;
-static_assert(sizeof(F3) == 12, "the tile holds packed float3 positions");
-size_t smem_of(uint32_t tile_cap) { return (size_t)(tile_cap + kTilePad) * sizeof(F3); }
-
-// The final-list units' tile: kFinalTileMax entries whatever the search's
-// tile.  A 32-cell-wide final unit in the dam's lattice (8 particles a cell)
-// has a 9 x 34-cell neighbourhood of 2,448 particles; 2,560 entries stage all
-// of them at four workgroups per CU (1,536 left them to the global-memory
-// filter: 237 against 216 us on the 1M step, 1.95 against 1.63 ms at 8M;
-// 3,072 costs a workgroup per CU and is slower again).
-uint32_t final_tile(const Tuning&) { return kFinalTileMax; }
-
 }  // namespace
-
-void size_unit_grids(Tuning& T, int num_cu) {
-    struct K {
-        int id;
-        const void* f;
-    } ks[] = {{K_NS, (const void*)k_ns<true>}, {K_FINAL_LIST, (const void*)k_final_list<true>}};
-    const uint32_t ncu = num_cu > 0 ? (uint32_t)num_cu : 1u;
-    uint32_t lo = 0xFFFFFFFFu;
-    for (int i = 0; i < K_NUM; ++i) T.grid[i] = 0;
-    const void* single[] = {(const void*)k_ns<false>, (const void*)k_final_list<false>};
-    for (const void* f : single)
-        (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem_of(kTileCapMax));
-    for (auto& k : ks) {
-        // allow the largest tile, then ask how many workgroups of the
-        // current one fit a CU
-        (void)hipFuncSetAttribute(k.f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem_of(kTileCapMax));
-        int nb = 0;
-        const uint32_t tc = k.id == K_FINAL_LIST ? final_tile(T) : T.tile_cap;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k.f, kBlock, smem_of(tc)) != hipSuccess ||
-            nb < 1)
-            nb = 1;
-        T.grid[k.id] = ncu * (uint32_t)nb < 8u ? 8u : ncu * (uint32_t)nb;
-        lo = T.grid[k.id] < lo ? T.grid[k.id] : lo;
-    }
-    T.grid_units = lo;
-}
 
 const char* kernel_name(int id) {
     static const char* names[K_NUM] = {"k_predict_hash", "k_scan_tiles", "k_scan_cells", "k_scatter",
@@ -2349,6 +2075,31 @@ struct Mark {
 }  // namespace
 
 namespace {
+// Lanes per particle of the passes that walk a list per particle: as many as
+// leave the chip (65,536 lanes at one wave a SIMD) about full.  Measured, k_deltap
+// with 16 / 4 / 1 lanes: 8.2 / 10.4 / 12.1 us for 960 particles, 8.3 / 10.3 / 12.6
+// for 8,000, 12.2 / 10.4 / 12.7 for 32,768, 18.4 / 12.5 / 13.3 for 65,600 and
+// 28.8 / 17.7 / 14.2 for 130,000; k_lambda and the final passes cross at the same
+// sizes.
+constexpr uint32_t kRowMax = 16384, kQuadMax = 81920;
+template <class F>
+void by_lanes(uint32_t n, F&& f) {
+    if (n <= kRowMax) f(std::integral_constant<int, 16>{});
+    else if (n <= kQuadMax) f(std::integral_constant<int, 4>{});
+    else f(std::integral_constant<int, 1>{});
+}
+// Whether a record's byte offset passes 32 bits.
+template <class F>
+void by_width(uint32_t cap, F&& f) {
+    if (cap < kGatherMaxSlots) f(std::false_type{});
+    else f(std::true_type{});
+}
+// workgroups that walk the work items for statistics, one item a thread or more
+uint32_t stat_blocks(uint32_t n) { return std::min(64u, 1u + ceil_div(n, 4096u)); }
+// workgroups of the big-cell list builds (a loop over 32 particles each)
+dim3 big_grid(uint32_t n) { return dim3(std::min(4096u, ceil_div(n, kGroups))); }
+dim3 lane_grid(uint32_t n, int lanes) { return dim3(ceil_div(n > 0 ? n : 1u, 256u / (uint32_t)lanes)); }
+
 template <bool kB>
 hipError_t step_seq(const Bufs& b, const Scenes<kB>& SC, const Tuning& T, float* x, float* v, uint32_t n, int iters,
                     int any_xsph, int any_vort, uint32_t uw, hipStream_t s, Timer* tm, float4* qtape) {
@@ -2357,8 +2108,6 @@ hipError_t step_seq(const Bufs& b, const Scenes<kB>& SC, const Tuning& T, float*
     const uint32_t budget = (T.tile_cap * 3u) / 4u > 0 ? (T.tile_cap * 3u) / 4u : 1u;
     uint32_t lguw = 0;
     while ((1u << lguw) < uw) ++lguw;
-    auto grid = [&](int k) { return dim3(T.grid[k] ? T.grid[k] : T.grid_units); };
-    const size_t smem = smem_of(T.tile_cap);
     if (n > 0) {
         Mark m(tm, s, K_PREDICT_HASH);
         hipLaunchKernelGGL(k_predict_hash<kB>, dim3(nb), dim3(256), 0, s, x, v, n, b, SC, b.key, b.rank, b.count, b.tflag,
@@ -2397,8 +2146,12 @@ hipError_t step_seq(const Bufs& b, const Scenes<kB>& SC, const Tuning& T, float*
     }
     {
         Mark m(tm, s, K_NS);
-        hipLaunchKernelGGL(k_ns<kB>, grid(K_NS), dim3(kBlock), smem, s, b, SC, T.tile_cap);
-        hipLaunchKernelGGL(k_ns_heavy<kB>, dim3(kHeavyBlocks), dim3(1024), 0, s, b, SC);
+        by_width(b.cap, [&](auto wide) {
+            const uint32_t ng = ceil_div(n, kGroups);
+            hipLaunchKernelGGL((k_ns_groups<kB, wide()>), dim3(ng + stat_blocks(n)), dim3(kBlock), 0, s, b, SC,
+                               T.tile_cap, ng);
+            hipLaunchKernelGGL((k_ns_big<kB, wide()>), big_grid(n), dim3(kBlock), 0, s, b, SC);
+        });
     }
     const bool pow4 = !kB && SC.s0.P.sn == 4;  // a batch's scenes may differ: general powi
     for (int it = 0; it < iters; ++it) {
@@ -2406,13 +2159,17 @@ hipError_t step_seq(const Bufs& b, const Scenes<kB>& SC, const Tuning& T, float*
         if (qtape) bi.Q = qtape + (size_t)it * b.cap;
         {
             Mark m(tm, s, K_LAMBDA);
-            hipLaunchKernelGGL(k_lambda<kB>, dim3(nb), dim3(256), 0, s, bi, SC);
+            by_lanes(n, [&](auto L) {
+                hipLaunchKernelGGL((k_lambda<kB, L()>), lane_grid(n, L()), dim3(256), 0, s, bi, SC);
+            });
         }
         Mark m(tm, s, K_DELTAP);
-        if (pow4)
-            hipLaunchKernelGGL((k_deltap<kB, true>), dim3(nb), dim3(256), 0, s, bi, SC);
-        else
-            hipLaunchKernelGGL((k_deltap<kB, false>), dim3(nb), dim3(256), 0, s, bi, SC);
+        by_lanes(n, [&](auto L) {
+            if (pow4)
+                hipLaunchKernelGGL((k_deltap<kB, true, L()>), lane_grid(n, L()), dim3(256), 0, s, bi, SC);
+            else
+                hipLaunchKernelGGL((k_deltap<kB, false, L()>), lane_grid(n, L()), dim3(256), 0, s, bi, SC);
+        });
     }
     if (!any_vort && !any_xsph) {
         Mark m(tm, s, K_OUT);
@@ -2440,9 +2197,12 @@ hipError_t step_seq(const Bufs& b, const Scenes<kB>& SC, const Tuning& T, float*
     }
     {
         Mark m(tm, s, K_FINAL_LIST);
-        const uint32_t ft = final_tile(T);
-        hipLaunchKernelGGL(k_final_list<kB>, grid(K_FINAL_LIST), dim3(kBlock), smem_of(ft), s, b, SC, ft, lguw, lgnc);
-        hipLaunchKernelGGL(k_final_heavy<kB>, dim3(kHeavyBlocks), dim3(1024), 0, s, b, SC);
+        by_width(b.cap, [&](auto wide) {
+            const uint32_t ng = ceil_div(n, kGroups);
+            hipLaunchKernelGGL((k_final_groups<kB, wide()>), dim3(ng + stat_blocks(n)), dim3(kBlock), 0, s, b, SC,
+                               kFinalTile, lguw, lgnc, ng);
+            hipLaunchKernelGGL((k_final_big<kB, wide()>), big_grid(n), dim3(kBlock), 0, s, b, SC);
+        });
     }
     // the overflow positions' per-cell partials, before each pass that adds them
     const dim3 ovf_grid(kOvfBlocks);
@@ -2450,16 +2210,22 @@ hipError_t step_seq(const Bufs& b, const Scenes<kB>& SC, const Tuning& T, float*
         {
             Mark m(tm, s, K_VORT);
             hipLaunchKernelGGL((k_ovf_part<kB, PASS_VORT>), ovf_grid, dim3(256), 0, s, b, SC);
-            hipLaunchKernelGGL(k_vort<kB>, dim3(nb), dim3(kBlock), 0, s, b, SC);
+            by_lanes(n, [&](auto L) {
+                hipLaunchKernelGGL((k_vort<kB, L()>), lane_grid(n, L()), dim3(kBlock), 0, s, b, SC);
+            });
         }
         Mark m(tm, s, K_CONFINE);
         hipLaunchKernelGGL((k_ovf_part<kB, PASS_CONF>), ovf_grid, dim3(256), 0, s, b, SC);
-        hipLaunchKernelGGL(k_confine<kB>, dim3(nb), dim3(kBlock), 0, s, b, SC);
+        by_lanes(n, [&](auto L) {
+            hipLaunchKernelGGL((k_confine<kB, L()>), lane_grid(n, L()), dim3(kBlock), 0, s, b, SC);
+        });
     }
     if (any_xsph) {
         Mark m(tm, s, K_XSPH_OUT);
         hipLaunchKernelGGL((k_ovf_part<kB, PASS_XSPH>), ovf_grid, dim3(256), 0, s, b, SC);
-        hipLaunchKernelGGL(k_xsph_out<kB>, dim3(nb), dim3(kBlock), 0, s, b, SC, x, v);
+        by_lanes(n, [&](auto L) {
+            hipLaunchKernelGGL((k_xsph_out<kB, L()>), lane_grid(n, L()), dim3(kBlock), 0, s, b, SC, x, v);
+        });
     } else {
         Mark m(tm, s, K_OUT);
         hipLaunchKernelGGL(k_out<kB>, dim3(nb), dim3(256), 0, s, b, SC, (const float4*)b.R, x, v);
