@@ -792,6 +792,14 @@ __device__ __forceinline__ uint32_t cell27(const int gp[3], uint32_t c, const Gr
     return scene_key(gp[0] + (q % 3) - 1, gp[1] + (q / 3) - 1, gp[2] + dz, G);
 }
 
+// The same around the cell of key `key`.
+__device__ __forceinline__ uint32_t key27(uint32_t key, uint32_t c, const Grid& G) {
+    const uint32_t k = key - G.base, dz = c / 9u, q = c % 9u;
+    const uint32_t x = (k + q % 3u - 1u) & (G.gx - 1u), y = ((k >> G.lgx) + q / 3u - 1u) & (G.gy - 1u),
+                   z = ((k >> (G.lgx + G.lgy)) + dz - 1u) & (G.gz - 1u);
+    return G.base + (((z << G.lgy) + y) << G.lgx) + x;
+}
+
 constexpr uint32_t kGroup = 8;
 constexpr uint32_t kGroups = kBlock / kGroup;  // groups of a workgroup
 constexpr uint32_t kMaxPair = 64;              // the largest max_pair accepted
@@ -1121,21 +1129,28 @@ __device__ uint32_t ns_heavy_list(const Grid& G, CellView b, const float4* __res
                 via = true;
             }
         }
-        for (uint32_t p = p0; p < p1; p += 64u) {
-            const uint32_t t = p + lane;
-            uint32_t j = 0;
-            bool hit = false;
-            if (t < p1) {
-                j = via ? b.aux[o0 + t] : o0 + t;
-                hit = pair_test<false>(self - f3of(Pf[j]), h2);
+        for (uint32_t p = p0; p < p1; p += 256u) {
+            uint32_t j[4];
+            F3 pj[4];
+#pragma unroll
+            for (uint32_t u = 0; u < 4u; ++u) {
+                const uint32_t t = min(p + u * 64u + lane, p1 - 1u);
+                j[u] = via ? b.aux[o0 + t] : o0 + t;
             }
-            const uint64_t m = __ballot(hit);
-            const uint32_t k = n + (uint32_t)__popcll(m & below);
-            if (hit && k < ncap) nl[list_at(cap, g, k)] = j;
-            n += (uint32_t)__popcll(m);
-            if (n > ncap) {
-                trunc = true;
-                return ncap;
+#pragma unroll
+            for (uint32_t u = 0; u < 4u; ++u) pj[u] = f3of(Pf[j[u]]);
+#pragma unroll
+            for (uint32_t u = 0; u < 4u; ++u) {
+                const bool hit = p + u * 64u + lane < p1 && pair_test<false>(self - pj[u], h2);
+                const uint64_t m = __ballot(hit);
+                if (m == 0ull) continue;
+                const uint32_t k = n + (uint32_t)__popcll(m & below);
+                if (hit && k < ncap) nl[list_at(cap, g, k)] = j[u];
+                n += (uint32_t)__popcll(m);
+                if (n > ncap) {
+                    trunc = true;
+                    return ncap;
+                }
             }
         }
     }
@@ -1535,20 +1550,28 @@ __device__ uint32_t heavy_list(const Grid& G, CellView b, const float4* __restri
             }
         }
         bool any = false;  // a pair of this cell was appended
-        for (uint32_t p = p0; p < p1; p += 64u) {
-            const uint32_t t = p + lane;
-            uint32_t j = 0;
-            bool hit = false;
-            if (t < p1) {
-                j = via ? b.aux[o0 + t] : o0 + t;
-                hit = pair_test<true>(f3of(Pf[j]) - self, cut2);
+        for (uint32_t p = p0; p < p1; p += 256u) {
+            uint32_t j[4];
+            F3 pj[4];
+#pragma unroll
+            for (uint32_t u = 0; u < 4u; ++u) {
+                const uint32_t t = min(p + u * 64u + lane, p1 - 1u);
+                j[u] = via ? b.aux[o0 + t] : o0 + t;
             }
-            const uint64_t m = __ballot(hit);
-            const uint32_t k = n + (uint32_t)__popcll(m & below);
-            if (hit && k < kFinalK) fl[list_at(cap, q, k)] = j | ((!any && (m & below) == 0ull) ? 0x80000000u : 0u);
-            n += (uint32_t)__popcll(m);
-            any = any || m != 0ull;
-            if (n >= lim) return lim;
+#pragma unroll
+            for (uint32_t u = 0; u < 4u; ++u) pj[u] = f3of(Pf[j[u]]);
+#pragma unroll
+            for (uint32_t u = 0; u < 4u; ++u) {
+                const bool hit = p + u * 64u + lane < p1 && pair_test<true>(pj[u] - self, cut2);
+                const uint64_t m = __ballot(hit);
+                if (m == 0ull) continue;
+                const uint32_t k = n + (uint32_t)__popcll(m & below);
+                if (hit && k < kFinalK)
+                    fl[list_at(cap, q, k)] = j[u] | ((!any && (m & below) == 0ull) ? 0x80000000u : 0u);
+                n += (uint32_t)__popcll(m);
+                any = true;
+                if (n >= lim) return lim;
+            }
         }
     }
     return n;
@@ -1744,10 +1767,13 @@ struct PassTerms {
     const float4* __restrict__ R;
     const float4* __restrict__ OM4;
     F3 self, selfv;
+    uint32_t key;  // of the final cell
     float arg, cut2;
     __device__ __forceinline__ PassTerms(const Bufs& b, const Phys& P, uint32_t g)
-        : R(b.R), OM4(b.OM4), self(f3of(b.R[2 * g])),
-          selfv(kPass == PASS_CONF ? mk3(0.f, 0.f, 0.f) : f3of(b.R[2 * g + 1])),
+        : PassTerms(b, P, g, b.R[2 * g]) {}
+    __device__ __forceinline__ PassTerms(const Bufs& b, const Phys& P, uint32_t g, float4 r0)
+        : R(b.R), OM4(b.OM4), self(f3of(r0)),
+          selfv(kPass == PASS_CONF ? mk3(0.f, 0.f, 0.f) : f3of(b.R[2 * g + 1])), key(__float_as_uint(r0.w)),
           arg(kPass == PASS_XSPH ? P.inv_h : P.warg), cut2(kPass == PASS_XSPH ? P.cut2_w : P.cut2_wd) {}
     __device__ __forceinline__ El2 elem(uint32_t j) const {
         if (kPass == PASS_CONF) {
@@ -1771,16 +1797,49 @@ struct PassTerms {
     }
 };
 
-// Partial sum of cell c (0..26) of the 27 around the pass particle's final cell.
-template <class Pass>
-__device__ __forceinline__ F3 pass_cell(const Bufs& b, const Grid& G, const Pass& ps, uint32_t c) {
-    int gp[3];
-    grid_pos(ps.self, G.cw, gp);
-    auto elem = [&](uint32_t j) { return ps.elem(j); };
-    auto term = [&](const El2& e) { return ps.term(e); };
-    const uint32_t key = cell27(gp, c, G);
-    return big_cells(b) ? sum_cell<true>(cell_view(b), key, ps.self, ps.cut2, elem, term)
-                        : sum_cell<false>(cell_view(b), key, ps.self, ps.cut2, elem, term);
+// Partial sum of cell c (0..26) of the 27 around the pass particle's final
+// cell, by a row of 16 lanes: 16 candidates at a time, a lane each, and the
+// terms of those in range added in slot order by every lane (the others add
+// +0), as sum_cell adds them; the next candidates are loaded while one step is
+// added.  Called by all lanes of the row.
+template <bool kBig, class Pass>
+__device__ __forceinline__ F3 sum_cell_row(CellView b, const Grid& G, const Pass& ps, uint32_t c, uint32_t l) {
+    const uint32_t key = key27(ps.key, c, G);
+    const uint32_t st = b.offset[key], n = b.offset[key + 1] - st;
+    float cs[3] = {0.f, 0.f, 0.f};
+    uint32_t p0 = 0, p1 = n;
+    bool via = false;
+    if (kBig && n > kSmallCell) {
+        const BigPart bp = big_part<true>(b.bseg + b.bslot[st], ps.self, ps.cut2, n);
+        if (bp.how == 0u) p1 = 0u;
+        if (aux_pays(bp, n)) {
+            p0 = bp.p0;
+            p1 = bp.p1;
+            via = true;
+        }
+    }
+    if (p0 < p1) {
+        auto slot = [&](uint32_t t) {
+            const uint32_t u = min(t, p1 - 1u);
+            return kBig && via ? b.aux[st + u] : st + u;
+        };
+        El2 el = ps.elem(slot(p0 + l));
+        uint32_t jn = slot(p0 + 16u + l);
+        for (uint32_t p = p0; p < p1; p += 16u) {
+            const El2 nx = ps.elem(jn);
+            jn = slot(p + 32u + l);
+            const F3 d = f3of(el.p) - ps.self;
+            const bool in = p + l < p1 && !(glm_dot(d, d) > ps.cut2);
+            if (__builtin_amdgcn_ballot_w64(in)) {
+                F3 t = mk3(0.f, 0.f, 0.f);
+                if (in) t = ps.term(el);
+                const float v[3] = {t.x, t.y, t.z};
+                add_lanes<16>(cs, v);
+            }
+            el = nx;
+        }
+    }
+    return mk3(cs[0], cs[1], cs[2]);
 }
 
 // The pass's sum for final-order position q with stored count n: the list
@@ -1813,27 +1872,38 @@ __device__ __forceinline__ F3 pass_sum(const Bufs& b, const Grid& G, const Pass&
 
 
 // Per-cell partials of pass kPass for the overflow slots.  A wave task is
-// (slot k, cell c): lane l sums cell c of the 27 around final-order position
-// 64 * ovf[k] + l, when that position overflowed, in slot order (sum_cell, as
-// the direct sum does) into part[(k * 27 + c) * 64 + l].  The lanes are
-// neighbours in final-cell order, so they mostly scan the same cell and load
-// the same records, and the pass reads each row of 64 whole.
+// (slot k, cell c, four consecutive positions of the slot's block): row r sums
+// cell c of the 27 around final-order position 64 * ovf[k] + 4 * sub + r, when
+// that position overflowed, in slot order (sum_cell_row) into
+// part[(k * 27 + c) * 64 + 4 * sub + r].  Consecutive tasks share a cell index,
+// so a workgroup's rows mostly scan the same cell, and the pass reads each row
+// of 64 whole.
+//
+// A cell of a pile is one serial sum of thousands of terms, whose length set the
+// launch's time while the chip idled (a tenth of the VALU issue) when a thread
+// did it: 139 us a launch (vorticity) over the 40 chained steps of the 32k dam and
+// 1.49 ms over the first ten of the 1M dam; by rows 48 us and 0.40 ms.
 template <bool kB, int kPass>
 __global__ __launch_bounds__(256) void k_ovf_part(Bufs b, Scenes<kB> SC) {
     const uint32_t ns = min(b.ctr[CTR_OVF], b.ovf_max);
-    const uint32_t ntask = ns * 27u;
-    const uint32_t nl = b.offset[b.CT];
-    const uint32_t lane = lane_id();
-    const uint32_t w0 = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, nw = (gridDim.x * blockDim.x) >> 6;
-    for (uint32_t t = w0; t < ntask; t += nw) {
-        const uint32_t k = t / 27u, c = t - k * 27u;
-        const uint32_t q = b.ovf[k] * 64u + lane;
+    if (ns == 0u) return;  // uniform over the grid
+    const uint32_t nl = b.offset[b.CT], lane = lane_id(), l = lane & 15u;
+    const bool any_big = big_cells(b);
+    const uint64_t ntask = (uint64_t)ns * (27u * 16u);
+    const uint32_t w0 = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    const uint32_t nw = (gridDim.x * blockDim.x) >> 6;
+    for (uint64_t t = w0; t < ntask; t += nw) {
+        const uint32_t kc = (uint32_t)(t >> 4), k = kc / 27u, c = kc - k * 27u;
+        const uint32_t at = ((uint32_t)t & 15u) * 4u + (lane >> 4);  // position in the block
+        const uint32_t q = b.ovf[k] * 64u + at;
         const bool active = q < nl && b.fcnt[q] == kFinalK + 1u;
+        if (!__any(active)) continue;
         const uint32_t g = active ? b.cperm[q] : 0u;
         by_scene<kB>((kB && active) ? b.sid[g] : 0u, active, [&](uint32_t sc) {
             const PassTerms<kPass> ps(b, SC[sc].P, g);
-            const F3 cs = pass_cell(b, SC[sc].G, ps, c);
-            b.part[((size_t)k * 27u + c) * 64u + lane] = make_float4(cs.x, cs.y, cs.z, 0.f);
+            const F3 cs = any_big ? sum_cell_row<true>(cell_view(b), SC[sc].G, ps, c, l)
+                                  : sum_cell_row<false>(cell_view(b), SC[sc].G, ps, c, l);
+            if (l == 0u) b.part[((size_t)k * 27u + c) * 64u + at] = make_float4(cs.x, cs.y, cs.z, 0.f);
         });
     }
 }

@@ -71,3 +71,17 @@ def test_lane_rules(n):
     sc = scenes.small_dam(48, 48, 36, h=0.1, box=(3.2, 3.2, 1.6), iters=2, seed=5, scorr_k=0.001, v_sigma=0.1)
     keep = np.sort(np.random.default_rng(n).permutation(sc.n)[:n])
     check(dataclasses.replace(sc, x=sc.x[keep].copy(), v=sc.v[keep].copy()))
+
+
+@pytest.mark.parametrize("per_cell", [17, 33, 64, 65])
+def test_overflowing_final_lists(per_cell):
+    """More than 64 pairs a particle: the sums go cell by cell, 16 candidates a
+    step, with and without cells of more than 64 particles."""
+    h = 0.1
+    base = scenes.small_dam(4, 4, 4, h=h, box=(0.5, 0.4, 0.4), iters=1, seed=3, scorr_k=0.001)
+    rng = np.random.default_rng(per_cell)
+    x = np.concatenate([(np.array([i % 5, i // 5 % 4, i // 20]) + rng.uniform(0.05, 0.95, (per_cell, 3))) * h
+                        for i in range(80)]).astype(np.float32)
+    got = check(dataclasses.replace(base, x=x, v=rng.normal(0.0, 0.05, x.shape).astype(np.float32)))
+    print(per_cell, got["stats"]["list_overflow"], flush=True)
+    assert got["stats"]["list_overflow"] > 0
