@@ -90,11 +90,18 @@ constexpr uint32_t kOvfBlocks = 2048;
 constexpr uint32_t kNoSlot = 0xFFFFFFFFu;       // oslot: no particle of the block overflowed (yet)
 constexpr uint32_t kPendingSlot = 0xFFFFFFFEu;  // oslot: being allocated (never seen across kernels)
 constexpr uint32_t kFullSlot = 0xFFFFFFFDu;     // oslot: no slot was left
-// A list build whose next cell would take it past kHeavyScan candidates (a
-// particle beside a pile) is done by a whole wave instead of a group of eight
-// lanes.
-constexpr uint32_t kHeavyScan = 2048;
-static_assert(kHeavyScan >= 27u * kSmallCell, "a build without big cells never reaches the budget");
+// A list build whose next cell would take it past kHeavySearch (final lists:
+// kHeavyFinal) candidates -- a particle beside a pile -- is done by a whole wave
+// instead of a group of eight lanes: the bound on one list's serial scan (256
+// candidates a step instead of 32).  In bulk the groups are the faster, since
+// the particles beside a pile share its candidates: with 2,048 for both k_final_big
+// took 143 us a launch over the 40 chained steps of the 32k dam and 1.71 ms over
+// the first ten of the 1M dam, with these 84 us and 0.98 ms; 4,096 to 32,768
+// measured like 3,072.
+constexpr uint32_t kHeavySearch = 2048;
+constexpr uint32_t kHeavyFinal = 3072;
+static_assert(kHeavySearch >= 27u * kSmallCell && kHeavyFinal >= 27u * kSmallCell,
+              "a build without big cells never reaches the budget");
 
 enum Ctr : int {
     CTR_UNITS = 0,

@@ -830,7 +830,7 @@ struct GroupShared {
 // lim), and a single group left is scanned through aux when that skips a
 // quarter of the cell or more.  Returns kDeferred, leaving the list unfinished,
 // before a range that would take the candidates tested past `budget` (only a
-// neighbourhood holding a big cell can: 27 * kSmallCell < kHeavyScan).
+// neighbourhood holding a big cell can: 27 * kSmallCell is less).
 // kWide: more than 2^28 slots, whose records' byte offsets pass 32 bits.
 // Called by all eight lanes; every value but the candidates is the same on them.
 //
@@ -995,8 +995,9 @@ __device__ __forceinline__ uint32_t group_list(GroupShared& S, const Grid& G, Ce
 #pragma unroll
                     for (uint32_t u = 0; u < 4u; ++u) {
                         const bool in = t0 + l + u * kGroup < p1, ok = test(pj[u]);
-                        const uint32_t bits = byte_of(in, ok);
-                        append(bits, in && ok, j[u], n == n0);
+                        // few candidates beside a pile are pairs: no ranking where none of the wave's is
+                        if ((__builtin_amdgcn_ballot_w64(in) & __builtin_amdgcn_ballot_w64(ok)) == 0ull) continue;
+                        append(byte_of(in, ok), in && ok, j[u], n == n0);
                     }
                 }
                 if (n > lim) break;
@@ -1022,7 +1023,7 @@ __device__ __forceinline__ bool group_search(GroupShared& S, const Bufs& b, cons
     const uint32_t ncap = (uint32_t)sc.P.cap;
     const float4 pk = b.Pf[g];
     const uint32_t n = group_list<false, kBig, kWide>(S, G, cell_view(b), b.Pf, f3of(pk), __float_as_uint(pk.w),
-                                                      sc.P.h2, ncap, b.nlist, b.cap, g, g, kHeavyScan);
+                                                      sc.P.h2, ncap, b.nlist, b.cap, g, g, kHeavySearch);
     if (kBig && n == kDeferred) return true;
     if ((lane_id() & (kGroup - 1u)) == 0u) {
         b.ncnt[g] = min(n, ncap);
@@ -1159,7 +1160,7 @@ __device__ uint32_t ns_heavy_list(const Grid& G, CellView b, const float4* __res
 
 // The search lists of a step with big cells (a step without them has its lists
 // from k_ns_groups): 32 slots a workgroup at a time by groups of eight lanes;
-// a list of more than kHeavyScan candidates is then built by its group's whole
+// a list of more than kHeavySearch candidates is then built by its group's whole
 // wave.
 template <bool kB, bool kWide>
 __global__ __launch_bounds__(kBlock) void k_ns_big(Bufs b, Scenes<kB> SC) {
@@ -1475,7 +1476,7 @@ __device__ __forceinline__ bool group_final(GroupShared& S, const Bufs& b, const
     const Grid G = sc.G;
     const float4 pk = b.R[2 * g];
     const uint32_t n = group_list<true, kBig, kWide>(S, G, cell_view(b), b.Pf, f3of(pk), __float_as_uint(pk.w),
-                                                     final_cut2(sc.P), kFinalK, b.flist, b.cap, q, g, kHeavyScan);
+                                                     final_cut2(sc.P), kFinalK, b.flist, b.cap, q, g, kHeavyFinal);
     if (kBig && n == kDeferred) return true;
     if ((lane_id() & (kGroup - 1u)) == 0u) {
         b.fcnt[q] = n > kFinalK ? ovf_mark(b, q) : n;
