@@ -33,6 +33,8 @@
 // with beta = m / rho0, gamma = c beta, kappa = epsilon dt / inv_rho0.
 #include "pbfx_device.hpp"
 
+#include <type_traits>
+
 namespace pbfx {
 namespace {
 
@@ -216,41 +218,47 @@ __device__ __forceinline__ void for_cells(const Grid& G, F3 p, F&& f) {
             for (int dx = -1; dx <= 1; ++dx) f(grid_hash(g[0] + dx, g[1] + dy, g[2] + dz, G), dx, dy, dz);
 }
 
-// How a thread takes part in a pass over a particle's candidate set: the
-// light kernel runs one thread per particle not flagged heavy (bit), the
-// heavy kernel one wave per listed particle, its lanes taking every 64th
-// candidate and reducing their sums in a fixed order.
+// How a lane takes part in a pass over a particle's candidate set: the first
+// workgroups give each particle not flagged heavy (bit) a group of L lanes, the
+// rest of the grid (kAdjHeavyBlocks) a wave to each listed one; the lanes of a
+// group take every L-th candidate and reduce their sums in a fixed order.
+// f(role, L) for this group's particles.
+//
+// A wave leaves most of its lanes idle over cells of a few tens of particles, so
+// it only takes particles with more than kAdjHeavy candidates: with 256 there, a
+// thread each below and the heavy ones in launches of their own, whose sizes the
+// host read back, ten steps at 65,536 particles took 66 ms forward and backward
+// (now 29) and three at 320,000 39 ms (now 18).
 struct Role {
     uint32_t i, lane, stride;
-    bool on;
 };
-template <bool kHeavy>
-__device__ __forceinline__ Role role(const StepTape& t, const AdjBufs& a, uint32_t bit) {
-    Role r;
-    if (!kHeavy) {
-        r.i = gtid();
-        r.lane = 0;
-        r.stride = 1;
-        r.on = r.i < t.n_live && !(a.hflag[r.i] & bit);
-    } else {
-        const uint32_t w = gtid() >> 6;
-        const uint32_t set = (uint32_t)__builtin_ctz(bit);
-        r.lane = threadIdx.x & 63u;
-        r.stride = 64;
-        r.on = w < a.nh[set];
-        r.i = r.on ? a.hlist[(size_t)set * a.cap + w] : 0u;
+constexpr uint32_t kAdjHeavyBlocks = 1024;
+template <int L, class F>
+__device__ __forceinline__ void for_roles(const StepTape& t, const AdjBufs& a, uint32_t bit, F&& f) {
+    const uint32_t nlight = (t.n_live * (uint32_t)L + 255u) / 256u;
+    if (blockIdx.x < nlight) {
+        const uint32_t i = gtid() / L;
+        if (i < t.n_live && !(a.hflag[i] & bit)) f(Role{i, threadIdx.x % L, L}, std::integral_constant<int, L>{});
+        return;
     }
-    return r;
+    const uint32_t set = (uint32_t)__builtin_ctz(bit), n = a.nh[set];
+    const uint32_t nw = (gridDim.x - nlight) * 4u;
+    for (uint32_t w = ((blockIdx.x - nlight) * 256u + threadIdx.x) >> 6; w < n; w += nw)
+        f(Role{a.hlist[(size_t)set * a.cap + w], threadIdx.x & 63u, 64u}, std::integral_constant<int, 64>{});
 }
 __device__ __forceinline__ void mark_heavy(const AdjBufs& a, uint32_t i, uint32_t set) {
     a.hlist[(size_t)set * a.cap + atomicAdd(&a.nh[set], 1u)] = i;
 }
-// sum over the wave (the heavy kernels; every lane holds the total)
-__device__ __forceinline__ double wsum(double v) {
-    for (int d = 32; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
+// sum over the group of L lanes (every lane holds the total)
+template <int L>
+__device__ __forceinline__ double gsum(double v) {
+    for (int d = L / 2; d > 0; d >>= 1) v += __shfl_xor(v, d, 64);
     return v;
 }
-__device__ __forceinline__ D3 wsum3(D3 v) { return md3(wsum(v.x), wsum(v.y), wsum(v.z)); }
+template <int L>
+__device__ __forceinline__ D3 gsum3(D3 v) {
+    return md3(gsum<L>(v.x), gsum<L>(v.y), gsum<L>(v.z));
+}
 
 // S(i): the slots of the 27 cells around the final cell of p (the forward
 // sum's candidates, pbf_contribution.inl:7-57); this thread's share.
@@ -332,7 +340,8 @@ __global__ __launch_bounds__(256) void k_adj_ckey(StepTape t, AdjBufs a, Grid G,
         grid_pos(f3of(t.PI[s]), G.cw, g);
         k = grid_hash(g[0], g[1], g[2], G);
     }
-    const uint32_t r = wave_rank(a.ccount, k, active, k);
+    // final cells need not follow slot order: equal keys are merged over the whole wave
+    const uint32_t r = wave_rank_any(a.ccount, k, active, k);
     if (active) {
         mark_tile(a.ctflag, k >> lgT);
         a.ckey[s] = k;
@@ -397,60 +406,54 @@ __global__ __launch_bounds__(256) void k_adj_last(StepTape t, AdjBufs a, Grid G,
 // (pbf_neighbor_search_util.cu:386-408,428-452: l lists the candidates with
 // r^2 < h^2 in its own scan order until the list is full).  fill = false:
 // count into rcount (and flag reverse lists above kAdjHeavy); fill = true:
-// write rlist.  A heavy wave takes the candidates 64 at a time and keeps the
+// write rlist.  A group takes its lanes' candidates at a time and keeps the
 // scan order with a ballot.
-template <bool fill, bool kHeavy>
+template <bool fill, int L>
 __global__ __launch_bounds__(256) void k_adj_rev(StepTape t, AdjBufs a, Grid G, Phys P) {
-    const Role r = role<kHeavy>(t, a, 4u);
-    if (!r.on) return;
-    const uint32_t j = r.i;
-    const F3 self = f3of(t.Q[j]);
-    const uint32_t full = (uint32_t)P.cap;
-    uint32_t cnt = 0;
-    uint32_t* out = fill ? a.rlist + a.roff[j] : nullptr;
-    for_cells(G, self, [&](uint32_t c, int dx, int dy, int dz) {
-        const uint32_t b0 = t.offset[c], e = t.offset[c + 1];
-        const uint32_t pos = (uint32_t)((1 - dz) * 9 + (1 - dy) * 3 + (1 - dx));  // j seen from l
-        for (uint32_t base = b0; base < e; base += r.stride) {
-            const uint32_t l = base + r.lane;
-            bool listed = false;
-            if (l < e && l != j) {
-                const F3 d = f3of(t.Q[l]) - self;  // the search's d = p_l - p_j
-                const float r2 = __builtin_fmaf(d.z, d.z, __builtin_fmaf(d.y, d.y, d.x * d.x));
-                if (r2 < P.h2) {
-                    const uint32_t n = t.ncnt[l];
-                    listed = n > 0 && n < full;
-                    if (n == full) {
-                        const uint2 L = a.last[l];
-                        listed = pos < L.x || (pos == L.x && j <= L.y);
+    for_roles<L>(t, a, 4u, [&](const Role& r, auto width) {
+        constexpr int W = decltype(width)::value;
+        const uint32_t j = r.i;
+        const F3 self = f3of(t.Q[j]);
+        const uint32_t full = (uint32_t)P.cap;
+        uint32_t cnt = 0;
+        uint32_t* out = fill ? a.rlist + a.roff[j] : nullptr;
+        const uint32_t sh = (threadIdx.x & 63u) & ~(uint32_t)(W - 1);  // the group's first lane
+        for_cells(G, self, [&](uint32_t c, int dx, int dy, int dz) {
+            const uint32_t b0 = t.offset[c], e = t.offset[c + 1];
+            const uint32_t pos = (uint32_t)((1 - dz) * 9 + (1 - dy) * 3 + (1 - dx));  // j seen from l
+            for (uint32_t base = b0; base < e; base += r.stride) {
+                const uint32_t l = base + r.lane;
+                bool listed = false;
+                if (l < e && l != j) {
+                    const F3 d = f3of(t.Q[l]) - self;  // the search's d = p_l - p_j
+                    const float r2 = __builtin_fmaf(d.z, d.z, __builtin_fmaf(d.y, d.y, d.x * d.x));
+                    if (r2 < P.h2) {
+                        const uint32_t n = t.ncnt[l];
+                        listed = n > 0 && n < full;
+                        if (n == full) {
+                            const uint2 La = a.last[l];
+                            listed = pos < La.x || (pos == La.x && j <= La.y);
+                        }
                     }
                 }
-            }
-            if (!kHeavy) {
-                if (listed) {
-                    if (fill) out[cnt] = l;
-                    ++cnt;
-                }
-            } else {
-                const uint64_t m = __ballot(listed);
+                const uint64_t m = (__ballot(listed) >> sh) & (W == 64 ? ~0ull : (1ull << (W & 63)) - 1ull);
                 if (fill && listed) out[cnt + (uint32_t)__popcll(m & ((1ull << r.lane) - 1ull))] = l;
                 cnt += (uint32_t)__popcll(m);
             }
+        });
+        if (!fill && r.lane == 0) {
+            a.rcount[j] = cnt;
+            if (cnt) mark_tile(a.rtflag, j >> a.lgRT);
+            if (cnt > kAdjHeavy) {
+                atomicOr(&a.hflag[j], 8u);
+                mark_heavy(a, j, 3);
+            }
         }
     });
-    if (!fill && r.lane == 0) {
-        a.rcount[j] = cnt;
-        if (cnt) mark_tile(a.rtflag, j >> a.lgRT);
-        if (cnt > kAdjHeavy) {
-            atomicOr(&a.hflag[j], 8u);
-            mark_heavy(a, j, 3);
-        }
-    }
 }
 
 // ------------------------------------------------------------ final stage
-// Every pass below has a light (one thread per particle) and a heavy (one
-// wave per particle) instantiation over the same body.
+// Every pass below gives a particle a group of lanes or a wave (for_roles).
 
 // Clears dL/dVc = dL/dv_out, dL/dP = dL/dx_out (the stage's starting point).
 __global__ __launch_bounds__(256) void k_adj_final_init(StepTape t, AdjBufs a) {
@@ -462,228 +465,235 @@ __global__ __launch_bounds__(256) void k_adj_final_init(StepTape t, AdjBufs a) {
 
 // XSPH, own pairs: dL/dVc_i, the position terms of i's own sum, dL/dc
 // (v_out = Vc + gamma sum_j (Vc_j - Vc_i) W(|p_j - p_i|)).
-template <bool kHeavy>
+template <int L>
 __global__ __launch_bounds__(256) void k_adj_xsph_own(StepTape t, AdjBufs a, Grid G, Phys P) {
-    const Role r = role<kHeavy>(t, a, 1u);
-    if (!r.on) return;
-    const uint32_t i = r.i;
-    const AdjConst k = adj_const(P);
-    const F3 selff = f3of(t.PI[i]);
-    const D3 self = wid3(selff), vi = wid(t.R[2 * i + 1]);
-    const D3 gi = ld3d(a.av, i);
-    double sumW = 0.0;
-    D3 acc = dz3(), apos = dz3();
-    for_S(t, G, selff, r, [&](uint32_t j) {
-        if (j == i) return;
-        const D3 pd = wid(t.PI[j]) - self;
-        if (dot3(pd, pd) > (double)P.cut2_w) return;
-        double W, gw;
-        if (!poly6_adj(pd, k, W, gw)) return;
-        const D3 e = wid(t.R[2 * j + 1]) - vi;
-        acc = acc + sc3(e, W);
-        sumW += W;
-        apos = apos - sc3(pd, gw * k.gamma * dot3(gi, e));
+    for_roles<L>(t, a, 1u, [&](const Role& r, auto width) {
+        constexpr int W = decltype(width)::value;
+        const uint32_t i = r.i;
+        const AdjConst k = adj_const(P);
+        const F3 selff = f3of(t.PI[i]);
+        const D3 self = wid3(selff), vi = wid(t.R[2 * i + 1]);
+        const D3 gi = ld3d(a.av, i);
+        double sumW = 0.0;
+        D3 acc = dz3(), apos = dz3();
+        for_S(t, G, selff, r, [&](uint32_t j) {
+            if (j == i) return;
+            const D3 pd = wid(t.PI[j]) - self;
+            if (dot3(pd, pd) > (double)P.cut2_w) return;
+            double W, gw;
+            if (!poly6_adj(pd, k, W, gw)) return;
+            const D3 e = wid(t.R[2 * j + 1]) - vi;
+            acc = acc + sc3(e, W);
+            sumW += W;
+            apos = apos - sc3(pd, gw * k.gamma * dot3(gi, e));
+        });
+        if (W > 1) {
+            acc = gsum3<W>(acc);
+            sumW = gsum<W>(sumW);
+            apos = gsum3<W>(apos);
+            if (r.lane) return;
+        }
+        const bool nan = isnan(acc.x) || isnan(acc.y) || isnan(acc.z);
+        a.xnan[i] = nan ? 1u : 0u;
+        if (nan) return;  // velocity kept: v_out = Vc
+        st(a.aVc, i, sc3(gi, 1.0 - k.gamma * sumW));
+        st(a.aP, i, ld(a.aP, i) + apos);
+        a.pc[i] = k.beta * dot3(gi, acc);
     });
-    if (kHeavy) {
-        acc = wsum3(acc);
-        sumW = wsum(sumW);
-        apos = wsum3(apos);
-        if (r.lane) return;
-    }
-    const bool nan = isnan(acc.x) || isnan(acc.y) || isnan(acc.z);
-    a.xnan[i] = nan ? 1u : 0u;
-    if (nan) return;  // velocity kept: v_out = Vc
-    st(a.aVc, i, sc3(gi, 1.0 - k.gamma * sumW));
-    st(a.aP, i, ld(a.aP, i) + apos);
-    a.pc[i] = k.beta * dot3(gi, acc);
 }
 
 // XSPH, transposed pairs (l, i), i in S(l).
-template <bool kHeavy>
+template <int L>
 __global__ __launch_bounds__(256) void k_adj_xsph_rev(StepTape t, AdjBufs a, Grid G, Phys P) {
-    const Role r = role<kHeavy>(t, a, 2u);
-    if (!r.on) return;
-    const uint32_t i = r.i;
-    const AdjConst k = adj_const(P);
-    const D3 pi = wid(t.PI[i]), vi = wid(t.R[2 * i + 1]);
-    D3 avc = dz3(), apos = dz3();
-    for_T(a, G, f3of(t.Q[i]), r, [&](uint32_t q) {
-        const float4 pl = a.gP[q];
-        const float4 vl = a.gV[q];
-        if (__float_as_uint(pl.w) == i || vl.w != 0.f) return;
-        const D3 pd = pi - wid(pl);
-        if (dot3(pd, pd) > (double)P.cut2_w) return;
-        double W, gw;
-        if (!poly6_adj(pd, k, W, gw)) return;
-        const double4 g4 = a.gD[q];
-        const D3 gl = md3(g4.x, g4.y, g4.z);
-        avc = avc + sc3(gl, k.gamma * W);
-        apos = apos + sc3(pd, gw * k.gamma * dot3(gl, vi - wid(vl)));
+    for_roles<L>(t, a, 2u, [&](const Role& r, auto width) {
+        constexpr int W = decltype(width)::value;
+        const uint32_t i = r.i;
+        const AdjConst k = adj_const(P);
+        const D3 pi = wid(t.PI[i]), vi = wid(t.R[2 * i + 1]);
+        D3 avc = dz3(), apos = dz3();
+        for_T(a, G, f3of(t.Q[i]), r, [&](uint32_t q) {
+            const float4 pl = a.gP[q];
+            const float4 vl = a.gV[q];
+            if (__float_as_uint(pl.w) == i || vl.w != 0.f) return;
+            const D3 pd = pi - wid(pl);
+            if (dot3(pd, pd) > (double)P.cut2_w) return;
+            double W, gw;
+            if (!poly6_adj(pd, k, W, gw)) return;
+            const double4 g4 = a.gD[q];
+            const D3 gl = md3(g4.x, g4.y, g4.z);
+            avc = avc + sc3(gl, k.gamma * W);
+            apos = apos + sc3(pd, gw * k.gamma * dot3(gl, vi - wid(vl)));
+        });
+        if (W > 1) {
+            avc = gsum3<W>(avc);
+            apos = gsum3<W>(apos);
+            if (r.lane) return;
+        }
+        st(a.aVc, i, ld(a.aVc, i) + avc);
+        st(a.aP, i, ld(a.aP, i) + apos);
     });
-    if (kHeavy) {
-        avc = wsum3(avc);
-        apos = wsum3(apos);
-        if (r.lane) return;
-    }
-    st(a.aVc, i, ld(a.aVc, i) + avc);
-    st(a.aP, i, ld(a.aP, i) + apos);
 }
 
 // Confinement, direct terms (Vc = V + kappa (N x omega_i), N = eta/|eta|,
 // eta_i = sum_j |omega_j| K(r) e_ij): dL/domega_i, dL/deta_i, dL/d eps;
 // dL/dV starts as dL/dVc.
-template <bool kHeavy>
+template <int L>
 __global__ __launch_bounds__(256) void k_adj_conf_own(StepTape t, AdjBufs a, Grid G, Phys P) {
-    const Role r = role<kHeavy>(t, a, 1u);
-    if (!r.on) return;
-    const uint32_t i = r.i;
-    const AdjConst k = adj_const(P);
-    const F3 selff = f3of(t.PI[i]);
-    const D3 self = wid3(selff);
-    D3 eta = dz3();
-    for_S(t, G, selff, r, [&](uint32_t j) {
-        SpikyAdj sd;
-        if (j == i || !spiky_adj(wid(t.PI[j]) - self, k, sd)) return;
-        const D3 om = wid(t.OM4[j]);
-        eta = eta + sc3(sd.f(), sqrt(dot3(om, om)));
+    for_roles<L>(t, a, 1u, [&](const Role& r, auto width) {
+        constexpr int W = decltype(width)::value;
+        const uint32_t i = r.i;
+        const AdjConst k = adj_const(P);
+        const F3 selff = f3of(t.PI[i]);
+        const D3 self = wid3(selff);
+        D3 eta = dz3();
+        for_S(t, G, selff, r, [&](uint32_t j) {
+            SpikyAdj sd;
+            if (j == i || !spiky_adj(wid(t.PI[j]) - self, k, sd)) return;
+            const D3 om = wid(t.OM4[j]);
+            eta = eta + sc3(sd.f(), sqrt(dot3(om, om)));
+        });
+        if (W > 1) {
+            eta = gsum3<W>(eta);
+            if (r.lane) return;
+        }
+        const D3 avc = ld(a.aVc, i);
+        st(a.aV, i, avc);
+        const double nr = sqrt(dot3(eta, eta));
+        D3 aom = dz3(), eb = dz3();
+        if (nr > 0.0) {
+            const D3 Nh = sc3(eta, 1.0 / nr), om = wid(t.OM4[i]);
+            a.pe[i] = dot3(avc, cross3(Nh, om)) * k.dpdvc;
+            const D3 y = sc3(avc, k.kappa);
+            aom = cross3(y, Nh);
+            const D3 nb = cross3(om, y);
+            eb = sc3(nb - sc3(Nh, dot3(Nh, nb)), 1.0 / nr);
+        }
+        st(a.aOm, i, aom);
+        st(a.etab, i, eb);
     });
-    if (kHeavy) {
-        eta = wsum3(eta);
-        if (r.lane) return;
-    }
-    const D3 avc = ld(a.aVc, i);
-    st(a.aV, i, avc);
-    const double nr = sqrt(dot3(eta, eta));
-    D3 aom = dz3(), eb = dz3();
-    if (nr > 0.0) {
-        const D3 Nh = sc3(eta, 1.0 / nr), om = wid(t.OM4[i]);
-        a.pe[i] = dot3(avc, cross3(Nh, om)) * k.dpdvc;
-        const D3 y = sc3(avc, k.kappa);
-        aom = cross3(y, Nh);
-        const D3 nb = cross3(om, y);
-        eb = sc3(nb - sc3(Nh, dot3(Nh, nb)), 1.0 / nr);
-    }
-    st(a.aOm, i, aom);
-    st(a.etab, i, eb);
 }
 
 // Confinement through eta, own pairs: the position terms of eta_i.
-template <bool kHeavy>
+template <int L>
 __global__ __launch_bounds__(256) void k_adj_eta_own(StepTape t, AdjBufs a, Grid G, Phys P) {
-    const Role r = role<kHeavy>(t, a, 1u);
-    if (!r.on) return;
-    const uint32_t i = r.i;
-    const D3 eb = ld(a.etab, i);
-    if (zero3(eb)) return;  // uniform over a heavy wave
-    const AdjConst k = adj_const(P);
-    const F3 selff = f3of(t.PI[i]);
-    const D3 self = wid3(selff);
-    D3 apos = dz3();
-    for_S(t, G, selff, r, [&](uint32_t j) {
-        SpikyAdj sd;
-        if (j == i || !spiky_adj(wid(t.PI[j]) - self, k, sd)) return;
-        const D3 om = wid(t.OM4[j]);
-        apos = apos - sc3(sd.H(eb), sqrt(dot3(om, om)));
+    for_roles<L>(t, a, 1u, [&](const Role& r, auto width) {
+        constexpr int W = decltype(width)::value;
+        const uint32_t i = r.i;
+        const D3 eb = ld(a.etab, i);
+        if (zero3(eb)) return;  // uniform over a heavy wave
+        const AdjConst k = adj_const(P);
+        const F3 selff = f3of(t.PI[i]);
+        const D3 self = wid3(selff);
+        D3 apos = dz3();
+        for_S(t, G, selff, r, [&](uint32_t j) {
+            SpikyAdj sd;
+            if (j == i || !spiky_adj(wid(t.PI[j]) - self, k, sd)) return;
+            const D3 om = wid(t.OM4[j]);
+            apos = apos - sc3(sd.H(eb), sqrt(dot3(om, om)));
+        });
+        if (W > 1) {
+            apos = gsum3<W>(apos);
+            if (r.lane) return;
+        }
+        st(a.aP, i, ld(a.aP, i) + apos);
     });
-    if (kHeavy) {
-        apos = wsum3(apos);
-        if (r.lane) return;
-    }
-    st(a.aP, i, ld(a.aP, i) + apos);
 }
 
 // Confinement through eta, transposed pairs (l, i): dL/d|omega_i| and the
 // position terms.
-template <bool kHeavy>
+template <int L>
 __global__ __launch_bounds__(256) void k_adj_eta_rev(StepTape t, AdjBufs a, Grid G, Phys P) {
-    const Role r = role<kHeavy>(t, a, 2u);
-    if (!r.on) return;
-    const uint32_t i = r.i;
-    const AdjConst k = adj_const(P);
-    const D3 self = wid(t.PI[i]);
-    const D3 omi = wid(t.OM4[i]);
-    const double wi = sqrt(dot3(omi, omi));
-    double mb = 0.0;
-    D3 apos = dz3();
-    for_T(a, G, f3of(t.Q[i]), r, [&](uint32_t q) {
-        const float4 pl = a.gP[q];
-        if (__float_as_uint(pl.w) == i) return;
-        const D3 el = ld(a.gD, q);
-        if (zero3(el)) return;
-        SpikyAdj sd;
-        if (!spiky_adj(self - wid(pl), k, sd)) return;
-        mb += dot3(el, sd.f());
-        apos = apos + sc3(sd.H(el), wi);
+    for_roles<L>(t, a, 2u, [&](const Role& r, auto width) {
+        constexpr int W = decltype(width)::value;
+        const uint32_t i = r.i;
+        const AdjConst k = adj_const(P);
+        const D3 self = wid(t.PI[i]);
+        const D3 omi = wid(t.OM4[i]);
+        const double wi = sqrt(dot3(omi, omi));
+        double mb = 0.0;
+        D3 apos = dz3();
+        for_T(a, G, f3of(t.Q[i]), r, [&](uint32_t q) {
+            const float4 pl = a.gP[q];
+            if (__float_as_uint(pl.w) == i) return;
+            const D3 el = ld(a.gD, q);
+            if (zero3(el)) return;
+            SpikyAdj sd;
+            if (!spiky_adj(self - wid(pl), k, sd)) return;
+            mb += dot3(el, sd.f());
+            apos = apos + sc3(sd.H(el), wi);
+        });
+        if (W > 1) {
+            mb = gsum<W>(mb);
+            apos = gsum3<W>(apos);
+            if (r.lane) return;
+        }
+        if (wi > 0.0) st(a.aOm, i, ld(a.aOm, i) + sc3(omi, mb / wi));
+        st(a.aP, i, ld(a.aP, i) + apos);
     });
-    if (kHeavy) {
-        mb = wsum(mb);
-        apos = wsum3(apos);
-        if (r.lane) return;
-    }
-    if (wi > 0.0) st(a.aOm, i, ld(a.aOm, i) + sc3(omi, mb / wi));
-    st(a.aP, i, ld(a.aP, i) + apos);
 }
 
 // Vorticity (omega_i = beta sum_j (V_j - V_i) x (K(r) e_ij)), own pairs:
 // dL/dV and the position terms.  V as the forward forms it (FP32).
-template <bool kHeavy>
+template <int L>
 __global__ __launch_bounds__(256) void k_adj_vort_own(StepTape t, AdjBufs a, Grid G, Phys P, uint32_t cap) {
-    const Role r = role<kHeavy>(t, a, 1u);
-    if (!r.on) return;
-    const uint32_t i = r.i;
-    const D3 ab = ld(a.aOm, i);
-    if (zero3(ab)) return;  // uniform over a heavy wave
-    const AdjConst k = adj_const(P);
-    const F3 selff = f3of(t.PI[i]);
-    const D3 self = wid3(selff);
-    const D3 vi = wid3(mulsv(P.inv_dt, selff - ld3(t.X, cap, i)));
-    D3 av = dz3(), apos = dz3();
-    for_S(t, G, selff, r, [&](uint32_t j) {
-        SpikyAdj sd;
-        const F3 pjf = f3of(t.PI[j]);
-        if (j == i || !spiky_adj(wid3(pjf) - self, k, sd)) return;
-        const D3 e = wid3(mulsv(P.inv_dt, pjf - ld3(t.X, cap, j))) - vi;
-        av = av - sc3(cross3(sd.f(), ab), k.beta);
-        apos = apos - sd.H(sc3(cross3(ab, e), k.beta));
+    for_roles<L>(t, a, 1u, [&](const Role& r, auto width) {
+        constexpr int W = decltype(width)::value;
+        const uint32_t i = r.i;
+        const D3 ab = ld(a.aOm, i);
+        if (zero3(ab)) return;  // uniform over a heavy wave
+        const AdjConst k = adj_const(P);
+        const F3 selff = f3of(t.PI[i]);
+        const D3 self = wid3(selff);
+        const D3 vi = wid3(mulsv(P.inv_dt, selff - ld3(t.X, cap, i)));
+        D3 av = dz3(), apos = dz3();
+        for_S(t, G, selff, r, [&](uint32_t j) {
+            SpikyAdj sd;
+            const F3 pjf = f3of(t.PI[j]);
+            if (j == i || !spiky_adj(wid3(pjf) - self, k, sd)) return;
+            const D3 e = wid3(mulsv(P.inv_dt, pjf - ld3(t.X, cap, j))) - vi;
+            av = av - sc3(cross3(sd.f(), ab), k.beta);
+            apos = apos - sd.H(sc3(cross3(ab, e), k.beta));
+        });
+        if (W > 1) {
+            av = gsum3<W>(av);
+            apos = gsum3<W>(apos);
+            if (r.lane) return;
+        }
+        st(a.aV, i, ld(a.aV, i) + av);
+        st(a.aP, i, ld(a.aP, i) + apos);
     });
-    if (kHeavy) {
-        av = wsum3(av);
-        apos = wsum3(apos);
-        if (r.lane) return;
-    }
-    st(a.aV, i, ld(a.aV, i) + av);
-    st(a.aP, i, ld(a.aP, i) + apos);
 }
 
 // Vorticity, transposed pairs (l, i).
-template <bool kHeavy>
+template <int L>
 __global__ __launch_bounds__(256) void k_adj_vort_rev(StepTape t, AdjBufs a, Grid G, Phys P, uint32_t cap) {
-    const Role r = role<kHeavy>(t, a, 2u);
-    if (!r.on) return;
-    const uint32_t i = r.i;
-    const AdjConst k = adj_const(P);
-    const F3 selff = f3of(t.PI[i]);
-    const D3 self = wid3(selff);
-    const D3 vi = wid3(mulsv(P.inv_dt, selff - ld3(t.X, cap, i)));
-    D3 av = dz3(), apos = dz3();
-    for_T(a, G, f3of(t.Q[i]), r, [&](uint32_t q) {
-        const float4 pl = a.gP[q];
-        if (__float_as_uint(pl.w) == i) return;
-        const D3 al = ld(a.gD, q);
-        if (zero3(al)) return;
-        SpikyAdj sd;
-        if (!spiky_adj(self - wid(pl), k, sd)) return;
-        const D3 e = vi - wid(a.gV[q]);
-        av = av + sc3(cross3(sd.f(), al), k.beta);
-        apos = apos + sd.H(sc3(cross3(al, e), k.beta));
+    for_roles<L>(t, a, 2u, [&](const Role& r, auto width) {
+        constexpr int W = decltype(width)::value;
+        const uint32_t i = r.i;
+        const AdjConst k = adj_const(P);
+        const F3 selff = f3of(t.PI[i]);
+        const D3 self = wid3(selff);
+        const D3 vi = wid3(mulsv(P.inv_dt, selff - ld3(t.X, cap, i)));
+        D3 av = dz3(), apos = dz3();
+        for_T(a, G, f3of(t.Q[i]), r, [&](uint32_t q) {
+            const float4 pl = a.gP[q];
+            if (__float_as_uint(pl.w) == i) return;
+            const D3 al = ld(a.gD, q);
+            if (zero3(al)) return;
+            SpikyAdj sd;
+            if (!spiky_adj(self - wid(pl), k, sd)) return;
+            const D3 e = vi - wid(a.gV[q]);
+            av = av + sc3(cross3(sd.f(), al), k.beta);
+            apos = apos + sd.H(sc3(cross3(al, e), k.beta));
+        });
+        if (W > 1) {
+            av = gsum3<W>(av);
+            apos = gsum3<W>(apos);
+            if (r.lane) return;
+        }
+        st(a.aV, i, ld(a.aV, i) + av);
+        st(a.aP, i, ld(a.aP, i) + apos);
     });
-    if (kHeavy) {
-        av = wsum3(av);
-        apos = wsum3(apos);
-        if (r.lane) return;
-    }
-    st(a.aV, i, ld(a.aV, i) + av);
-    st(a.aP, i, ld(a.aP, i) + apos);
 }
 
 // The update V = (P - X)/dt: dL/dP += dL/dV / dt, dL/dX = -dL/dV / dt.
@@ -718,6 +728,9 @@ __device__ void collide_jac(const Phys& P, const Boundary& B, F3& dp, F3 pk, dou
         ++sweeps;
         F3 pp = pred_x + dp;
         bool hit = false;
+        const F3 dp0 = dp;
+        double J0[9];
+        for (int q = 0; q < 9; ++q) J0[q] = J[q];
         for (uint32_t q = 0; q < B.n_inner + B.n_outer; ++q) {
             const bool is_inner = q < B.n_inner;
             const float4 s = is_inner ? B.inner[q] : B.outer[q - B.n_inner];
@@ -753,15 +766,20 @@ __device__ void collide_jac(const Phys& P, const Boundary& B, F3& dp, F3 pk, dou
             pp = pred_x + dp;
         }
         if (!hit) break;
+        // a sweep is a function of dp and J: one that changes neither ends the loop
+        bool still = same3(dp, dp0);
+        for (int q = 0; q < 9; ++q) still = still && __double_as_longlong(J[q]) == __double_as_longlong(J0[q]);
+        if (still) break;
     }
 }
 
 // dL/d(pre-collision position) = J^T dL/dP'.  dp is recomputed exactly as
 // k_deltap computes it (FP32), so the responses replay the forward's
 // decisions.
+constexpr uint32_t kCollLanes = 4;  // lanes per particle: the FP32 sum in list order (sum_pairs)
 __global__ __launch_bounds__(256) void k_adj_coll(StepTape t, AdjBufs a, const float4* __restrict__ Q, Phys P,
                                                   Boundary B, uint32_t cap) {
-    const uint32_t i = gtid();
+    const uint32_t i = gtid() / kCollLanes, l = gtid() % kCollLanes;
     if (i >= t.n_live) return;
     D3 ag = ld(a.aP, i);
     if (B.n_planes + B.n_inner + B.n_outer > 0) {
@@ -769,13 +787,8 @@ __global__ __launch_bounds__(256) void k_adj_coll(StepTape t, AdjBufs a, const f
         const F3 self = f3of(se);
         const float si = se.w;
         const float self_cl = (si < 0.f) ? -si : 0.f;
-        const uint32_t n = t.ncnt[i];
-        F3 sum = mk3(0.f, 0.f, 0.f);
-        for (uint32_t q = 0; q < n; ++q) {
-            const float4 pe = Q[t.nlist[list_at(cap, i, q)]];
-            float W;
-            F3 kg;
-            pair_terms(self, f3of(pe), P, W, kg);
+        float sum[3] = {0.f, 0.f, 0.f};
+        sum_pairs<kCollLanes>(t.nlist, cap, i, l, t.ncnt[i], self, Q, P, sum, [&](float W, F3 kg, float4 pe, float(&c)[3]) {
             const float sj = pe.w;
             float corr;
             if (P.mode == 0) {
@@ -788,121 +801,126 @@ __global__ __launch_bounds__(256) void k_adj_coll(StepTape t, AdjBufs a, const f
             } else {
                 corr = P.sk * powi(W * P.inv_wdq, P.sn);
             }
-            const float aa = -(si + sj + corr);
-            acc(sum, mulsv(aa, kg));
-        }
-        F3 dp = mk3(sum.x * P.m * P.inv_rho0, sum.y * P.m * P.inv_rho0, sum.z * P.m * P.inv_rho0);
+            const F3 ak = mulsv(-(si + sj + corr), kg);
+            c[0] = ak.x;
+            c[1] = ak.y;
+            c[2] = ak.z;
+        });
+        if (l != 0u) return;
+        F3 dp = mk3(sum[0] * P.m * P.inv_rho0, sum[1] * P.m * P.inv_rho0, sum[2] * P.m * P.inv_rho0);
         double J[9] = {1.0, 0.0, 0.0, 0.0, 1.0, 0.0, 0.0, 0.0, 1.0};
         collide_jac(P, B, dp, self, J);
         ag = md3(J[0] * ag.x + J[3] * ag.y + J[6] * ag.z, J[1] * ag.x + J[4] * ag.y + J[7] * ag.z,
                  J[2] * ag.x + J[5] * ag.y + J[8] * ag.z);
     }
-    st(a.abar, i, ag);
+    if (l == 0u) st(a.abar, i, ag);
 }
 
 // delta p = beta sum_j A_ij kg_ij, A_ij = -(s_i + s_j + corr(W_ij)):
 // dL/ds_i and the position terms through kg and corr, own pairs (i, j) and
 // transposed pairs (l, i); then the coefficients of the lambda pass.
 // Particles on long reverse lists run one wave each.
-template <bool kHeavy>
+template <int L>
 __global__ __launch_bounds__(256) void k_adj_lam(StepTape t, AdjBufs a, const float4* __restrict__ Q, Phys P,
                                                  uint32_t cap) {
-    const Role r = role<kHeavy>(t, a, 8u);
-    if (!r.on) return;
-    const uint32_t i = r.i;
-    const AdjConst k = adj_const(P);
-    const float4 se = Q[i];
-    const D3 self = wid(se);
-    const double si = se.w;
-    const D3 ai = ld(a.abar, i);
-    double sb = 0.0, kg2s = 0.0;
-    D3 kgs = dz3(), apos = dz3();
-    const uint32_t n = t.ncnt[i];
-    for (uint32_t q = r.lane; q < n; q += r.stride) {
-        const float4 pe = Q[t.nlist[list_at(cap, i, q)]];
-        const D3 d = self - wid(pe);
-        PairAdj pa;
-        if (!pair_adj(d, k, pa)) continue;  // r = 0: W = a (constant), kg = 0
-        kgs = kgs + pa.kg;
-        kg2s += dot3(pa.kg, pa.kg);
-        const double sj = pe.w;
-        const double A = -(si + sj + corr_of(k, pa.W, si, sj));
-        const double Ab = k.beta * dot3(pa.kg, ai);
-        sb -= Ab;
-        sb -= Ab * corr_ds(k, pa.W, si);
-        const double Wb = -Ab * corr_dW(k, pa.W, si, sj);
-        apos = apos + sc3(pa.H(ai), k.beta * A) + sc3(d, Wb * pa.gw);
-    }
-    const uint32_t r1 = a.roff[i + 1];
-    for (uint32_t q = a.roff[i] + r.lane; q < r1; q += r.stride) {
-        const uint32_t l = a.rlist[q];
-        const float4 pe = Q[l];
-        const D3 d = wid(pe) - self;  // the pair (l, i): d = p_l - p_i
-        PairAdj pa;
-        if (!pair_adj(d, k, pa)) continue;
-        const double sl = pe.w;
-        const D3 al = ld(a.abar, l);
-        const double A = -(sl + si + corr_of(k, pa.W, sl, si));
-        const double Ab = k.beta * dot3(pa.kg, al);
-        sb -= Ab;
-        sb -= Ab * corr_ds(k, pa.W, si);
-        const double Wb = -Ab * corr_dW(k, pa.W, sl, si);
-        apos = apos - (sc3(pa.H(al), k.beta * A) + sc3(d, Wb * pa.gw));
-    }
-    if (kHeavy) {
-        sb = wsum(sb);
-        kg2s = wsum(kg2s);
-        kgs = wsum3(kgs);
-        apos = wsum3(apos);
-        if (r.lane) return;
-    }
-    // s = C / D, C = beta sum W - 1, D = m2r2 (|sum kg|^2 + sum |kg|^2) + eps
-    const double D = k.m2r2 * (dot3(kgs, kgs) + kg2s) + k.relax;
-    const double ksb = k.beta * sb / D;
-    const double g2 = -2.0 * k.m2r2 * sb * si / D;
-    a.coef[i] = make_double4(ksb, g2 * kgs.x, g2 * kgs.y, g2 * kgs.z);
-    a.g2[i] = g2;
-    st(a.aQ, i, ai + apos);
+    for_roles<L>(t, a, 8u, [&](const Role& r, auto width) {
+        constexpr int W = decltype(width)::value;
+        const uint32_t i = r.i;
+        const AdjConst k = adj_const(P);
+        const float4 se = Q[i];
+        const D3 self = wid(se);
+        const double si = se.w;
+        const D3 ai = ld(a.abar, i);
+        double sb = 0.0, kg2s = 0.0;
+        D3 kgs = dz3(), apos = dz3();
+        const uint32_t n = t.ncnt[i];
+        for (uint32_t q = r.lane; q < n; q += r.stride) {
+            const float4 pe = Q[t.nlist[list_at(cap, i, q)]];
+            const D3 d = self - wid(pe);
+            PairAdj pa;
+            if (!pair_adj(d, k, pa)) continue;  // r = 0: W = a (constant), kg = 0
+            kgs = kgs + pa.kg;
+            kg2s += dot3(pa.kg, pa.kg);
+            const double sj = pe.w;
+            const double A = -(si + sj + corr_of(k, pa.W, si, sj));
+            const double Ab = k.beta * dot3(pa.kg, ai);
+            sb -= Ab;
+            sb -= Ab * corr_ds(k, pa.W, si);
+            const double Wb = -Ab * corr_dW(k, pa.W, si, sj);
+            apos = apos + sc3(pa.H(ai), k.beta * A) + sc3(d, Wb * pa.gw);
+        }
+        const uint32_t r1 = a.roff[i + 1];
+        for (uint32_t q = a.roff[i] + r.lane; q < r1; q += r.stride) {
+            const uint32_t l = a.rlist[q];
+            const float4 pe = Q[l];
+            const D3 d = wid(pe) - self;  // the pair (l, i): d = p_l - p_i
+            PairAdj pa;
+            if (!pair_adj(d, k, pa)) continue;
+            const double sl = pe.w;
+            const D3 al = ld(a.abar, l);
+            const double A = -(sl + si + corr_of(k, pa.W, sl, si));
+            const double Ab = k.beta * dot3(pa.kg, al);
+            sb -= Ab;
+            sb -= Ab * corr_ds(k, pa.W, si);
+            const double Wb = -Ab * corr_dW(k, pa.W, sl, si);
+            apos = apos - (sc3(pa.H(al), k.beta * A) + sc3(d, Wb * pa.gw));
+        }
+        if (W > 1) {
+            sb = gsum<W>(sb);
+            kg2s = gsum<W>(kg2s);
+            kgs = gsum3<W>(kgs);
+            apos = gsum3<W>(apos);
+            if (r.lane) return;
+        }
+        // s = C / D, C = beta sum W - 1, D = m2r2 (|sum kg|^2 + sum |kg|^2) + eps
+        const double D = k.m2r2 * (dot3(kgs, kgs) + kg2s) + k.relax;
+        const double ksb = k.beta * sb / D;
+        const double g2 = -2.0 * k.m2r2 * sb * si / D;
+        a.coef[i] = make_double4(ksb, g2 * kgs.x, g2 * kgs.y, g2 * kgs.z);
+        a.g2[i] = g2;
+        st(a.aQ, i, ai + apos);
+    });
 }
 
 // lambda pass: the position terms through W and kg of s_i (own pairs) and
 // s_l (transposed pairs); dL/dP of the iteration's input.
-template <bool kHeavy>
+template <int L>
 __global__ __launch_bounds__(256) void k_adj_pos(StepTape t, AdjBufs a, const float4* __restrict__ Q, Phys P,
                                                  uint32_t cap) {
-    const Role r = role<kHeavy>(t, a, 8u);
-    if (!r.on) return;
-    const uint32_t i = r.i;
-    const AdjConst k = adj_const(P);
-    const D3 self = wid(Q[i]);
-    const double4 ci = a.coef[i];
-    const double g2i = a.g2[i];
-    D3 apos = dz3();
-    if (ci.x != 0.0 || g2i != 0.0) {
-        const uint32_t n = t.ncnt[i];
-        for (uint32_t q = r.lane; q < n; q += r.stride) {
-            const D3 d = self - wid(Q[t.nlist[list_at(cap, i, q)]]);
+    for_roles<L>(t, a, 8u, [&](const Role& r, auto width) {
+        constexpr int W = decltype(width)::value;
+        const uint32_t i = r.i;
+        const AdjConst k = adj_const(P);
+        const D3 self = wid(Q[i]);
+        const double4 ci = a.coef[i];
+        const double g2i = a.g2[i];
+        D3 apos = dz3();
+        if (ci.x != 0.0 || g2i != 0.0) {
+            const uint32_t n = t.ncnt[i];
+            for (uint32_t q = r.lane; q < n; q += r.stride) {
+                const D3 d = self - wid(Q[t.nlist[list_at(cap, i, q)]]);
+                PairAdj pa;
+                if (!pair_adj(d, k, pa)) continue;
+                apos = apos + sc3(d, ci.x * pa.gw) + pa.H(md3(ci.y, ci.z, ci.w) + sc3(pa.kg, g2i));
+            }
+        }
+        const uint32_t r1 = a.roff[i + 1];
+        for (uint32_t q = a.roff[i] + r.lane; q < r1; q += r.stride) {
+            const uint32_t l = a.rlist[q];
+            const double4 cl = a.coef[l];
+            const double g2l = a.g2[l];
+            if (cl.x == 0.0 && g2l == 0.0) continue;
+            const D3 d = wid(Q[l]) - self;
             PairAdj pa;
             if (!pair_adj(d, k, pa)) continue;
-            apos = apos + sc3(d, ci.x * pa.gw) + pa.H(md3(ci.y, ci.z, ci.w) + sc3(pa.kg, g2i));
+            apos = apos - (sc3(d, cl.x * pa.gw) + pa.H(md3(cl.y, cl.z, cl.w) + sc3(pa.kg, g2l)));
         }
-    }
-    const uint32_t r1 = a.roff[i + 1];
-    for (uint32_t q = a.roff[i] + r.lane; q < r1; q += r.stride) {
-        const uint32_t l = a.rlist[q];
-        const double4 cl = a.coef[l];
-        const double g2l = a.g2[l];
-        if (cl.x == 0.0 && g2l == 0.0) continue;
-        const D3 d = wid(Q[l]) - self;
-        PairAdj pa;
-        if (!pair_adj(d, k, pa)) continue;
-        apos = apos - (sc3(d, cl.x * pa.gw) + pa.H(md3(cl.y, cl.z, cl.w) + sc3(pa.kg, g2l)));
-    }
-    if (kHeavy) {
-        apos = wsum3(apos);
-        if (r.lane) return;
-    }
-    st(a.aP, i, ld(a.aQ, i) + apos);
+        if (W > 1) {
+            apos = gsum3<W>(apos);
+            if (r.lane) return;
+        }
+        st(a.aP, i, ld(a.aQ, i) + apos);
+    });
 }
 
 // ------------------------------------------------------------ predict + sort
@@ -925,28 +943,26 @@ __global__ __launch_bounds__(256) void k_adj_in(StepTape t, AdjBufs a, Phys P) {
     a.avin[3 * i + 2] = gv.z;
 }
 
-// sum of v over the workgroup (256 threads), valid in thread 0
-__device__ __forceinline__ double block_sum(double v, double* sh) {
-    sh[threadIdx.x] = v;
+// psum[w] = the sum of pc (w = 0) or pe over the live slots, workgroup w, in a
+// fixed order: four strided partial sums a thread, then the threads' in a tree.
+constexpr uint32_t kReduceBlock = 1024;
+__global__ __launch_bounds__(kReduceBlock) void k_adj_reduce(StepTape t, AdjBufs a) {
+    __shared__ double sh[kReduceBlock];
+    const double* src = blockIdx.x ? a.pe : a.pc;
+    double v[4] = {0.0, 0.0, 0.0, 0.0};
+    for (uint32_t q = threadIdx.x; q < t.n_live; q += 4u * kReduceBlock)
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; ++u) {
+            const uint32_t k = q + u * kReduceBlock;
+            v[u] += k < t.n_live ? src[k] : 0.0;
+        }
+    sh[threadIdx.x] = (v[0] + v[1]) + (v[2] + v[3]);
     __syncthreads();
-    for (uint32_t s = blockDim.x / 2; s > 0; s >>= 1) {
+    for (uint32_t s = kReduceBlock / 2; s > 0; s >>= 1) {
         if (threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
         __syncthreads();
     }
-    return sh[0];
-}
-
-// psum = (sum of pc, sum of pe) over the live slots, in a fixed order
-__global__ __launch_bounds__(256) void k_adj_reduce(StepTape t, AdjBufs a) {
-    __shared__ double sh[256];
-    for (int w = 0; w < 2; ++w) {
-        const double* src = w ? a.pe : a.pc;
-        double v = 0.0;
-        for (uint32_t q = threadIdx.x; q < t.n_live; q += blockDim.x) v += src[q];
-        const double tot = block_sum(v, sh);
-        if (threadIdx.x == 0) a.psum[w] = tot;
-        __syncthreads();
-    }
+    if (threadIdx.x == 0) a.psum[blockIdx.x] = sh[0];
 }
 
 // largest |axin|, |avin| (NaN counts as infinity), as the bits of a double
@@ -959,8 +975,10 @@ __global__ __launch_bounds__(256) void k_adj_absmax(AdjBufs a, uint32_t n3) {
         if (isnan(a.axin[q]) || isnan(a.avin[q])) m = __builtin_inf();
     }
     for (int d = 32; d > 0; d >>= 1) m = fmax(m, __shfl_xor(m, d, 64));
-    if ((threadIdx.x & 63u) == 0 && m > 0.0)
-        atomicMax(a.amax, (unsigned long long)__double_as_longlong(m));
+    // a stale read only costs an atomic; one address takes about 10 ns each
+    const unsigned long long bits = (unsigned long long)__double_as_longlong(m);
+    if ((threadIdx.x & 63u) == 0 && m > 0.0 && bits > *reinterpret_cast<volatile unsigned long long*>(a.amax))
+        atomicMax(a.amax, bits);
 }
 
 __global__ __launch_bounds__(256) void k_adj_scale(double* x, double* y, uint32_t n, double f) {
@@ -980,10 +998,22 @@ __global__ __launch_bounds__(256) void k_adj_ident(const uint32_t* __restrict__ 
 
 inline uint32_t nblk(uint32_t n) { return (n + 255u) / 256u; }
 
+// Lanes per particle of the light groups: 16 while that leaves the chip about
+// full, 8 above (a pass of the differentiable form with 16 / 8 / 4 lanes: 5.9 /
+// 7.9 / 11.0 ms for 8,000 particles, 29.2 / 30.0 / 35.8 for 65,536, 14.5 / 12.1 /
+// 11.9 for 163,840 over 6, 10 and 4 steps).  Reductions over lanes reorder the
+// FP64 sums; the rule fixes the order for a particle count.
+constexpr uint32_t kAdjRowMax = 81920;
+template <class F>
+void adj_lanes(uint32_t n, F&& f) {
+    if (n <= kAdjRowMax) f(std::integral_constant<int, 16>{});
+    else f(std::integral_constant<int, 8>{});
+}
+
 }  // namespace
 
 hipError_t launch_adj_step(const Bufs& b, const Scene& s0, const StepTape& t, const AdjBufs& a, int iters,
-                           hipStream_t s, uint32_t* h_nh) {
+                           hipStream_t s) {
     const Grid& G = s0.G;
     const Phys& P = s0.P;
     const uint32_t nl = t.n_live;
@@ -1003,65 +1033,47 @@ hipError_t launch_adj_step(const Bufs& b, const Scene& s0, const StepTape& t, co
         e = launch_sort_cells(a.coffset, a.big, a.nbig, a.ctmp, a.crank, a.cap, s);
         if (e != hipSuccess) return e;
         hipLaunchKernelGGL(k_adj_corder, gl, blk, 0, s, t, a);
-        // heavy lists of the final passes and the search cells: their
-        // lengths size the heavy launches
         e = hipMemsetAsync(a.nh, 0, 4 * sizeof(uint32_t), s);
         if (e != hipSuccess) return e;
         hipLaunchKernelGGL(k_adj_classify, gl, blk, 0, s, t, a, G);
-        e = hipMemcpyAsync(h_nh, a.nh, 3 * sizeof(uint32_t), hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
-        if (e != hipSuccess) return e;
-        auto ghv = [](uint32_t n) { return dim3(nblk(n * 64u > 0 ? n * 64u : 1u)); };
-        const uint32_t hs = h_nh[0], ht = h_nh[1], hn = h_nh[2];
         // reverse lists
         hipLaunchKernelGGL(k_adj_last, gl, blk, 0, s, t, a, G, P, cap);
-        hipLaunchKernelGGL((k_adj_rev<false, false>), gl, blk, 0, s, t, a, G, P);
-        if (hn) hipLaunchKernelGGL((k_adj_rev<false, true>), ghv(hn), blk, 0, s, t, a, G, P);
-        e = launch_count_scan(a.rcount, a.roff, a.rtsum, a.rtflag, a.rtprefix, a.nRT, a.lgRT, a.RT, s);
+        adj_lanes(nl, [&](auto width) {
+            constexpr int L = decltype(width)::value;
+            const dim3 gp(nblk(nl * (uint32_t)L) + kAdjHeavyBlocks);
+            hipLaunchKernelGGL((k_adj_rev<false, L>), gp, blk, 0, s, t, a, G, P);
+            e = launch_count_scan(a.rcount, a.roff, a.rtsum, a.rtflag, a.rtprefix, a.nRT, a.lgRT, a.RT, s);
+            if (e != hipSuccess) return;
+            hipLaunchKernelGGL((k_adj_rev<true, L>), gp, blk, 0, s, t, a, G, P);
+            // final stage
+            hipLaunchKernelGGL(k_adj_final_init, gl, blk, 0, s, t, a);
+            if (P.xsph_on) {
+                hipLaunchKernelGGL(k_adj_xsph_own<L>, gp, blk, 0, s, t, a, G, P);
+                hipLaunchKernelGGL(k_adj_gather, gl, blk, 0, s, t, a, P, cap, 0);
+                hipLaunchKernelGGL(k_adj_xsph_rev<L>, gp, blk, 0, s, t, a, G, P);
+            }
+            if (P.vort_on) {
+                hipLaunchKernelGGL(k_adj_conf_own<L>, gp, blk, 0, s, t, a, G, P);
+                hipLaunchKernelGGL(k_adj_eta_own<L>, gp, blk, 0, s, t, a, G, P);
+                hipLaunchKernelGGL(k_adj_gather, gl, blk, 0, s, t, a, P, cap, 1);
+                hipLaunchKernelGGL(k_adj_eta_rev<L>, gp, blk, 0, s, t, a, G, P);
+                hipLaunchKernelGGL(k_adj_gather, gl, blk, 0, s, t, a, P, cap, 2);
+                hipLaunchKernelGGL(k_adj_vort_own<L>, gp, blk, 0, s, t, a, G, P, cap);
+                hipLaunchKernelGGL(k_adj_vort_rev<L>, gp, blk, 0, s, t, a, G, P, cap);
+            }
+            hipLaunchKernelGGL(k_adj_update, gl, blk, 0, s, t, a, P, P.vort_on);
+            // Jacobi iterations, last first
+            for (int it = iters - 1; it >= 0; --it) {
+                const float4* Q = t.Q + (size_t)it * cap;
+                hipLaunchKernelGGL(k_adj_coll, dim3(nblk(nl * kCollLanes)), blk, 0, s, t, a, Q, P, s0.B, cap);
+                hipLaunchKernelGGL(k_adj_lam<L>, gp, blk, 0, s, t, a, Q, P, cap);
+                hipLaunchKernelGGL(k_adj_pos<L>, gp, blk, 0, s, t, a, Q, P, cap);
+            }
+        });
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL((k_adj_rev<true, false>), gl, blk, 0, s, t, a, G, P);
-        if (hn) hipLaunchKernelGGL((k_adj_rev<true, true>), ghv(hn), blk, 0, s, t, a, G, P);
-        e = hipMemcpyAsync(h_nh + 3, a.nh + 3, sizeof(uint32_t), hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
-        if (e != hipSuccess) return e;
-        const uint32_t hr = h_nh[3];
-        const dim3 ghS = ghv(hs), ghT = ghv(ht);
-        // final stage
-        hipLaunchKernelGGL(k_adj_final_init, gl, blk, 0, s, t, a);
-        if (P.xsph_on) {
-            hipLaunchKernelGGL(k_adj_xsph_own<false>, gl, blk, 0, s, t, a, G, P);
-            if (hs) hipLaunchKernelGGL(k_adj_xsph_own<true>, ghS, blk, 0, s, t, a, G, P);
-            hipLaunchKernelGGL(k_adj_gather, gl, blk, 0, s, t, a, P, cap, 0);
-            hipLaunchKernelGGL(k_adj_xsph_rev<false>, gl, blk, 0, s, t, a, G, P);
-            if (ht) hipLaunchKernelGGL(k_adj_xsph_rev<true>, ghT, blk, 0, s, t, a, G, P);
-        }
-        if (P.vort_on) {
-            hipLaunchKernelGGL(k_adj_conf_own<false>, gl, blk, 0, s, t, a, G, P);
-            if (hs) hipLaunchKernelGGL(k_adj_conf_own<true>, ghS, blk, 0, s, t, a, G, P);
-            hipLaunchKernelGGL(k_adj_eta_own<false>, gl, blk, 0, s, t, a, G, P);
-            if (hs) hipLaunchKernelGGL(k_adj_eta_own<true>, ghS, blk, 0, s, t, a, G, P);
-            hipLaunchKernelGGL(k_adj_gather, gl, blk, 0, s, t, a, P, cap, 1);
-            hipLaunchKernelGGL(k_adj_eta_rev<false>, gl, blk, 0, s, t, a, G, P);
-            if (ht) hipLaunchKernelGGL(k_adj_eta_rev<true>, ghT, blk, 0, s, t, a, G, P);
-            hipLaunchKernelGGL(k_adj_gather, gl, blk, 0, s, t, a, P, cap, 2);
-            hipLaunchKernelGGL(k_adj_vort_own<false>, gl, blk, 0, s, t, a, G, P, cap);
-            if (hs) hipLaunchKernelGGL(k_adj_vort_own<true>, ghS, blk, 0, s, t, a, G, P, cap);
-            hipLaunchKernelGGL(k_adj_vort_rev<false>, gl, blk, 0, s, t, a, G, P, cap);
-            if (ht) hipLaunchKernelGGL(k_adj_vort_rev<true>, ghT, blk, 0, s, t, a, G, P, cap);
-        }
-        hipLaunchKernelGGL(k_adj_update, gl, blk, 0, s, t, a, P, P.vort_on);
-        // Jacobi iterations, last first
-        for (int it = iters - 1; it >= 0; --it) {
-            const float4* Q = t.Q + (size_t)it * cap;
-            hipLaunchKernelGGL(k_adj_coll, gl, blk, 0, s, t, a, Q, P, s0.B, cap);
-            hipLaunchKernelGGL(k_adj_lam<false>, gl, blk, 0, s, t, a, Q, P, cap);
-            if (hr) hipLaunchKernelGGL(k_adj_lam<true>, ghv(hr), blk, 0, s, t, a, Q, P, cap);
-            hipLaunchKernelGGL(k_adj_pos<false>, gl, blk, 0, s, t, a, Q, P, cap);
-            if (hr) hipLaunchKernelGGL(k_adj_pos<true>, ghv(hr), blk, 0, s, t, a, Q, P, cap);
-        }
     }
     if (t.n_in > 0) hipLaunchKernelGGL(k_adj_in, dim3(nblk(t.n_in)), blk, 0, s, t, a, P);
-    hipLaunchKernelGGL(k_adj_reduce, dim3(1), blk, 0, s, t, a);
+    hipLaunchKernelGGL(k_adj_reduce, dim3(2), dim3(kReduceBlock), 0, s, t, a);
     return hipGetLastError();
 }
 

@@ -47,7 +47,6 @@ struct AdjState {
     AdjBufs a{};
     unsigned long long* h_amax = nullptr;  // pinned
     double* h_psum = nullptr;         // pinned [2]
-    uint32_t* h_nh = nullptr;         // pinned [4]
 };
 
 struct pbfx_ctx {
@@ -228,7 +227,6 @@ void free_adj(pbfx_ctx* c) {
         if (p) (void)hipFree(p);
     if (A->h_amax) (void)hipHostFree(A->h_amax);
     if (A->h_psum) (void)hipHostFree(A->h_psum);
-    if (A->h_nh) (void)hipHostFree(A->h_nh);
     delete A;
     c->adj = nullptr;
 }
@@ -1204,7 +1202,6 @@ pbfx_status pbfx_adj_enable(pbfx_ctx* c, uint32_t max_steps, uint32_t every) {
     if (e == hipSuccess) e = hipMemset(a.rtflag, 0, ((size_t)a.nRT + 1) * sizeof(uint32_t));
     if (e == hipSuccess) e = hipHostMalloc((void**)&A->h_amax, sizeof(*A->h_amax), hipHostMallocDefault);
     if (e == hipSuccess) e = hipHostMalloc((void**)&A->h_psum, 2 * sizeof(double), hipHostMallocDefault);
-    if (e == hipSuccess) e = hipHostMalloc((void**)&A->h_nh, 4 * sizeof(uint32_t), hipHostMallocDefault);
     if (e != hipSuccess) {
         free_adj(c);
         return hip_fail(c, e);
@@ -1336,7 +1333,7 @@ pbfx_status pbfx_adj_backward(pbfx_ctx* c, const double* gx, const double* gv, d
         }
         for (uint32_t t = t1; t-- > t0;) {
             const StepTape& T = A->tape[t - t0];
-            e = launch_adj_step(c->b, c->last_table[0], T, a, (int)A->iters, s, A->h_nh);
+            e = launch_adj_step(c->b, c->last_table[0], T, a, (int)A->iters, s);
             if (e == hipSuccess) e = launch_adj_absmax(a, T.n_in, s);
             if (e == hipSuccess) e = hipMemcpyAsync(A->h_psum, a.psum, 2 * sizeof(double), hipMemcpyDeviceToHost, s);
             if (e == hipSuccess) e = hipMemcpyAsync(A->h_amax, a.amax, sizeof(*a.amax), hipMemcpyDeviceToHost, s);

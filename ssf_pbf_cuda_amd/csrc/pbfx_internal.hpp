@@ -320,7 +320,7 @@ struct AdjBufs {
     unsigned long long* amax;  // [1] largest |adjoint| of the step input, as the bits of a double
 };
 constexpr uint32_t kAdjMaxBlocks = 4096;   // workgroups of a per-particle adjoint launch
-constexpr uint32_t kAdjHeavy = 256;        // candidates above which a particle gets a wave
+constexpr uint32_t kAdjHeavy = 1024;       // candidates above which a particle gets a wave
 
 // Launchers (pbfx_kernels.hip).  All enqueue on `s` and never synchronise.
 // n_in: particles entering (all scenes); uw: cells per work unit along x,
@@ -358,10 +358,9 @@ hipError_t launch_fill_u32(uint32_t* p, size_t n, uint32_t value, hipStream_t s)
 
 // Adjoint launchers (pbfx_adjoint.hip).  launch_adj_step: dL/d(step input)
 // into a.axin / a.avin from a.ax / a.av, and the step's dL/dc, dL/d eps into
-// a.psum, for the recorded step t of the single scene s0.  It waits on `s`
-// twice, to read the heavy-list lengths into h_nh (pinned, 4 words).
+// a.psum, for the recorded step t of the single scene s0.
 hipError_t launch_adj_step(const Bufs& b, const Scene& s0, const StepTape& t, const AdjBufs& a, int iters,
-                           hipStream_t s, uint32_t* h_nh);
+                           hipStream_t s);
 // a.amax = max |a.axin|, |a.avin| over n rows (as double bits).
 hipError_t launch_adj_absmax(const AdjBufs& a, uint32_t n, hipStream_t s);
 // x[0..n) *= f for each of the arrays (may be NULL).
