@@ -652,26 +652,17 @@ __device__ __forceinline__ uint32_t wave_rank(uint32_t* ctr, uint32_t k, bool ac
 // each distinct key of the wave once and touches no memory, so that the
 // wave's atomics are all in flight together afterwards.
 __device__ __forceinline__ uint32_t wave_rank_any(uint32_t* ctr, uint32_t k, bool active, uint32_t slot) {
-    const uint32_t lane = lane_id();
-    const uint64_t below = (1ull << lane) - 1ull;
-    uint64_t todo = __ballot(active);
-    uint32_t leader = lane, rank = 0, cnt = 0;
+    uint64_t todo = __ballot(active), peers = 0;
     while (todo) {
-        const int l = __ffsll((unsigned long long)todo) - 1;
-        const uint32_t kl = (uint32_t)__shfl((int)k, l, 64);
-        const bool mine = active && k == kl;
-        const uint64_t m = __ballot(mine);
-        if (mine) {
-            leader = (uint32_t)l;
-            rank = (uint32_t)__popcll(m & below);
-        }
-        if (lane == (uint32_t)l) cnt = (uint32_t)__popcll(m);
+        const uint32_t kl = (uint32_t)__builtin_amdgcn_readlane((int)k, __builtin_ctzll(todo));
+        const uint64_t m = __ballot(active && k == kl);
+        if (k == kl) peers = m;
         todo &= ~m;
     }
+    const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(peers >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)peers, 0u));
     uint32_t base = 0;
-    if (active && leader == lane) base = atomicAdd(&ctr[slot], cnt);
-    base = (uint32_t)__shfl((int)base, (int)leader, 64);
-    return base + rank;
+    if (active && rank == 0u) base = atomicAdd(&ctr[slot], (uint32_t)__popcll(peers));
+    return (uint32_t)__shfl((int)base, peers ? __builtin_ctzll(peers) : 0, 64) + rank;
 }
 
 // Marks a scan tile as occupied: a read first, so that the common case (the

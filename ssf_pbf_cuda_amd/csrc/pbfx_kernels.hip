@@ -165,7 +165,7 @@ __global__ __launch_bounds__(1024) void k_scan_tiles(const uint32_t* __restrict_
 //                unit with more than kChunk own particles into several items
 //                that share its neighbourhood (item = (first cell, W | chunk
 //                << 6)).  Also counts the occupied tiles (CTR_SCANTILES).
-//   EMIT_FINAL   each run of uw final cells (nc = 1 << lgnc counters) holding
+//   EMIT_FINAL   each run of uw final cells (1 << lgrun counters) holding
 //                at least kSparse particles, one item per kChunk of them.
 // Listed here, the counter takes one atomic per occupied tile (128 on the 1M
 // dam).  Listed by the wave that meets a run's first particle, as the reorder
@@ -175,7 +175,7 @@ __global__ __launch_bounds__(1024) void k_scan_tiles(const uint32_t* __restrict_
 // the two scans 18 us together, now 23.
 enum EmitMode : int { EMIT_NONE = 0, EMIT_SEARCH, EMIT_FINAL };
 struct EmitArgs {
-    uint32_t uw, lguw, budget;
+    uint32_t uw, lguw, lgrun, budget;  // lgrun: tile words per run
     uint2* units;
     uint32_t* nunits;
 };
@@ -263,7 +263,7 @@ __global__ __launch_bounds__(256) void k_scan_cells(uint32_t* __restrict__ count
     // thread t takes consecutive runs, so that the items stay in key order
     __shared__ uint32_t ubase;
     auto off = [&](uint32_t c) { return cell[at(c)]; };
-    const uint32_t lgrun = kEmit == EMIT_SEARCH ? E.lguw : lgnc;  // tile words per run
+    const uint32_t lgrun = E.lgrun;
     const uint32_t nrun = T >> lgrun, rper = (nrun + blockDim.x - 1) / blockDim.x;
     const uint32_t r0 = threadIdx.x * rper, r1 = min(r0 + rper, nrun);
     auto items = [&](auto&& item) {
@@ -1278,13 +1278,17 @@ __global__ __launch_bounds__(256) void k_deltap(Bufs b, Scenes<kB> SC) {
 // The vorticity, confinement and XSPH sums visit the 27 cells around each
 // particle's FINAL position, bucketed by the search's cell ranges
 // (pbf/interaction/cuda/detail/pbf_contribution.inl:7-57).  Particles are
-// regrouped by run of uw final cells along x (the work unit of the final
-// passes; the order inside a run is irrelevant, every sum is per particle):
-// a counting sort over C/uw runs.  Each run has nc = min(8, uw) counters,
-// one per group of workgroups (b mod nc, i.e. per XCD), each on its own cache
-// line (count_slot), so that a run that collects particles from all over the
-// domain -- a wall or corner pile of ~20k particles on the 1M dam -- is not
-// counted through one contended line; key = run * nc + copy.  The same
+// regrouped by run of at most eight final cells along x (the order inside a run
+// does not change a result, every sum is per particle): a counting sort.  Each
+// run has four counters, one per group of workgroups (b mod 4), each on its own
+// cache line (count_slot), so that a run that collects particles from all over
+// the domain -- a corner pile of 7,000 particles on the 1M dam -- is not counted
+// through one contended line; key = run * 4 + copy.  Narrower runs keep
+// neighbours together in the lists and gathers of the final passes, fewer
+// counters are contended: cells per run / counters 16/8, 8/4, 4/4, 1/1 take 1051,
+// 1054, 1065, 1127 us for a step of the 1M dam, 9.09, 8.99, 8.95, 9.33 ms of the
+// 8M double dam, 37.5, 36.7, 35.9, 35.8 ms for ten steps of the wild 1M flow and
+// 16.7, 16.6, 16.4, 16.4 ms for a batch of 256 scenes.  The same
 // pass packs each slot's record R = (x*, 0), (v, 0) with
 // v = inv_dt*(x* - x_sorted) (updateVelocityCUDA, pbf_update.cu:25-39), so
 // that a particle visited in run order costs one cache line.  Final cells
@@ -1421,20 +1425,20 @@ __device__ __forceinline__ F3 sum27_global(const Grid& G, CellView b, F3 self, f
 
 // Whether the final-cell run of slot g is too sparse for a unit (fewer than
 // kSparse particles).
-__device__ __forceinline__ bool sparse_run(const Bufs& b, uint32_t lgnc, uint32_t g) {
-    const uint32_t run = b.ckey[g] >> lgnc;
-    return b.coffset[(run + 1u) << lgnc] - b.coffset[run << lgnc] < kSparse;
+__device__ __forceinline__ bool sparse_run(const Bufs& b, uint32_t lgrun, uint32_t g) {
+    const uint32_t run = b.ckey[g] >> lgrun;
+    return b.coffset[(run + 1u) << lgrun] - b.coffset[run << lgrun] < kSparse;
 }
 
 // Own particles of a final-run work item: positions coffset[run] + chunk*kChunk .. of the run order.
 struct OwnCur {
     uint32_t c0, n;
 };
-__device__ __forceinline__ OwnCur own_cur(const Bufs& b, uint2 unit, uint32_t lguw, uint32_t lgnc) {
+__device__ __forceinline__ OwnCur own_cur(const Bufs& b, uint2 unit, uint32_t lguw, uint32_t lgrun) {
     OwnCur o;
     const uint32_t run = unit.x >> lguw, skip = (unit.y >> 6) * kChunk;
-    o.c0 = b.coffset[run << lgnc] + skip;
-    o.n = min(kChunk, b.coffset[(run + 1u) << lgnc] - o.c0);
+    o.c0 = b.coffset[run << lgrun] + skip;
+    o.n = min(kChunk, b.coffset[(run + 1u) << lgrun] - o.c0);
     return o;
 }
 
@@ -1490,7 +1494,7 @@ __device__ __forceinline__ bool group_final(GroupShared& S, const Bufs& b, const
 // items for their statistics.
 template <bool kB, bool kWide>
 __global__ __launch_bounds__(kBlock) void k_final_groups(Bufs b, Scenes<kB> SC, uint32_t tile_cap, uint32_t lguw,
-                                                         uint32_t lgnc, uint32_t ngroup) {
+                                                         uint32_t lgrun, uint32_t ngroup) {
     __shared__ GroupShared GS;
     Tally tl;
     if (blockIdx.x < ngroup) {
@@ -1498,13 +1502,13 @@ __global__ __launch_bounds__(kBlock) void k_final_groups(Bufs b, Scenes<kB> SC, 
         const uint32_t q = xcd_block(blockIdx.x, ngroup) * kGroups + threadIdx.x / kGroup;
         const bool active = q < b.offset[b.CT];
         const uint32_t g = active ? b.cperm[q] : 0u;
-        if (active && (threadIdx.x & (kGroup - 1u)) == 0u && sparse_run(b, lgnc, g)) tl.slowpart++;
+        if (active && (threadIdx.x & (kGroup - 1u)) == 0u && sparse_run(b, lgrun, g)) tl.slowpart++;
         by_scene<kB>((kB && active) ? b.sid[g] : 0u, active && !any_big,
                      [&](uint32_t sc) { group_final<false, kWide>(GS, b, SC[sc], q, g, tl); });
     } else {
         item_stats<kB>(b, SC, b.cunits, b.ctr[CTR_CUNITS], tile_cap, (blockIdx.x - ngroup) * kBlock + threadIdx.x,
                        (gridDim.x - ngroup) * kBlock, tl,
-                       [&](uint2 unit) { tl.slowpart += own_cur(b, unit, lguw, lgnc).n; });
+                       [&](uint2 unit) { tl.slowpart += own_cur(b, unit, lguw, lgrun).n; });
     }
     flush_tally(b.ctr, tl);
 }
@@ -2191,7 +2195,7 @@ hipError_t step_seq(const Bufs& b, const Scenes<kB>& SC, const Tuning& T, float*
     }
     {
         Mark m(tm, s, K_SCAN_CELLS);
-        const EmitArgs E{uw, lguw, budget, b.units, &b.ctr[CTR_UNITS]};
+        const EmitArgs E{uw, lguw, lguw, budget, b.units, &b.ctr[CTR_UNITS]};
         hipLaunchKernelGGL(k_scan_cells<EMIT_SEARCH>, dim3(b.nT + 1), dim3(kScanBlock), 0, s, b.count, b.offset, b.tsum,
                            b.tflag, b.tprefix, b.nT, b.lgT, CT, 0u, E, b.ctr);
     }
@@ -2247,20 +2251,21 @@ hipError_t step_seq(const Bufs& b, const Scenes<kB>& SC, const Tuning& T, float*
         hipLaunchKernelGGL(k_out<kB>, dim3(nb), dim3(256), 0, s, b, SC, (const float4*)nullptr, x, v);
         return hipGetLastError();
     }
-    // runs of uw final cells, nc = min(8, uw) counters each: CR = CT / uw * nc
-    // counters (never more than CT), scanned in tiles of up to 4096 that divide CR
-    const uint32_t lgnc = lguw < 3u ? lguw : 3u;
-    const uint32_t CR = (CT >> lguw) << lgnc;
+    // runs of at most eight final cells with four counters each (fewer in narrower
+    // runs): CR counters, never more than CT, lgrun of them per work unit of uw
+    // cells; scanned in tiles of up to 4096 that divide CR
+    const uint32_t lgsub = std::min(lguw, 3u), lgnc = std::min(lgsub, 2u);
+    const uint32_t lgrun = lgnc + lguw - lgsub, CR = (CT >> lguw) << lgrun;
     uint32_t lgTr = 0;
     while (lgTr < 12u && ((CR >> (lgTr + 1)) << (lgTr + 1)) == CR && (1u << (lgTr + 1)) <= CR) ++lgTr;
     const uint32_t nTr = CR >> lgTr;
     {
         Mark m(tm, s, K_CUR_SORT);
-        hipLaunchKernelGGL(k_cur_hash<kB>, dim3(nb), dim3(256), 0, s, b, SC, lguw, lgnc, lgTr, CR);
+        hipLaunchKernelGGL(k_cur_hash<kB>, dim3(nb), dim3(256), 0, s, b, SC, lgsub, lgnc, lgTr, CR);
         hipLaunchKernelGGL(k_tile_reduce, dim3(nTr + 1), dim3(kScanBlock), 0, s, b.ccount, b.ctflag, b.ctsum, nTr, lgTr, CR,
                            lgnc);
         hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(1024), 0, s, b.ctsum, b.ctprefix, nTr + 1, b.ctr, 0u);
-        const EmitArgs E{uw, lguw, 0u, b.cunits, &b.ctr[CTR_CUNITS]};
+        const EmitArgs E{uw, lguw, lgrun, 0u, b.cunits, &b.ctr[CTR_CUNITS]};
         hipLaunchKernelGGL(k_scan_cells<EMIT_FINAL>, dim3(nTr + 1), dim3(kScanBlock), 0, s, b.ccount, b.coffset, b.ctsum,
                            b.ctflag, b.ctprefix, nTr, lgTr, CR, lgnc, E, (uint32_t*)nullptr);
         hipLaunchKernelGGL(k_cur_scatter, dim3(nb), dim3(256), 0, s, b.offset, CT, b.ckey, b.crank, b.coffset, b.cperm,
@@ -2271,7 +2276,7 @@ hipError_t step_seq(const Bufs& b, const Scenes<kB>& SC, const Tuning& T, float*
         by_width(b.cap, [&](auto wide) {
             const uint32_t ng = ceil_div(n, kGroups);
             hipLaunchKernelGGL((k_final_groups<kB, wide()>), dim3(ng + stat_blocks(n)), dim3(kBlock), 0, s, b, SC,
-                               kFinalTile, lguw, lgnc, ng);
+                               kFinalTile, lguw, lgrun, ng);
             hipLaunchKernelGGL((k_final_big<kB, wide()>), big_grid(n), dim3(kBlock), 0, s, b, SC);
         });
     }
