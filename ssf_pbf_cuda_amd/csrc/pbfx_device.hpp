@@ -116,12 +116,18 @@ __device__ __forceinline__ uint32_t find_scene(const uint32_t* __restrict__ off,
 }
 
 // The scenes of a launch: a single scene travels as a kernel argument;
-// several are read from the device table.
+// several are read from the device table, which no kernel writes, through the
+// constant address space: with a uniform index the constants come by scalar
+// loads into scalar registers, as a single scene's do.
 template <bool kB>
 struct Scenes {
     const Scene* table;
     Scene s0;
-    __device__ __forceinline__ const Scene& operator[](uint32_t s) const { return kB ? table[s] : s0; }
+    __device__ __forceinline__ const Scene& operator[](uint32_t s) const {
+        if (!kB) return s0;
+        using Constant = const __attribute__((address_space(4))) Scene;
+        return *(const Scene*)((Constant*)table + s);
+    }
 };
 
 template <bool kB>
@@ -129,24 +135,36 @@ __device__ __forceinline__ uint32_t scene_index(const uint32_t* __restrict__ off
     return kB ? find_scene(off, n, i) : 0u;
 }
 
+// x, computed anew at each pass of by_scene's loop: what hangs on it (a slot's
+// addresses) isn't kept in registers over the loop.
+template <bool kB>
+__device__ __forceinline__ uint32_t in_scene(uint32_t x) {
+    if (kB) asm volatile("" : "+v"(x));
+    return x;
+}
+
 // Runs f(s) for the active lanes, one scene at a time: s is uniform over the
-// lanes that call f (read from the first pending lane), so the scene's
-// constants come through scalar loads.  f must not use wave-wide operations.
+// wave (read from the first pending lane), so the scene's constants are scalar.
+// f must not use wave-wide operations.  As per-lane values the constants took up
+// to 70 vector registers a lane (vorticity 128 against 80 of a single scene,
+// XSPH 146 against 78), half the waves in flight: a step of 256 scenes 15.85 ms,
+// now 15.15.
 template <bool kB, class F>
 __device__ __forceinline__ void by_scene(uint32_t sid, bool active, F&& f) {
     if (!kB) {
         if (active) f(0u);
         return;
     }
-    bool todo = active;
-    while (__any(todo)) {
-        if (todo) {
-            const uint32_t s = __builtin_amdgcn_readfirstlane(sid);
-            if (sid == s) {
-                f(s);
-                todo = false;
-            }
-        }
+    uint64_t todo = __ballot(active);
+    while (todo) {
+        const uint32_t u = (uint32_t)__builtin_amdgcn_readlane((int)sid, __builtin_ctzll(todo));
+        // a copy that the compiler can't tell from u: where sid == u it would put the
+        // per-lane sid for it, and the scene's constants into vector registers
+        uint32_t s = u;
+        asm("" : "+s"(s));
+        const bool mine = active && sid == u;
+        todo &= ~__ballot(mine);
+        if (mine) f(s);
     }
 }
 

@@ -1082,7 +1082,7 @@ __global__ __launch_bounds__(kBlock) void k_ns_groups(Bufs b, Scenes<kB> SC, uin
         const uint32_t g = xcd_block(blockIdx.x, ngroup) * kGroups + threadIdx.x / kGroup;
         const bool active = g < b.offset[b.CT];
         by_scene<kB>((kB && active) ? b.sid[g] : 0u, active,
-                     [&](uint32_t sc) { group_search<false, kWide>(GS, b, SC[sc], g, tl); });
+                     [&](uint32_t sc) { group_search<false, kWide>(GS, b, SC[sc], in_scene<kB>(g), tl); });
     } else {
         item_stats<kB>(b, SC, b.units, b.ctr[CTR_UNITS], tile_cap, (blockIdx.x - ngroup) * kBlock + threadIdx.x,
                        (gridDim.x - ngroup) * kBlock, tl, [](uint2) {});
@@ -1202,9 +1202,10 @@ __global__ __launch_bounds__(kBlock) void k_ns_big(Bufs b, Scenes<kB> SC) {
 template <bool kB, int L>
 __global__ __launch_bounds__(256) void k_lambda(Bufs b, Scenes<kB> SC) {
     const uint32_t t = xcd_block() * blockDim.x + threadIdx.x;
-    const uint32_t i = t / L, l = t % L;
-    const bool active = i < b.offset[b.CT];
-    by_scene<kB>((kB && active) ? b.sid[i] : 0u, active, [&](uint32_t sc) {
+    const uint32_t slot = t / L, l = t % L;
+    const bool active = slot < b.offset[b.CT];
+    by_scene<kB>((kB && active) ? b.sid[slot] : 0u, active, [&](uint32_t sc) {
+        const uint32_t i = in_scene<kB>(slot);
         const Phys P = SC[sc].P;
         const F3 self = f3of(b.Pf[i]);
         float a[5] = {0.f, 0.f, 0.f, 0.f, 0.f};  // sum W, sum kg, sum |kg|^2
@@ -1232,10 +1233,11 @@ __global__ __launch_bounds__(256) void k_lambda(Bufs b, Scenes<kB> SC) {
 template <bool kB, int L>
 __global__ __launch_bounds__(256) void k_deltap(Bufs b, Scenes<kB> SC) {
     const uint32_t t = xcd_block() * blockDim.x + threadIdx.x;
-    const uint32_t i = t / L, l = t % L;
-    const bool active = i < b.offset[b.CT];
+    const uint32_t slot = t / L, l = t % L;
+    const bool active = slot < b.offset[b.CT];
     Tally tl;
-    by_scene<kB>((kB && active) ? b.sid[i] : 0u, active, [&](uint32_t sc) {
+    by_scene<kB>((kB && active) ? b.sid[slot] : 0u, active, [&](uint32_t sc) {
+        const uint32_t i = in_scene<kB>(slot);
         const Phys P = SC[sc].P;
         const Boundary B = SC[sc].B;
         const float4 se = b.Q[i];
@@ -1510,7 +1512,7 @@ __global__ __launch_bounds__(kBlock) void k_final_groups(Bufs b, Scenes<kB> SC, 
         const uint32_t g = active ? b.cperm[q] : 0u;
         if (active && (threadIdx.x & (kGroup - 1u)) == 0u && sparse_run(b, lgrun, g)) tl.slowpart++;
         by_scene<kB>((kB && active) ? b.sid[g] : 0u, active && !any_big,
-                     [&](uint32_t sc) { group_final<false, kWide>(GS, b, SC[sc], q, g, tl); });
+                     [&](uint32_t sc) { group_final<false, kWide>(GS, b, SC[sc], in_scene<kB>(q), in_scene<kB>(g), tl); });
     } else {
         item_stats<kB>(b, SC, b.cunits, b.ctr[CTR_CUNITS], tile_cap, (blockIdx.x - ngroup) * kBlock + threadIdx.x,
                        (gridDim.x - ngroup) * kBlock, tl,
@@ -1718,7 +1720,10 @@ __device__ __forceinline__ void for_final(const Bufs& b, F&& body) {
     const uint32_t q = t / L, l = t % L;
     const bool active = q < b.offset[b.CT];
     const uint32_t g = active ? b.cperm[q] : 0u;
-    by_scene<kB>((kB && active) ? b.sid[g] : 0u, active, [&](uint32_t sc) { body(q, g, b.fcnt[q], sc, l); });
+    by_scene<kB>((kB && active) ? b.sid[g] : 0u, active, [&](uint32_t sc) {
+        const uint32_t qs = in_scene<kB>(q), gs = in_scene<kB>(g);
+        body(qs, gs, b.fcnt[qs], sc, l);
+    });
 }
 
 // The pair terms of the final passes.  Each takes its root (and the three
