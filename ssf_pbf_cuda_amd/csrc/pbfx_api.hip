@@ -346,10 +346,7 @@ pbfx_status do_step(pbfx_ctx* c, float* x, float* v, uint32_t n, const uint32_t*
 }
 
 pbfx_status read_counters(pbfx_ctx* c, hipStream_t s) {
-    hipError_t e = hipMemcpyAsync(c->h_pinned, c->b.ctr, kCtrWords * sizeof(uint32_t), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(c->h_pinned + kCtrWords, c->b.offset + c->b.CT, 2 * sizeof(uint32_t),
-                           hipMemcpyDeviceToHost, s);
+    hipError_t e = hipMemcpyAsync(c->h_pinned, c->b.ctr, (kCtrWords + 2) * sizeof(uint32_t), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) return hip_fail(c, e);
     // fold the statistics copies into h[0..CTR_NUM)
@@ -490,7 +487,7 @@ pbfx_status create_common(pbfx_ctx* c) {
     PBFX_ALLOC(b.part, (size_t)b.ovf_max * 27u * 64u);
     PBFX_ALLOC(b.tflag, (size_t)b.nT + 1);
     PBFX_ALLOC(b.ctflag, (size_t)b.nT + 1);
-    PBFX_ALLOC(b.ctr, kCtrWords);
+    PBFX_ALLOC(b.ctr, kCtrWords + 2);
     PBFX_ALLOC(c->d_scenes, n);
     PBFX_ALLOC(c->d_kbase, n + 1);
     PBFX_ALLOC(c->d_in_off, n + 1);
@@ -509,7 +506,7 @@ pbfx_status create_common(pbfx_ctx* c) {
     if (e == hipSuccess) e = hipMemset(b.ctsum, 0, ((size_t)b.nT + 1) * sizeof(uint32_t));
     if (e == hipSuccess) e = hipMemset(b.tflag, 0, ((size_t)b.nT + 1) * sizeof(uint32_t));
     if (e == hipSuccess) e = hipMemset(b.ctflag, 0, ((size_t)b.nT + 1) * sizeof(uint32_t));
-    if (e == hipSuccess) e = hipMemset(b.ctr, 0, kCtrWords * sizeof(uint32_t));
+    if (e == hipSuccess) e = hipMemset(b.ctr, 0, (kCtrWords + 2) * sizeof(uint32_t));
     if (e == hipSuccess) e = hipMemset(b.sid, 0, bc * sizeof(uint32_t));
     if (e == hipSuccess) e = hipMemcpy(c->d_kbase, kbase.data(), (n + 1) * sizeof(uint32_t), hipMemcpyHostToDevice);
     if (e == hipSuccess) {
@@ -518,6 +515,7 @@ pbfx_status create_common(pbfx_ctx* c) {
     }
     if (e != hipSuccess) return hip_fail(c, e);
     b.scenes = c->d_scenes;
+    b.live = b.ctr + kCtrWords;
     b.kbase = c->d_kbase;
     b.in_off = c->d_in_off;
     uint32_t stride = 0;
@@ -1525,10 +1523,7 @@ pbfx_status pbfx_step_static(const pbfx_params* params, const float domain_end[3
     hipStream_t s = (hipStream_t)stream;
     // the counters and flags the step accumulates into start at zero; the
     // array keeps the last call's contents, possibly of another layout
-    hipError_t e = launch_fill_u32(b.count, (size_t)CT + 1, 0u, s);
-    if (e == hipSuccess) e = launch_fill_u32(b.tflag, (size_t)nT + 1, 0u, s);
-    if (e == hipSuccess) e = launch_fill_u32(b.ccount, (size_t)CT + 1, 0u, s);
-    if (e == hipSuccess) e = launch_fill_u32(b.ctflag, (size_t)nT + 1, 0u, s);
+    hipError_t e = launch_clear_counts(b, s);
     const uint32_t uw = d->T.unit_width < G.gx ? d->T.unit_width : G.gx;
     if (e == hipSuccess)
         e = launch_step(b, S, d->T, x, v, num, iters, params->xsph_on, params->vort_on, uw < kMaxW ? uw : kMaxW, s,

@@ -222,6 +222,7 @@ struct Bufs {
     float4* part;      // [ovf_max * 27 * 64] the slots' per-cell partial sums: (slot, cell, lane)
     uint32_t ovf_max;
     uint32_t* ctr;
+    uint32_t* live;    // [2] live and input count of the last step, behind ctr so that one copy reads both (or NULL)
     uint32_t lgT;
     uint32_t nT;
 };
@@ -353,8 +354,8 @@ hipError_t launch_density(const Bufs& b, const Scene& s0, const float* x, float*
 hipError_t launch_sort_cells(const uint32_t* offset, const uint32_t* cells, const uint32_t* ncells, uint32_t* vals,
                              uint32_t* scratch, uint32_t cap, hipStream_t s);
 hipError_t launch_restore(const Bufs& b, const float* xs, const float* vs, float* xo, float* vo, hipStream_t s);
-// p[0..n) = value by a kernel (no memset node when the caller captures a graph).
-hipError_t launch_fill_u32(uint32_t* p, size_t n, uint32_t value, hipStream_t s);
+// Clears the cell counts and tile flags of both sorts, in one launch.
+hipError_t launch_clear_counts(const Bufs& b, hipStream_t s);
 
 // Adjoint launchers (pbfx_adjoint.hip).  launch_adj_step: dL/d(step input)
 // into a.axin / a.avin from a.ax / a.av, and the step's dL/dc, dL/d eps into

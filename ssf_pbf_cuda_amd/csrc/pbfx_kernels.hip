@@ -35,13 +35,16 @@ namespace {
 // Input i belongs to the scene whose input range holds it.  A batch takes
 // its input count from the device (in_off[nscenes], at most n, the count the
 // grid was sized for), so that a recorded graph of steps stays valid while
-// deletion shrinks the scenes.
+// deletion shrinks the scenes.  The first workgroup also clears the step's
+// counters.
 template <bool kB>
 __global__ __launch_bounds__(256) void k_predict_hash(const float* __restrict__ x, const float* __restrict__ v,
                                                       uint32_t n, Bufs b, Scenes<kB> SC, uint32_t* __restrict__ key,
                                                       uint32_t* __restrict__ rank, uint32_t* __restrict__ count,
                                                       uint32_t* __restrict__ tflag, uint32_t lgT) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (blockIdx.x == 0u)
+        for (uint32_t t = threadIdx.x; t < kCtrWords; t += blockDim.x) b.ctr[t] = 0;
     const bool active = i < (kB ? min(n, b.in_off[b.nscenes]) : n);
     uint32_t k = 0;
     const uint32_t si = active ? scene_index<kB>(b.in_off, b.nscenes, i) : 0u;
@@ -82,16 +85,18 @@ __device__ __forceinline__ uint32_t count_slot(uint32_t c, uint32_t C, uint32_t 
 
 // ------------------------------------------------- K2a: per-tile totals
 // Totals of the cell counts of each occupied scan tile (unoccupied tiles are
-// all zero); tile nT is the deleted bucket (cell C).
+// all zero); tile nT is the deleted bucket (cell C).  Left out up to kDirectTiles
+// tiles, where k_scan_cells sums the counts before its tile itself.
 // Scan workgroups have kScanBlock threads; a tile of at most kScanTile cells
 // gives each thread at most kScanPer of them.
-constexpr uint32_t kScanBlock = 256;
+constexpr uint32_t kScanBlock = 1024;
 constexpr uint32_t kScanPer = kScanTile / kScanBlock;
+constexpr uint32_t kScanWaves = kScanBlock / 64;
 
-__global__ __launch_bounds__(256) void k_tile_reduce(const uint32_t* __restrict__ count,
-                                                     const uint32_t* __restrict__ tflag, uint32_t* __restrict__ tsum,
-                                                     uint32_t nT, uint32_t lgT, uint32_t C, uint32_t lgnc) {
-    __shared__ uint32_t wsum[kWaves];
+__global__ __launch_bounds__(kScanBlock) void k_tile_reduce(const uint32_t* __restrict__ count,
+                                                            const uint32_t* __restrict__ tflag, uint32_t* __restrict__ tsum,
+                                                            uint32_t nT, uint32_t lgT, uint32_t C, uint32_t lgnc) {
+    __shared__ uint32_t wsum[kScanWaves];
     const uint32_t t = blockIdx.x;
     if (t == nT) {
         if (threadIdx.x == 0) tsum[nT] = count[C];
@@ -119,10 +124,10 @@ __global__ __launch_bounds__(256) void k_tile_reduce(const uint32_t* __restrict_
 
 // ------------------------------------------------- K2: scan of the tile totals
 // One workgroup: exclusive scan of tsum[0..nT] (nT real tiles + the deleted
-// bucket), and reset of the step counters.
+// bucket).  Left out up to kPrefixTiles tiles, where k_scan_cells sums the totals
+// before its tile itself.
 __global__ __launch_bounds__(1024) void k_scan_tiles(const uint32_t* __restrict__ tsum,
-                                                     uint32_t* __restrict__ tprefix, uint32_t nT1,
-                                                     uint32_t* __restrict__ ctr, uint32_t reset) {
+                                                     uint32_t* __restrict__ tprefix, uint32_t nT1) {
     __shared__ uint32_t wsum[16];
     const uint32_t per = (nT1 + blockDim.x - 1) / blockDim.x;
     const uint32_t b0 = threadIdx.x * per;
@@ -146,15 +151,21 @@ __global__ __launch_bounds__(1024) void k_scan_tiles(const uint32_t* __restrict_
             tprefix[b0 + j] = run;
             run += tsum[b0 + j];
         }
-    if (reset)
-        for (uint32_t t = threadIdx.x; t < kCtrWords; t += blockDim.x) ctr[t] = 0;
 }
 
 // ------------------------------------------------- K3: scan of the cell counts
 // Workgroup t scans the counts of cell tile t (empty tiles only write their
 // prefix), clears the counts it read and the tile's occupied flag; the last
-// workgroup writes the deleted bucket: off[C] = live count, off[C+1] = n.
+// workgroup writes the deleted bucket: off[C] = live count, off[C+1] = n (also to
+// live[0..1] when given).
 // (CUB DeviceScan::ExclusiveSum in pbf_counting_sort.cu:62-71.)
+//
+// What the cells before the tile hold comes from tprefix (k_scan_tiles), from the
+// tile totals (tprefix NULL) or from the counts themselves (tsum NULL: then
+// another workgroup may still read a count, and the next kernel over them clears
+// them).  A small step is a chain of short launches, about 2 us each and another
+// between two of them; with totals and prefixes in launches of their own, its two
+// scans were six of 35.
 //
 // With the offsets of its tile in LDS, the workgroup also lists the work
 // items of the tile's runs (kEmit, no run straddles a tile) with one atomic
@@ -195,35 +206,63 @@ __device__ __forceinline__ void search_items(uint32_t r0, uint32_t kb, uint32_t 
     }
 }
 
+// Sum of v over the workgroup.
+__device__ __forceinline__ uint32_t block_sum(uint32_t v, uint32_t* wsum) {
+    uint32_t total;
+    block_excl_scan(v, wsum, total);
+    return total;
+}
+
 template <int kEmit>
-__global__ __launch_bounds__(256) void k_scan_cells(uint32_t* __restrict__ count, uint32_t* __restrict__ offset,
-                                                    const uint32_t* __restrict__ tsum, uint32_t* __restrict__ tflag,
-                                                    const uint32_t* __restrict__ tprefix, uint32_t nT,
-                                                    uint32_t lgT, uint32_t C, uint32_t lgnc, EmitArgs E,
-                                                    uint32_t* __restrict__ stat) {
-    __shared__ uint32_t wsum[kWaves];
+__global__ __launch_bounds__(kScanBlock) void k_scan_cells(uint32_t* __restrict__ count, uint32_t* __restrict__ offset,
+                                                           const uint32_t* __restrict__ tsum, uint32_t* __restrict__ tflag,
+                                                           const uint32_t* __restrict__ tprefix, uint32_t nT,
+                                                           uint32_t lgT, uint32_t C, uint32_t lgnc, EmitArgs E,
+                                                           uint32_t* __restrict__ stat, uint32_t* __restrict__ live) {
+    __shared__ uint32_t wsum[kScanWaves];
     const uint32_t t = blockIdx.x;
+    const uint32_t T = 1u << lgT, c0 = t << lgT;
+    uint32_t base;
+    if (tprefix) {
+        base = tprefix[t];
+    } else {
+        uint32_t s = 0;
+        if (tsum) {
+            for (uint32_t j = threadIdx.x; j < t; j += kScanBlock) s += tsum[j];
+        } else {
+            const uint32_t lgw = lgT - lgnc;
+#pragma unroll 8
+            for (uint32_t j = threadIdx.x; j < c0; j += kScanBlock) {
+                const uint32_t tile = j >> lgT, in = j & (T - 1u);  // tile's words, copy by copy
+                s += count[(in >> lgw) * (C >> lgnc) + (tile << lgw) + (in & ((1u << lgw) - 1u))];
+            }
+        }
+        base = block_sum(s, wsum);
+    }
     if (t == nT) {
         if (threadIdx.x == 0) {
-            offset[C] = tprefix[nT];
-            offset[C + 1] = tprefix[nT] + tsum[nT];
-            count[C] = 0;
-            tflag[nT] = 0;
+            const uint32_t end = base + (tsum ? tsum[nT] : count[C]);
+            offset[C] = base;
+            offset[C + 1] = end;
+            if (live) {
+                live[0] = base;
+                live[1] = end;
+            }
+            if (tsum) {
+                count[C] = 0;
+                tflag[nT] = 0;
+            }
         }
         return;
     }
-    const uint32_t T = 1u << lgT;
-    const uint32_t c0 = t << lgT;
-    const uint32_t tot = tsum[t];
-    const uint32_t base = tprefix[t];
-    if (tot == 0) {
+    if ((tsum ? tsum[t] : tflag[t]) == 0u) {
         for (uint32_t i = threadIdx.x; i < T; i += blockDim.x) offset[c0 + i] = base;
         return;
     }
     if (kEmit == EMIT_SEARCH && threadIdx.x == 0) atomicAdd(&stat[CTR_NUM * (1u + (t & (kStatRep - 1u))) + CTR_SCANTILES], 1u);
     // The tile passes through LDS so that global reads and writes are
     // coalesced; thread t scans cells t*per .. t*per+per-1 there.  Word w is
-    // kept at w + w/16, so the threads' 16-word strides hit distinct banks.
+    // kept at w + w/16, so the threads' strides hit distinct banks.
     __shared__ uint32_t cell[kScanTile + kScanTile / 16 + 1];
     auto at = [](uint32_t w) { return w + (w >> 4); };
     {
@@ -252,13 +291,13 @@ __global__ __launch_bounds__(256) void k_scan_cells(uint32_t* __restrict__ count
         cell[at(my0 + j)] = run;
         run += c;
     }
-    if (kEmit != EMIT_NONE && threadIdx.x == 0) cell[at(T)] = base + tot;
+    if (kEmit != EMIT_NONE && threadIdx.x == 0) cell[at(T)] = base + total;
     __syncthreads();
     for (uint32_t i = threadIdx.x; i < T; i += blockDim.x) {
         offset[c0 + i] = cell[at(i)];
-        count[count_slot(c0 + i, C, lgnc)] = 0;
+        if (tsum) count[count_slot(c0 + i, C, lgnc)] = 0;
     }
-    if (threadIdx.x == 0) tflag[t] = 0;
+    if (tsum && threadIdx.x == 0) tflag[t] = 0;
     if (kEmit == EMIT_NONE) return;
     // thread t takes consecutive runs, so that the items stay in key order
     __shared__ uint32_t ubase;
@@ -291,12 +330,30 @@ __global__ __launch_bounds__(256) void k_scan_cells(uint32_t* __restrict__ count
 // The rank-0 particle of a cell above kSmallCell particles lists the cell
 // for k_sort_cells.
 // n_dev (a batch's device-resident input count, or NULL) bounds the inputs.
+// clear: counts and tile flags the scan left (a scan without tile totals).
+struct ClearArgs {
+    uint32_t *count, *tflag;  // NULL: nothing to clear
+    uint32_t nc, nt;
+};
+__device__ __forceinline__ void clear_counts(const ClearArgs& a) {
+    if (!a.count) return;
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, nt = gridDim.x * blockDim.x;
+    for (uint32_t i = t; i < a.nc; i += nt) a.count[i] = 0;
+    for (uint32_t i = t; i < a.nt; i += nt) a.tflag[i] = 0;
+}
+
+__global__ __launch_bounds__(256) void k_clear_counts(ClearArgs search, ClearArgs final) {
+    clear_counts(search);
+    clear_counts(final);
+}
+
 __global__ __launch_bounds__(256) void k_scatter(const uint32_t* __restrict__ key, const uint32_t* __restrict__ rank,
                                                  const uint32_t* __restrict__ offset, uint32_t* __restrict__ tmp,
                                                  uint32_t n, const uint32_t* __restrict__ n_dev,
                                                  uint32_t* __restrict__ big, uint32_t* __restrict__ nbig,
-                                                 uint32_t cap, uint32_t* __restrict__ bslot) {
+                                                 uint32_t cap, uint32_t* __restrict__ bslot, ClearArgs clear) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    clear_counts(clear);
     if (i >= (n_dev ? min(n, *n_dev) : n)) return;
     const uint32_t k = key[i], r = rank[i], o0 = offset[k];
     tmp[o0 + r] = i;
@@ -1065,31 +1122,6 @@ __device__ __forceinline__ void item_stats(const Bufs& b, const Scenes<kB>& SC, 
     }
 }
 
-// ------------------------------------------------- K6: neighbour lists
-// detectNeighborsCUDA (pbf_neighbor_search_util.cu:361-482): per particle the
-// 27 cells in z,y,x order, slots ascending, keep r2 < h^2 while fewer than
-// cap are kept; the list is frozen for all Jacobi iterations.  Stored as
-// sorted slots in groups of four (list_at), with the count in
-// ncnt[slot].  Every slot by a group of eight lanes (the first ngroup
-// workgroups, unless the step has big cells: k_ns_big); the rest of the grid
-// walks the work items for their statistics.
-template <bool kB, bool kWide>
-__global__ __launch_bounds__(kBlock) void k_ns_groups(Bufs b, Scenes<kB> SC, uint32_t tile_cap, uint32_t ngroup) {
-    __shared__ GroupShared GS;
-    Tally tl;
-    if (blockIdx.x < ngroup) {
-        if (big_cells(b)) return;
-        const uint32_t g = xcd_block(blockIdx.x, ngroup) * kGroups + threadIdx.x / kGroup;
-        const bool active = g < b.offset[b.CT];
-        by_scene<kB>((kB && active) ? b.sid[g] : 0u, active,
-                     [&](uint32_t sc) { group_search<false, kWide>(GS, b, SC[sc], in_scene<kB>(g), tl); });
-    } else {
-        item_stats<kB>(b, SC, b.units, b.ctr[CTR_UNITS], tile_cap, (blockIdx.x - ngroup) * kBlock + threadIdx.x,
-                       (gridDim.x - ngroup) * kBlock, tl, [](uint2) {});
-    }
-    flush_tally(b.ctr, tl);
-}
-
 // The search list of slot g (x* = self), built by a whole wave:
 // the 27 cells around its cell in z,y,x order with the same ranges and group
 // skips as group_list, 64 candidates at a time, lane l testing the
@@ -1163,12 +1195,10 @@ __device__ uint32_t ns_heavy_list(const Grid& G, CellView b, const float4* __res
 // a list of more than kHeavySearch candidates is then built by its group's whole
 // wave.
 template <bool kB, bool kWide>
-__global__ __launch_bounds__(kBlock) void k_ns_big(Bufs b, Scenes<kB> SC) {
-    if (!big_cells(b)) return;  // uniform over the grid
-    __shared__ GroupShared GS;
-    Tally tl;
+__device__ __forceinline__ void ns_big(GroupShared& GS, const Bufs& b, const Scenes<kB>& SC, uint32_t block,
+                                       uint32_t nblock, Tally& tl) {
     const uint32_t nl = b.offset[b.CT], nblk = (nl + kGroups - 1u) / kGroups;
-    for (uint32_t c = blockIdx.x; c < nblk; c += gridDim.x) {
+    for (uint32_t c = block; c < nblk; c += nblock) {
         const uint32_t g = c * kGroups + threadIdx.x / kGroup;
         const bool active = g < nl;
         bool left = false;
@@ -1192,6 +1222,45 @@ __global__ __launch_bounds__(kBlock) void k_ns_big(Bufs b, Scenes<kB> SC) {
             }
         }
     }
+}
+
+// ------------------------------------------------- K6: neighbour lists
+// detectNeighborsCUDA (pbf_neighbor_search_util.cu:361-482): per particle the
+// 27 cells in z,y,x order, slots ascending, keep r2 < h^2 while fewer than
+// cap are kept; the list is frozen for all Jacobi iterations.  Stored as
+// sorted slots in groups of four (list_at), with the count in
+// ncnt[slot].  Every slot by a group of eight lanes (the first ngroup
+// workgroups, unless the step has big cells: ns_big, in the same launch when kBig,
+// else in k_ns_big's); the rest of the grid walks the work items for their
+// statistics.
+template <bool kB, bool kWide, bool kBig>
+__global__ __launch_bounds__(kBlock) void k_ns_groups(Bufs b, Scenes<kB> SC, uint32_t tile_cap, uint32_t ngroup) {
+    __shared__ GroupShared GS;
+    Tally tl;
+    if (blockIdx.x < ngroup) {
+        if (big_cells(b)) {
+            if (!kBig) return;
+            ns_big<kB, kWide>(GS, b, SC, blockIdx.x, ngroup, tl);
+            flush_tally(b.ctr, tl);
+            return;
+        }
+        const uint32_t g = xcd_block(blockIdx.x, ngroup) * kGroups + threadIdx.x / kGroup;
+        const bool active = g < b.offset[b.CT];
+        by_scene<kB>((kB && active) ? b.sid[g] : 0u, active,
+                     [&](uint32_t sc) { group_search<false, kWide>(GS, b, SC[sc], in_scene<kB>(g), tl); });
+    } else {
+        item_stats<kB>(b, SC, b.units, b.ctr[CTR_UNITS], tile_cap, (blockIdx.x - ngroup) * kBlock + threadIdx.x,
+                       (gridDim.x - ngroup) * kBlock, tl, [](uint2) {});
+    }
+    flush_tally(b.ctr, tl);
+}
+
+template <bool kB, bool kWide>
+__global__ __launch_bounds__(kBlock) void k_ns_big(Bufs b, Scenes<kB> SC) {
+    if (!big_cells(b)) return;  // uniform over the grid
+    __shared__ GroupShared GS;
+    Tally tl;
+    ns_big<kB, kWide>(GS, b, SC, blockIdx.x, gridDim.x, tl);
     flush_tally(b.ctr, tl);
 }
 
@@ -1337,8 +1406,10 @@ __global__ __launch_bounds__(256) void k_cur_scatter(const uint32_t* __restrict_
                                                      const uint32_t* __restrict__ ckey,
                                                      const uint32_t* __restrict__ crank,
                                                      const uint32_t* __restrict__ coffset,
-                                                     uint32_t* __restrict__ cperm, uint32_t* __restrict__ oslot) {
+                                                     uint32_t* __restrict__ cperm, uint32_t* __restrict__ oslot,
+                                                     ClearArgs clear) {
     const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+    clear_counts(clear);
     const uint32_t nl = offset[CT];
     if (s >= nl) return;
     if (s <= (nl - 1u) / 64u) oslot[s] = kNoSlot;  // the final passes' blocks of 64 positions
@@ -1497,30 +1568,6 @@ __device__ __forceinline__ bool group_final(GroupShared& S, const Bufs& b, const
     return false;
 }
 
-// Every position by a group of eight lanes (the first ngroup workgroups, unless
-// the step has big cells: k_final_big); the rest of the grid walks the work
-// items for their statistics.
-template <bool kB, bool kWide>
-__global__ __launch_bounds__(kBlock) void k_final_groups(Bufs b, Scenes<kB> SC, uint32_t tile_cap, uint32_t lguw,
-                                                         uint32_t lgrun, uint32_t ngroup) {
-    __shared__ GroupShared GS;
-    Tally tl;
-    if (blockIdx.x < ngroup) {
-        const bool any_big = big_cells(b);
-        const uint32_t q = xcd_block(blockIdx.x, ngroup) * kGroups + threadIdx.x / kGroup;
-        const bool active = q < b.offset[b.CT];
-        const uint32_t g = active ? b.cperm[q] : 0u;
-        if (active && (threadIdx.x & (kGroup - 1u)) == 0u && sparse_run(b, lgrun, g)) tl.slowpart++;
-        by_scene<kB>((kB && active) ? b.sid[g] : 0u, active && !any_big,
-                     [&](uint32_t sc) { group_final<false, kWide>(GS, b, SC[sc], in_scene<kB>(q), in_scene<kB>(g), tl); });
-    } else {
-        item_stats<kB>(b, SC, b.cunits, b.ctr[CTR_CUNITS], tile_cap, (blockIdx.x - ngroup) * kBlock + threadIdx.x,
-                       (gridDim.x - ngroup) * kBlock, tl,
-                       [&](uint2 unit) { tl.slowpart += own_cur(b, unit, lguw, lgrun).n; });
-    }
-    flush_tally(b.ctr, tl);
-}
-
 // The final list of one particle (x* = self, final-order position q),
 // built by a whole wave: each cell's candidates (the same ranges and group
 // skips as group_list) 64 at a time, lane l testing the l-th; the hits are
@@ -1590,14 +1637,12 @@ __device__ uint32_t heavy_list(const Grid& G, CellView b, const float4* __restri
     return n;
 }
 
-// The final lists of a step with big cells, as k_ns_big builds the search's.
+// The final lists of a step with big cells, as ns_big builds the search's.
 template <bool kB, bool kWide>
-__global__ __launch_bounds__(kBlock) void k_final_big(Bufs b, Scenes<kB> SC) {
-    if (!big_cells(b)) return;  // uniform over the grid
-    __shared__ GroupShared GS;
-    Tally tl;
+__device__ __forceinline__ void final_big(GroupShared& GS, const Bufs& b, const Scenes<kB>& SC, uint32_t block,
+                                          uint32_t nblock, Tally& tl) {
     const uint32_t nl = b.offset[b.CT], nblk = (nl + kGroups - 1u) / kGroups;
-    for (uint32_t c = blockIdx.x; c < nblk; c += gridDim.x) {
+    for (uint32_t c = block; c < nblk; c += nblock) {
         const uint32_t q = c * kGroups + threadIdx.x / kGroup;
         const bool active = q < nl;
         const uint32_t g = active ? b.cperm[q] : 0u;
@@ -1621,6 +1666,39 @@ __global__ __launch_bounds__(kBlock) void k_final_big(Bufs b, Scenes<kB> SC) {
             }
         }
     }
+}
+
+// Every position by a group of eight lanes (the first ngroup workgroups, unless
+// the step has big cells: final_big, in the same launch when kBig); the rest of the grid walks the work
+// items for their statistics.
+template <bool kB, bool kWide, bool kBig>
+__global__ __launch_bounds__(kBlock) void k_final_groups(Bufs b, Scenes<kB> SC, uint32_t tile_cap, uint32_t lguw,
+                                                         uint32_t lgrun, uint32_t ngroup) {
+    __shared__ GroupShared GS;
+    Tally tl;
+    if (blockIdx.x < ngroup) {
+        const bool any_big = big_cells(b);
+        if (kBig && any_big) final_big<kB, kWide>(GS, b, SC, blockIdx.x, ngroup, tl);
+        const uint32_t q = xcd_block(blockIdx.x, ngroup) * kGroups + threadIdx.x / kGroup;
+        const bool active = q < b.offset[b.CT];
+        const uint32_t g = active ? b.cperm[q] : 0u;
+        if (active && (threadIdx.x & (kGroup - 1u)) == 0u && sparse_run(b, lgrun, g)) tl.slowpart++;
+        by_scene<kB>((kB && active) ? b.sid[g] : 0u, active && !any_big,
+                     [&](uint32_t sc) { group_final<false, kWide>(GS, b, SC[sc], in_scene<kB>(q), in_scene<kB>(g), tl); });
+    } else {
+        item_stats<kB>(b, SC, b.cunits, b.ctr[CTR_CUNITS], tile_cap, (blockIdx.x - ngroup) * kBlock + threadIdx.x,
+                       (gridDim.x - ngroup) * kBlock, tl,
+                       [&](uint2 unit) { tl.slowpart += own_cur(b, unit, lguw, lgrun).n; });
+    }
+    flush_tally(b.ctr, tl);
+}
+
+template <bool kB, bool kWide>
+__global__ __launch_bounds__(kBlock) void k_final_big(Bufs b, Scenes<kB> SC) {
+    if (!big_cells(b)) return;  // uniform over the grid
+    __shared__ GroupShared GS;
+    Tally tl;
+    final_big<kB, kWide>(GS, b, SC, blockIdx.x, gridDim.x, tl);
     flush_tally(b.ctr, tl);
 }
 
@@ -2090,11 +2168,6 @@ __global__ void k_scene_offsets(Bufs b, uint32_t* __restrict__ out) {
 
 // p[0..n) = value (grid-stride): clears counters and flags inside code that a
 // caller may capture in a graph, where memset nodes are avoided.
-__global__ __launch_bounds__(256) void k_fill_u32(uint32_t* __restrict__ p, size_t n, uint32_t value) {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-        p[i] = value;
-}
-
 __global__ void k_selftest(const float* __restrict__ a, const float* __restrict__ bb, float* __restrict__ out,
                            uint32_t n) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2184,6 +2257,28 @@ void by_width(uint32_t cap, F&& f) {
 uint32_t stat_blocks(uint32_t n) { return std::min(64u, 1u + ceil_div(n, 4096u)); }
 // workgroups of the big-cell list builds (a loop over 32 particles each)
 dim3 big_grid(uint32_t n) { return dim3(std::min(4096u, ceil_div(n, kGroups))); }
+// Tiles up to which a scan needs no launch for the tile totals (the last workgroup
+// then reads 8 x 4096 counts; a step of 10,000 particles over 8 tiles 97 us, with
+// the launch 101, of 960 over 4 tiles 150 and 155; the same at 16 tiles), and up to
+// which it needs none for their prefixes (at most 16 KiB read by each workgroup;
+// above, the reads grow with the square of the tiles).
+constexpr uint32_t kDirectTiles = 8, kPrefixTiles = 4096;
+// Particles up to which the lists of a step with big cells are built in the launch
+// of the others, which then has registers for five waves a SIMD instead of eight:
+// 40 chained steps of the wild 32,768-particle dam 18.8 ms, with launches of their
+// own 19.4; ten differentiable steps of 65,536 particles 29.0 and 29.2; 24 scenes of
+// 150,000 particles in all 287 us and 285.
+constexpr uint32_t kOneListMax = 81920;
+const uint32_t* totals_of(const uint32_t* tsum, bool direct) { return direct ? nullptr : tsum; }
+const uint32_t* prefix_of(const uint32_t* tprefix, uint32_t nT) { return nT <= kPrefixTiles ? nullptr : tprefix; }
+// The launches before k_scan_cells: the tile totals, and their prefixes.
+void scan_totals(uint32_t* count, uint32_t* tsum, uint32_t* tflag, uint32_t* tprefix, uint32_t nT, uint32_t lgT,
+                 uint32_t C, uint32_t lgnc, bool direct, hipStream_t s, Timer* tm) {
+    Mark m(tm, s, K_SCAN_TILES);
+    if (!direct)
+        hipLaunchKernelGGL(k_tile_reduce, dim3(nT + 1), dim3(kScanBlock), 0, s, count, tflag, tsum, nT, lgT, C, lgnc);
+    if (nT > kPrefixTiles) hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(1024), 0, s, tsum, tprefix, nT + 1);
+}
 dim3 lane_grid(uint32_t n, int lanes) { return dim3(ceil_div(n > 0 ? n : 1u, 256u / (uint32_t)lanes)); }
 
 template <bool kB>
@@ -2194,33 +2289,33 @@ hipError_t step_seq(const Bufs& b, const Scenes<kB>& SC, const Tuning& T, float*
     const uint32_t budget = (T.tile_cap * 3u) / 4u > 0 ? (T.tile_cap * 3u) / 4u : 1u;
     uint32_t lguw = 0;
     while ((1u << lguw) < uw) ++lguw;
-    if (n > 0) {
+    {
         Mark m(tm, s, K_PREDICT_HASH);
         hipLaunchKernelGGL(k_predict_hash<kB>, dim3(nb), dim3(256), 0, s, x, v, n, b, SC, b.key, b.rank, b.count, b.tflag,
                            b.lgT);
     }
-    {
-        Mark m(tm, s, K_SCAN_TILES);
-        hipLaunchKernelGGL(k_tile_reduce, dim3(b.nT + 1), dim3(kScanBlock), 0, s, b.count, b.tflag, b.tsum, b.nT, b.lgT, CT, 0u);
-        hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(1024), 0, s, b.tsum, b.tprefix, b.nT + 1, b.ctr, 1u);
-    }
+    const bool direct = b.nT <= kDirectTiles;
+    scan_totals(b.count, b.tsum, b.tflag, b.tprefix, b.nT, b.lgT, CT, 0u, direct, s, tm);
     {
         Mark m(tm, s, K_SCAN_CELLS);
         const EmitArgs E{uw, lguw, lguw, budget, b.units, &b.ctr[CTR_UNITS]};
-        hipLaunchKernelGGL(k_scan_cells<EMIT_SEARCH>, dim3(b.nT + 1), dim3(kScanBlock), 0, s, b.count, b.offset, b.tsum,
-                           b.tflag, b.tprefix, b.nT, b.lgT, CT, 0u, E, b.ctr);
+        hipLaunchKernelGGL(k_scan_cells<EMIT_SEARCH>, dim3(b.nT + 1), dim3(kScanBlock), 0, s, b.count, b.offset,
+                           totals_of(b.tsum, direct), b.tflag, prefix_of(b.tprefix, b.nT), b.nT, b.lgT, CT, 0u, E, b.ctr,
+                           b.live);
     }
     if (n == 0) return hipGetLastError();
     {
         Mark m(tm, s, K_SCATTER);
         hipLaunchKernelGGL(k_scatter, dim3(nb), dim3(256), 0, s, b.key, b.rank, b.offset, b.tmp, n,
-                           kB ? b.in_off + b.nscenes : (const uint32_t*)nullptr, b.big, &b.ctr[CTR_BIGCELLS], b.cap, b.bslot);
+                           kB ? b.in_off + b.nscenes : (const uint32_t*)nullptr, b.big, &b.ctr[CTR_BIGCELLS], b.cap, b.bslot,
+                           direct ? ClearArgs{b.count, b.tflag, CT + 1u, b.nT + 1u} : ClearArgs{});
         // the histogram ranks are dead after the scatter: their array holds the huge cells' chunks
         static_assert(CTR_HUGECELLS == CTR_BIGCELLS + 1, "the sort reads the two cell counts together");
         hipLaunchKernelGGL(k_sort_cells, dim3(256), dim3(1024), 0, s, b.offset, b.big, &b.ctr[CTR_BIGCELLS], b.tmp,
                            b.rank, b.cap);
-        hipLaunchKernelGGL(k_merge_huge, dim3(256), dim3(256), 0, s, b.offset, b.big, &b.ctr[CTR_BIGCELLS], b.tmp,
-                           (const uint32_t*)b.rank, b.cap);
+        if (n > kSortMax)  // else no cell is huge
+            hipLaunchKernelGGL(k_merge_huge, dim3(256), dim3(256), 0, s, b.offset, b.big, &b.ctr[CTR_BIGCELLS], b.tmp,
+                               (const uint32_t*)b.rank, b.cap);
     }
     {
         Mark m(tm, s, K_REORDER);
@@ -2234,7 +2329,12 @@ hipError_t step_seq(const Bufs& b, const Scenes<kB>& SC, const Tuning& T, float*
         Mark m(tm, s, K_NS);
         by_width(b.cap, [&](auto wide) {
             const uint32_t ng = ceil_div(n, kGroups);
-            hipLaunchKernelGGL((k_ns_groups<kB, wide()>), dim3(ng + stat_blocks(n)), dim3(kBlock), 0, s, b, SC,
+            if (n <= kOneListMax) {
+                hipLaunchKernelGGL((k_ns_groups<kB, wide(), true>), dim3(ng + stat_blocks(n)), dim3(kBlock), 0, s, b, SC,
+                                   T.tile_cap, ng);
+                return;
+            }
+            hipLaunchKernelGGL((k_ns_groups<kB, wide(), false>), dim3(ng + stat_blocks(n)), dim3(kBlock), 0, s, b, SC,
                                T.tile_cap, ng);
             hipLaunchKernelGGL((k_ns_big<kB, wide()>), big_grid(n), dim3(kBlock), 0, s, b, SC);
         });
@@ -2269,20 +2369,25 @@ hipError_t step_seq(const Bufs& b, const Scenes<kB>& SC, const Tuning& T, float*
     {
         Mark m(tm, s, K_CUR_SORT);
         hipLaunchKernelGGL(k_cur_hash<kB>, dim3(nb), dim3(256), 0, s, b, SC, lgsub, lgnc, lgTr, CR);
-        hipLaunchKernelGGL(k_tile_reduce, dim3(nTr + 1), dim3(kScanBlock), 0, s, b.ccount, b.ctflag, b.ctsum, nTr, lgTr, CR,
-                           lgnc);
-        hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(1024), 0, s, b.ctsum, b.ctprefix, nTr + 1, b.ctr, 0u);
+        const bool direct = nTr <= kDirectTiles;
+        scan_totals(b.ccount, b.ctsum, b.ctflag, b.ctprefix, nTr, lgTr, CR, lgnc, direct, s, nullptr);
         const EmitArgs E{uw, lguw, lgrun, 0u, b.cunits, &b.ctr[CTR_CUNITS]};
-        hipLaunchKernelGGL(k_scan_cells<EMIT_FINAL>, dim3(nTr + 1), dim3(kScanBlock), 0, s, b.ccount, b.coffset, b.ctsum,
-                           b.ctflag, b.ctprefix, nTr, lgTr, CR, lgnc, E, (uint32_t*)nullptr);
+        hipLaunchKernelGGL(k_scan_cells<EMIT_FINAL>, dim3(nTr + 1), dim3(kScanBlock), 0, s, b.ccount, b.coffset,
+                           totals_of(b.ctsum, direct), b.ctflag, prefix_of(b.ctprefix, nTr), nTr, lgTr, CR, lgnc, E,
+                           (uint32_t*)nullptr, (uint32_t*)nullptr);
         hipLaunchKernelGGL(k_cur_scatter, dim3(nb), dim3(256), 0, s, b.offset, CT, b.ckey, b.crank, b.coffset, b.cperm,
-                           b.oslot);
+                           b.oslot, direct ? ClearArgs{b.ccount, b.ctflag, CR + 1u, nTr + 1u} : ClearArgs{});
     }
     {
         Mark m(tm, s, K_FINAL_LIST);
         by_width(b.cap, [&](auto wide) {
             const uint32_t ng = ceil_div(n, kGroups);
-            hipLaunchKernelGGL((k_final_groups<kB, wide()>), dim3(ng + stat_blocks(n)), dim3(kBlock), 0, s, b, SC,
+            if (n <= kOneListMax) {
+                hipLaunchKernelGGL((k_final_groups<kB, wide(), true>), dim3(ng + stat_blocks(n)), dim3(kBlock), 0, s, b, SC,
+                                   kFinalTile, lguw, lgrun, ng);
+                return;
+            }
+            hipLaunchKernelGGL((k_final_groups<kB, wide(), false>), dim3(ng + stat_blocks(n)), dim3(kBlock), 0, s, b, SC,
                                kFinalTile, lguw, lgrun, ng);
             hipLaunchKernelGGL((k_final_big<kB, wide()>), big_grid(n), dim3(kBlock), 0, s, b, SC);
         });
@@ -2331,10 +2436,9 @@ hipError_t launch_step(const Bufs& b, const Scene& s0, const Tuning& T, float* x
 
 hipError_t launch_count_scan(uint32_t* count, uint32_t* offset, uint32_t* tsum, uint32_t* tflag, uint32_t* tprefix,
                              uint32_t nT, uint32_t lgT, uint32_t C, hipStream_t s) {
-    hipLaunchKernelGGL(k_tile_reduce, dim3(nT + 1), dim3(kScanBlock), 0, s, count, tflag, tsum, nT, lgT, C, 0u);
-    hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(1024), 0, s, tsum, tprefix, nT + 1, (uint32_t*)nullptr, 0u);
-    hipLaunchKernelGGL(k_scan_cells<EMIT_NONE>, dim3(nT + 1), dim3(kScanBlock), 0, s, count, offset, tsum, tflag, tprefix, nT,
-                       lgT, C, 0u, EmitArgs{}, (uint32_t*)nullptr);
+    scan_totals(count, tsum, tflag, tprefix, nT, lgT, C, 0u, false, s, nullptr);
+    hipLaunchKernelGGL(k_scan_cells<EMIT_NONE>, dim3(nT + 1), dim3(kScanBlock), 0, s, count, offset, tsum, tflag,
+                       prefix_of(tprefix, nT), nT, lgT, C, 0u, EmitArgs{}, (uint32_t*)nullptr, (uint32_t*)nullptr);
     return hipGetLastError();
 }
 
@@ -2391,10 +2495,9 @@ hipError_t launch_selftest_inv_sqrt(uint32_t lo, uint32_t hi, unsigned long long
     return hipGetLastError();
 }
 
-hipError_t launch_fill_u32(uint32_t* p, size_t n, uint32_t value, hipStream_t s) {
-    if (n == 0) return hipSuccess;
-    const size_t nb = (n + 255) / 256;
-    hipLaunchKernelGGL(k_fill_u32, dim3(nb < 4096 ? (uint32_t)nb : 4096u), dim3(256), 0, s, p, n, value);
+hipError_t launch_clear_counts(const Bufs& b, hipStream_t s) {
+    hipLaunchKernelGGL(k_clear_counts, dim3(std::min(1024u, ceil_div(b.CT + 1u, 256u))), dim3(256), 0, s,
+                       ClearArgs{b.count, b.tflag, b.CT + 1u, b.nT + 1u}, ClearArgs{b.ccount, b.ctflag, b.CT + 1u, b.nT + 1u});
     return hipGetLastError();
 }
 
