@@ -222,6 +222,13 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_cells(uint32_t* __restrict_
     __shared__ uint32_t wsum[kScanWaves];
     const uint32_t t = blockIdx.x;
     const uint32_t T = 1u << lgT, c0 = t << lgT;
+    // the tile's counts and what is summed before it are loaded together
+    uint32_t v[kScanPer];
+#pragma unroll
+    for (uint32_t k = 0; k < kScanPer; ++k) {
+        const uint32_t j = threadIdx.x + k * kScanBlock;
+        v[k] = t < nT && j < T ? count[count_slot(c0 + j, C, lgnc)] : 0u;
+    }
     uint32_t base;
     if (tprefix) {
         base = tprefix[t];
@@ -229,12 +236,20 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_cells(uint32_t* __restrict_
         uint32_t s = 0;
         if (tsum) {
             for (uint32_t j = threadIdx.x; j < t; j += kScanBlock) s += tsum[j];
+        } else if (T == kScanTile) {
+            // thread j takes four words (of one copy's region) of each tile before
+            const uint32_t in = threadIdx.x * 4u, lgw = lgT - lgnc;
+            const uint32_t* __restrict__ p = count + (in >> lgw) * (C >> lgnc) + (in & ((1u << lgw) - 1u));
+#pragma unroll 8
+            for (uint32_t k = 0; k < t; ++k) {
+                const uint4 c4 = *reinterpret_cast<const uint4*>(p + (k << lgw));
+                s += c4.x + c4.y + c4.z + c4.w;
+            }
         } else {
             const uint32_t lgw = lgT - lgnc;
-#pragma unroll 8
             for (uint32_t j = threadIdx.x; j < c0; j += kScanBlock) {
-                const uint32_t tile = j >> lgT, in = j & (T - 1u);  // tile's words, copy by copy
-                s += count[(in >> lgw) * (C >> lgnc) + (tile << lgw) + (in & ((1u << lgw) - 1u))];
+                const uint32_t in = j & (T - 1u);
+                s += count[(in >> lgw) * (C >> lgnc) + ((j >> lgT) << lgw) + (in & ((1u << lgw) - 1u))];
             }
         }
         base = block_sum(s, wsum);
@@ -265,18 +280,10 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_cells(uint32_t* __restrict_
     // kept at w + w/16, so the threads' strides hit distinct banks.
     __shared__ uint32_t cell[kScanTile + kScanTile / 16 + 1];
     auto at = [](uint32_t w) { return w + (w >> 4); };
-    {
-        uint32_t v[kScanPer];
 #pragma unroll
-        for (uint32_t k = 0; k < kScanPer; ++k) {
-            const uint32_t j = threadIdx.x + k * kScanBlock;
-            v[k] = j < T ? count[count_slot(c0 + j, C, lgnc)] : 0u;
-        }
-#pragma unroll
-        for (uint32_t k = 0; k < kScanPer; ++k) {
-            const uint32_t j = threadIdx.x + k * kScanBlock;
-            if (j < T) cell[at(j)] = v[k];
-        }
+    for (uint32_t k = 0; k < kScanPer; ++k) {
+        const uint32_t j = threadIdx.x + k * kScanBlock;
+        if (j < T) cell[at(j)] = v[k];
     }
     __syncthreads();
     const uint32_t per = (T + blockDim.x - 1) / blockDim.x;
