@@ -369,27 +369,44 @@ __global__ __launch_bounds__(256) void k_scatter(const uint32_t* __restrict__ ke
 
 // ------------------------------------------------- K4b: large cells in stable order
 // Ascending bitonic sort of src[0..len) (len <= kSortMax, distinct values)
-// into dst[0..len) through LDS, by the whole workgroup (dst may be src: all
-// of src is read before the first write).  Contains barriers: call uniformly.
+// into dst[0..len), by the whole workgroup (dst may be src: all of src is read
+// before the first write).  Exchanges over less than 64 places stay in a wave's
+// registers; wider ones go through LDS, a barrier each (28 of the 91 rounds of
+// 8,192 values; with all of them through LDS k_sort_cells took 162 us a launch over the
+// first ten chained steps of the wild 1M dam and 15.7 over 40 of the 32k dam, now 75
+// and 7.8).  Contains barriers: call uniformly.
 __device__ void lds_sort_segment(const uint32_t* src, uint32_t* dst, uint32_t len, uint32_t* __restrict__ buf) {
-    uint32_t P = 1u;
+    uint32_t P = 64u;
     while (P < len) P <<= 1;
-    for (uint32_t i = threadIdx.x; i < P; i += blockDim.x) buf[i] = i < len ? src[i] : 0xFFFFFFFFu;
+    // the rounds of k over j = from, from / 2 .. 1 (from < 64) on the value at place i
+    auto in_wave = [](uint32_t v, uint32_t i, uint32_t k, uint32_t from) {
+        for (uint32_t j = from; j > 0u; j >>= 1) {
+            const uint32_t o = (uint32_t)__shfl_xor((int)v, (int)j, 64);
+            v = ((i & j) == 0u) == ((i & k) == 0u) ? min(v, o) : max(v, o);
+        }
+        return v;
+    };
+    for (uint32_t i = threadIdx.x; i < P; i += blockDim.x) {
+        uint32_t v = i < len ? src[i] : 0xFFFFFFFFu;
+        for (uint32_t k = 2u; k <= 64u; k <<= 1) v = in_wave(v, i, k, k >> 1);
+        buf[i] = v;
+    }
     __syncthreads();
-    for (uint32_t k = 2u; k <= P; k <<= 1)
-        for (uint32_t j = k >> 1; j > 0u; j >>= 1) {
-            for (uint32_t i = threadIdx.x; i < P; i += blockDim.x) {
-                const uint32_t l = i ^ j;
-                if (l > i) {
-                    const uint32_t a = buf[i], bv = buf[l];
-                    if ((a > bv) == ((i & k) == 0u)) {
-                        buf[i] = bv;
-                        buf[l] = a;
-                    }
+    for (uint32_t k = 128u; k <= P; k <<= 1) {
+        for (uint32_t j = k >> 1; j >= 64u; j >>= 1) {
+            for (uint32_t t = threadIdx.x; t < P / 2u; t += blockDim.x) {
+                const uint32_t i = ((t & ~(j - 1u)) << 1) | (t & (j - 1u));
+                const uint32_t a = buf[i], b = buf[i + j];
+                if ((a > b) == ((i & k) == 0u)) {
+                    buf[i] = b;
+                    buf[i + j] = a;
                 }
             }
             __syncthreads();
         }
+        for (uint32_t i = threadIdx.x; i < P; i += blockDim.x) buf[i] = in_wave(buf[i], i, k, 32u);
+        __syncthreads();
+    }
     for (uint32_t i = threadIdx.x; i < len; i += blockDim.x) dst[i] = buf[i];
     __syncthreads();
 }
