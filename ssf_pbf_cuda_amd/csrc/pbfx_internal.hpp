@@ -14,7 +14,7 @@
 //   count                          u32[C+1]      cell histogram (cell C = deleted)
 //   offset                         u32[C+2]      exclusive scan: cell c owns [off[c], off[c+1])
 //   tsum, tflag, tprefix           u32[nT+1]     per-4096-cell-tile totals, occupied flags, scan
-//   units                          uint2[cap+]   work items (first cell key, width | chunk << 5)
+//   units                          uint2[cap+]   work items (first cell key, width | chunk << 6)
 //   ckey, crank, cperm, ccount, coffset, ctsum, ctprefix, cunits
 //                                                 the same sort keyed by each particle's final cell
 //   flist, fcnt                    u32[64*cap], u32[cap]  in-range pairs of the final passes by
@@ -27,8 +27,9 @@
 //                                                 each slot's block of 64 final-order positions,
 //                                                 each block's slot, and the slots' per-cell partial
 //                                                 sums (M = cap/64 + 1 in a context)
-//   ctr                            u32[16*65]    allocation counters, then 64 copies of the
-//                                                 statistics counters of the last step
+//   ctr                            u32[16*65+2]  allocation counters, then 64 copies of the
+//                                                 statistics counters of the last step, then its
+//                                                 live and input counts (contexts only)
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -1,19 +1,20 @@
 // pbfx_kernels.hip -- HIP kernels of the PBF solver step for gfx950 (CDNA4).
 //
-// One step = bookkeeping kernels (predict+hash+histogram, two-level scan,
-// scatter, stable reorder), then:
-//   k_ns          neighbour lists (frozen, capped), per work unit of cells
-//                 whose 27-cell neighbourhood is staged in LDS
-//   k_lambda      lambda over the lists, one thread per particle    (x I)
-//   k_deltap      delta-p + tensile correction + boundary response  (x I)
-//   k_cur_*       regrouping by final cell                (vort_on or xsph_on)
-//   k_final_list  in-range pairs around each final cell, per work unit
-//   k_vort        vorticity over the final lists                     (vort_on)
-//   k_confine     vorticity confinement                              (vort_on)
-//   k_xsph_out    XSPH + AoS write-back                              (xsph_on)
-//   k_out         AoS write-back                                     (otherwise)
-// All kernels are HBM/LDS-bound integer or FP32 vector work; nothing is a
-// contraction, so MFMA is not used.  Arithmetic follows the reference's
+// One step = bookkeeping kernels (predict+hash+histogram, scan, scatter, stable
+// reorder), then:
+//   k_ns_groups, k_ns_big        neighbour lists (frozen, capped), eight lanes a particle
+//   k_lambda                     lambda over the lists, 16, 4 or 1 lanes a particle (x I)
+//   k_deltap                     delta-p + tensile correction + boundary response   (x I)
+//   k_cur_*                      regrouping by final cell       (vort_on or xsph_on)
+//   k_final_groups, k_final_big  in-range pairs around each final cell
+//   k_ovf_part                   per-cell partial sums of particles in piles, before
+//                                each of the next three
+//   k_vort                       vorticity over the final lists             (vort_on)
+//   k_confine                    vorticity confinement                      (vort_on)
+//   k_xsph_out                   XSPH + AoS write-back                      (xsph_on)
+//   k_out                        AoS write-back                             (otherwise)
+// All kernels are integer or FP32 vector work; nothing is a contraction, so MFMA
+// is not used.  Arithmetic follows the reference's
 // operation order with IEEE division/sqrt and explicit fmaf (the library is
 // compiled with -ffp-contract=off), so results are reproducible bit-for-bit
 // on the host.
@@ -87,16 +88,16 @@ __device__ __forceinline__ uint32_t count_slot(uint32_t c, uint32_t C, uint32_t 
 // Totals of the cell counts of each occupied scan tile (unoccupied tiles are
 // all zero); tile nT is the deleted bucket (cell C).  Left out up to kDirectTiles
 // tiles, where k_scan_cells sums the counts before its tile itself.
-// Scan workgroups have kScanBlock threads; a tile of at most kScanTile cells
-// gives each thread at most kScanPer of them.
-constexpr uint32_t kScanBlock = 1024;
+// k_scan_cells has kScanBlock threads a workgroup; a tile of at most kScanTile
+// cells gives each thread at most kScanPer of them.
+constexpr uint32_t kScanBlock = 512;
 constexpr uint32_t kScanPer = kScanTile / kScanBlock;
 constexpr uint32_t kScanWaves = kScanBlock / 64;
 
-__global__ __launch_bounds__(kScanBlock) void k_tile_reduce(const uint32_t* __restrict__ count,
+__global__ __launch_bounds__(kBlock) void k_tile_reduce(const uint32_t* __restrict__ count,
                                                             const uint32_t* __restrict__ tflag, uint32_t* __restrict__ tsum,
                                                             uint32_t nT, uint32_t lgT, uint32_t C, uint32_t lgnc) {
-    __shared__ uint32_t wsum[kScanWaves];
+    __shared__ uint32_t wsum[kWaves];
     const uint32_t t = blockIdx.x;
     if (t == nT) {
         if (threadIdx.x == 0) tsum[nT] = count[C];
@@ -108,15 +109,15 @@ __global__ __launch_bounds__(kScanBlock) void k_tile_reduce(const uint32_t* __re
     }
     const uint32_t T = 1u << lgT, c0 = t << lgT;
     // all of a thread's loads are issued before the first add
-    uint32_t v[kScanPer];
+    uint32_t v[kScanTile / kBlock];
 #pragma unroll
-    for (uint32_t k = 0; k < kScanPer; ++k) {
-        const uint32_t j = threadIdx.x + k * kScanBlock;
+    for (uint32_t k = 0; k < kScanTile / kBlock; ++k) {
+        const uint32_t j = threadIdx.x + k * kBlock;
         v[k] = j < T ? count[count_slot(c0 + j, C, lgnc)] : 0u;
     }
     uint32_t s = 0;
 #pragma unroll
-    for (uint32_t k = 0; k < kScanPer; ++k) s += v[k];
+    for (uint32_t k = 0; k < kScanTile / kBlock; ++k) s += v[k];
     uint32_t total;
     block_excl_scan(s, wsum, total);
     if (threadIdx.x == 0) tsum[t] = total;
@@ -222,12 +223,14 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_cells(uint32_t* __restrict_
     __shared__ uint32_t wsum[kScanWaves];
     const uint32_t t = blockIdx.x;
     const uint32_t T = 1u << lgT, c0 = t << lgT;
-    // the tile's counts and what is summed before it are loaded together
+    // the tile's counts and what is summed before it are loaded together; an empty
+    // tile's are not, where the totals tell (most tiles of a large grid)
+    const bool own = t < nT && (!tsum || tsum[t] != 0u);
     uint32_t v[kScanPer];
 #pragma unroll
     for (uint32_t k = 0; k < kScanPer; ++k) {
         const uint32_t j = threadIdx.x + k * kScanBlock;
-        v[k] = t < nT && j < T ? count[count_slot(c0 + j, C, lgnc)] : 0u;
+        v[k] = own && j < T ? count[count_slot(c0 + j, C, lgnc)] : 0u;
     }
     uint32_t base;
     if (tprefix) {
@@ -237,13 +240,18 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_cells(uint32_t* __restrict_
         if (tsum) {
             for (uint32_t j = threadIdx.x; j < t; j += kScanBlock) s += tsum[j];
         } else if (T == kScanTile) {
-            // thread j takes four words (of one copy's region) of each tile before
-            const uint32_t in = threadIdx.x * 4u, lgw = lgT - lgnc;
-            const uint32_t* __restrict__ p = count + (in >> lgw) * (C >> lgnc) + (in & ((1u << lgw) - 1u));
+            // a thread takes four words (of one copy's region) at a time of each tile before
+            static_assert(kScanPer % 4u == 0u, "four words at a time");
+            const uint32_t lgw = lgT - lgnc;
+#pragma unroll
+            for (uint32_t h = 0; h < kScanPer / 4u; ++h) {
+                const uint32_t in = (threadIdx.x + h * kScanBlock) * 4u;
+                const uint32_t* __restrict__ p = count + (in >> lgw) * (C >> lgnc) + (in & ((1u << lgw) - 1u));
 #pragma unroll 8
-            for (uint32_t k = 0; k < t; ++k) {
-                const uint4 c4 = *reinterpret_cast<const uint4*>(p + (k << lgw));
-                s += c4.x + c4.y + c4.z + c4.w;
+                for (uint32_t k = 0; k < t; ++k) {
+                    const uint4 c4 = *reinterpret_cast<const uint4*>(p + (k << lgw));
+                    s += c4.x + c4.y + c4.z + c4.w;
+                }
             }
         } else {
             const uint32_t lgw = lgT - lgnc;
@@ -1446,11 +1454,11 @@ __global__ __launch_bounds__(256) void k_cur_scatter(const uint32_t* __restrict_
 // in that order.  Pairs with dot(d, d) > cut2 lie outside the kernel support
 // and add exactly +-0 for finite states; they are skipped.
 //
-// The final passes run in two stages.  k_final_list filters each particle's
-// candidates once and stores its in-range pairs (bit 31 marks the first pair
-// of each cell); the vorticity, confinement and XSPH passes then walk those
-// lists with every lane busy.  Adding only the cells that have pairs gives
-// the same sums: the skipped cells add +0.
+// The final passes run in two stages.  k_final_groups and k_final_big filter
+// each particle's candidates once and store its in-range pairs (bit 31 marks
+// the first pair of each cell); the vorticity, confinement and XSPH passes then
+// walk those lists with every lane busy.  Adding only the cells that have pairs
+// gives the same sums: the skipped cells add +0.
 
 // A candidate's records for a pass's term: p = (x*_j, pass-specific w),
 // q = the second record the pass needs (the velocity, or unused).  Loaded
@@ -2315,7 +2323,7 @@ void scan_totals(uint32_t* count, uint32_t* tsum, uint32_t* tflag, uint32_t* tpr
                  uint32_t C, uint32_t lgnc, bool direct, hipStream_t s, Timer* tm) {
     Mark m(tm, s, K_SCAN_TILES);
     if (!direct)
-        hipLaunchKernelGGL(k_tile_reduce, dim3(nT + 1), dim3(kScanBlock), 0, s, count, tflag, tsum, nT, lgT, C, lgnc);
+        hipLaunchKernelGGL(k_tile_reduce, dim3(nT + 1), dim3(kBlock), 0, s, count, tflag, tsum, nT, lgT, C, lgnc);
     if (nT > kPrefixTiles) hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(1024), 0, s, tsum, tprefix, nT + 1);
 }
 dim3 lane_grid(uint32_t n, int lanes) { return dim3(ceil_div(n > 0 ? n : 1u, 256u / (uint32_t)lanes)); }
