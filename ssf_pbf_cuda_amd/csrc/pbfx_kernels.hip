@@ -1840,15 +1840,17 @@ __device__ __forceinline__ void for_final(const Bufs& b, F&& body) {
 // divisions by it) from sqrt_inv_normal and div3_inv in a wave whose active
 // lanes all qualify (the IEEE sequences otherwise): over the piles of the first
 // ten chained steps of the 1M dam k_ovf_part went from 1.72 to 1.41 ms a launch
-// (vorticity) and from 1.58 to 1.33 ms (confinement).
+// (vorticity) and from 1.58 to 1.33 ms (confinement).  kPlain false: the IEEE
+// sequences only, the same values.
 
 // vorticity pair term (pbf_vorticity_confinement.cu:15-31)
+template <bool kPlain>
 __device__ __forceinline__ F3 vort_pair(F3 self, F3 selfv, F3 pj, F3 vj, float warg) {
     const F3 pd = pj - self;
     const F3 vd = vj - selfv;
     const float r2 = glm_dot(pd, pd);
     F3 w = mk3(0.f, 0.f, 0.f);
-    if (__builtin_expect(wave_plain_div(pd, r2), 1)) {
+    if (kPlain && __builtin_expect(wave_plain_div(pd, r2), 1)) {
         const RootInv q = sqrt_inv_normal(r2);
         if (r2 != 0.f) w = mulvs(glm_cross(vd, div3_inv(pd, q.s, q.inv)), wspiky_deriv(q.s, warg));
         return w;
@@ -1859,11 +1861,12 @@ __device__ __forceinline__ F3 vort_pair(F3 self, F3 selfv, F3 pj, F3 vj, float w
 }
 
 // confinement location-vector pair term (pbf_vorticity_confinement.cu:121-138)
+template <bool kPlain>
 __device__ __forceinline__ F3 loc_pair(F3 self, F3 pj, float wj, float warg) {
     const F3 pd = pj - self;
     const float r2 = glm_dot(pd, pd);
     F3 l = mk3(0.f, 0.f, 0.f);
-    if (__builtin_expect(wave_plain_div(pd, r2), 1)) {
+    if (kPlain && __builtin_expect(wave_plain_div(pd, r2), 1)) {
         const RootInv q = sqrt_inv_normal(r2);
         if (r2 != 0.f) l = mulvs(mulsv(wj, div3_inv(pd, q.s, q.inv)), wspiky_deriv(q.s, warg));
         return l;
@@ -1874,11 +1877,12 @@ __device__ __forceinline__ F3 loc_pair(F3 self, F3 pj, float wj, float warg) {
 }
 
 // XSPH pair term (pbf_xsph.cu:15-29)
+template <bool kPlain>
 __device__ __forceinline__ F3 xsph_pair(F3 self, F3 selfv, F3 pj, F3 vj, float inv_h) {
     const F3 pd = pj - self;
     const F3 vd = vj - selfv;
     const float r2 = glm_dot(pd, pd);
-    if (__builtin_expect(wave_plain_r2(r2), 1))
+    if (kPlain && __builtin_expect(wave_plain_r2(r2), 1))
         return mulvs(vd, wpoly6(r2 != 0.f ? sqrt_inv_normal(r2).s : 0.f, inv_h));
     return mulvs(vd, wpoly6(glm_length(pd), inv_h));
 }
@@ -1886,6 +1890,8 @@ __device__ __forceinline__ F3 xsph_pair(F3 self, F3 selfv, F3 pj, F3 vj, float i
 // The three final passes as (elements, pair term, support) for the particle
 // at slot g: the list walk, the direct sum, the per-cell partials and their
 // combination all evaluate a pass through these.
+// Blocks with overflowing positions up to which k_ovf_part sums their cells by rows.
+constexpr uint32_t kOvfRows = 20480;
 enum FinalPass : int { PASS_VORT = 0, PASS_CONF = 1, PASS_XSPH = 2 };
 
 template <int kPass>
@@ -1916,10 +1922,11 @@ struct PassTerms {
         }
         return El2{gr(2u * j), gr(2u * j + 1u)};
     }
+    template <bool kPlain = true>
     __device__ __forceinline__ F3 term(const El2& e) const {
-        if (kPass == PASS_VORT) return vort_pair(self, selfv, f3of(e.p), f3of(e.q), arg);
-        if (kPass == PASS_CONF) return loc_pair(self, f3of(e.p), e.p.w, arg);
-        return xsph_pair(self, selfv, f3of(e.p), f3of(e.q), arg);
+        if (kPass == PASS_VORT) return vort_pair<kPlain>(self, selfv, f3of(e.p), f3of(e.q), arg);
+        if (kPass == PASS_CONF) return loc_pair<kPlain>(self, f3of(e.p), e.p.w, arg);
+        return xsph_pair<kPlain>(self, selfv, f3of(e.p), f3of(e.q), arg);
     }
 };
 
@@ -2008,11 +2015,13 @@ __device__ __forceinline__ F3 pass_sum(const Bufs& b, const Grid& G, const Pass&
 // A cell of a pile is one serial sum of thousands of terms, whose length set the
 // launch's time while the chip idled (a tenth of the VALU issue) when a thread
 // did it: 139 us a launch (vorticity) over the 40 chained steps of the 32k dam and
-// 1.49 ms over the first ten of the 1M dam; by rows 48 us and 0.40 ms.
+// 1.49 ms over the first ten of the 1M dam; by rows 48 us and 0.40 ms.  Adding the
+// terms on every lane doubles the work, though: with more than kOvfRows blocks,
+// whose cells fill the chip a thread each, k_ovf_part_many does them.
 template <bool kB, int kPass>
 __global__ __launch_bounds__(256) void k_ovf_part(Bufs b, Scenes<kB> SC) {
     const uint32_t ns = min(b.ctr[CTR_OVF], b.ovf_max);
-    if (ns == 0u) return;  // uniform over the grid
+    if (ns == 0u || ns > kOvfRows) return;  // uniform over the grid
     const uint32_t nl = b.offset[b.CT], lane = lane_id(), l = lane & 15u;
     const bool any_big = big_cells(b);
     const uint64_t ntask = (uint64_t)ns * (27u * 16u);
@@ -2030,6 +2039,40 @@ __global__ __launch_bounds__(256) void k_ovf_part(Bufs b, Scenes<kB> SC) {
             const F3 cs = any_big ? sum_cell_row<true>(cell_view(b), SC[sc].G, ps, c, l)
                                   : sum_cell_row<false>(cell_view(b), SC[sc].G, ps, c, l);
             if (l == 0u) b.part[((size_t)k * 27u + c) * 64u + at] = make_float4(cs.x, cs.y, cs.z, 0.f);
+        });
+    }
+}
+
+// The same when more than kOvfRows blocks overflowed, a thread per (position,
+// cell): a wave task is (slot k, cell c), lane l summing the cell for position
+// 64 * ovf[k] + l.  Few candidates of such piles are pairs, so the terms take the
+// IEEE root without asking whether the wave's pairs allow the short one.  Chained
+// steps of the 8M double dam, 30 to 35 (2.0M particles overflow) 237 ms a step, by
+// rows 300, with the short root 261; steps 0 to 15 alike.  The 1M dam, which has at
+// most 16,384 blocks, is the slower for it (steps 0 to 60 10.7 ms against 8.2).
+template <bool kB, int kPass>
+__global__ __launch_bounds__(256) void k_ovf_part_many(Bufs b, Scenes<kB> SC) {
+    const uint32_t ns = min(b.ctr[CTR_OVF], b.ovf_max);
+    if (ns <= kOvfRows) return;  // uniform over the grid
+    const uint32_t nl = b.offset[b.CT], lane = lane_id();
+    const bool any_big = big_cells(b);
+    const uint32_t ntask = ns * 27u;
+    const uint32_t w0 = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    const uint32_t nw = (gridDim.x * blockDim.x) >> 6;
+    for (uint32_t t = w0; t < ntask; t += nw) {
+        const uint32_t k = t / 27u, c = t - k * 27u;
+        const uint32_t q = b.ovf[k] * 64u + lane;
+        const bool active = q < nl && b.fcnt[q] == kFinalK + 1u;
+        const uint32_t g = active ? b.cperm[q] : 0u;
+        by_scene<kB>((kB && active) ? b.sid[g] : 0u, active, [&](uint32_t sc) {
+            const Grid G = SC[sc].G;
+            const PassTerms<kPass> ps(b, SC[sc].P, g);
+            auto elem = [&](uint32_t j) { return ps.elem(j); };
+            auto term = [&](const El2& e) { return ps.template term<false>(e); };
+            const uint32_t key = key27(ps.key, c, G);
+            const F3 cs = any_big ? sum_cell<true>(cell_view(b), key, ps.self, ps.cut2, elem, term)
+                                  : sum_cell<false>(cell_view(b), key, ps.self, ps.cut2, elem, term);
+            b.part[((size_t)k * 27u + c) * 64u + lane] = make_float4(cs.x, cs.y, cs.z, 0.f);
         });
     }
 }
@@ -2440,24 +2483,28 @@ hipError_t step_seq(const Bufs& b, const Scenes<kB>& SC, const Tuning& T, float*
         });
     }
     // the overflow positions' per-cell partials, before each pass that adds them
-    const dim3 ovf_grid(kOvfBlocks);
+    auto ovf_part = [&](auto pass) {
+        hipLaunchKernelGGL((k_ovf_part<kB, pass()>), dim3(kOvfBlocks), dim3(256), 0, s, b, SC);
+        if (std::min(ceil_div(n, 64u), b.ovf_max) > kOvfRows)
+            hipLaunchKernelGGL((k_ovf_part_many<kB, pass()>), dim3(kOvfBlocks), dim3(256), 0, s, b, SC);
+    };
     if (any_vort) {
         {
             Mark m(tm, s, K_VORT);
-            hipLaunchKernelGGL((k_ovf_part<kB, PASS_VORT>), ovf_grid, dim3(256), 0, s, b, SC);
+            ovf_part(std::integral_constant<int, PASS_VORT>{});
             by_lanes(n, [&](auto L) {
                 hipLaunchKernelGGL((k_vort<kB, L()>), lane_grid(n, L()), dim3(kBlock), 0, s, b, SC);
             });
         }
         Mark m(tm, s, K_CONFINE);
-        hipLaunchKernelGGL((k_ovf_part<kB, PASS_CONF>), ovf_grid, dim3(256), 0, s, b, SC);
+        ovf_part(std::integral_constant<int, PASS_CONF>{});
         by_lanes(n, [&](auto L) {
             hipLaunchKernelGGL((k_confine<kB, L()>), lane_grid(n, L()), dim3(kBlock), 0, s, b, SC);
         });
     }
     if (any_xsph) {
         Mark m(tm, s, K_XSPH_OUT);
-        hipLaunchKernelGGL((k_ovf_part<kB, PASS_XSPH>), ovf_grid, dim3(256), 0, s, b, SC);
+        ovf_part(std::integral_constant<int, PASS_XSPH>{});
         by_lanes(n, [&](auto L) {
             hipLaunchKernelGGL((k_xsph_out<kB, L()>), lane_grid(n, L()), dim3(kBlock), 0, s, b, SC, x, v);
         });
