@@ -97,12 +97,19 @@ def parse():
     ap.add_argument("--adjoint-only", action="store_true",
                     help="run only the differentiable workload (for profiling it alone)")
     ap.add_argument("--cpu-seconds", type=float, default=15.0, help="CPU baseline budget (0: skip)")
-    ap.add_argument("--tile-cap", type=int, default=None, help="LDS tile (particles); default: autotuned")
+    ap.add_argument("--tile-cap", type=int, default=None, help="neighbourhood above which a work unit counts as slow (particles); default: autotuned")
     ap.add_argument("--unit-width", type=int, default=16)
     ap.add_argument("--calibrate-copy-mb", type=int, default=0,
                     help="finish with a plain device copy of this many MiB (a known-size kernel for "
                          "scaling hardware byte counters)")
     return ap.parse_args()
+
+
+def profile_name(workload: str) -> str:
+    """The name of a workload's counter profiles: '<workload>_groups' where one of
+    the current kernels (lists and sums by groups of lanes) stands beside an older."""
+    newer = os.path.join(ROOT, "profiles", f"valu_pbf_step_{workload}_groups.txt")
+    return f"{workload}_groups" if os.path.exists(newer) else workload
 
 
 def traffic_from_profiles(kernel: str, workload: str):
@@ -640,7 +647,7 @@ def main():
             "iterations": I,
             "tuning": r["tuning"],
         },
-        "roofline": roofline(r["kernels"], n, C, tiles, sc.name),
+        "roofline": roofline(r["kernels"], n, C, tiles, profile_name(sc.name)),
         "step_roofline": {
             "alg_bytes_per_step": sb,
             "alg_bytes_per_particle": STEP_BYTES_PER_PARTICLE(I),
@@ -667,7 +674,7 @@ def main():
             "ms_per_step": round(ms8, 5),
             "iterations": s8.iters,
             "tuning": r8["tuning"],
-            "roofline": roofline(r8["kernels"], s8.n, s8.cells, t8, s8.name),
+            "roofline": roofline(r8["kernels"], s8.n, s8.cells, t8, profile_name(s8.name)),
             "step_roofline_frac": round(sb8 / (ms8 * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
             "kernels": kernel_report(r8["kernels"], s8.n, s8.cells, t8, min(a.kernel_steps, 5)),
             "state": {k: r8["stats"][k] for k in ("units", "slow_units", "max_tile", "truncated", "list_overflow",

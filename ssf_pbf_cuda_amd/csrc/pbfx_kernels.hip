@@ -2049,7 +2049,7 @@ __global__ __launch_bounds__(256) void k_ovf_part(Bufs b, Scenes<kB> SC) {
 // IEEE root without asking whether the wave's pairs allow the short one.  Chained
 // steps of the 8M double dam, 30 to 35 (2.0M particles overflow) 237 ms a step, by
 // rows 300, with the short root 261; steps 0 to 15 alike.  The 1M dam, which has at
-// most 16,384 blocks, is the slower for it (steps 0 to 60 10.7 ms against 8.2).
+// most 16,384 blocks, is the slower for it (steps 0 to 60 10.5 ms against 8.1).
 template <bool kB, int kPass>
 __global__ __launch_bounds__(256) void k_ovf_part_many(Bufs b, Scenes<kB> SC) {
     const uint32_t ns = min(b.ctr[CTR_OVF], b.ovf_max);
