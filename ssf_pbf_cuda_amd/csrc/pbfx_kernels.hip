@@ -1095,8 +1095,12 @@ __device__ __forceinline__ uint32_t group_list(GroupShared& S, const Grid& G, Ce
         if (n > lim) break;
     }
     if (kFinal && n > lim) return n;
-    // the rest of the last word, which the walks load and do not use: a record at hand
-    if (l < 3u) keep[min(n, lim) + l] = slot;
+    // The rest of the last word, whose records the walks load and do not use: the
+    // own one for the search, where the slots of a wave are neighbours; for the final
+    // lists, whose positions' slots are scattered, slot 0, one line for all lanes (with
+    // the own record there the three passes took 44 / 53 / 59 us on the 1M dam, with
+    // this 39 / 43 / 53, and 655 / 858 / 869 us on the 8M double dam, now 606 / 788 / 809).
+    if (l < 3u) keep[min(n, lim) + l] = kFinal ? 0u : slot;
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     const uint32_t nw = (min(n, lim) + 3u) / 4u;
     for (uint32_t w = l; w < nw; w += kGroup)
