@@ -81,13 +81,12 @@ struct BigSeg {
 };
 constexpr uint32_t kFinalK = 64;          // stored in-range pairs per particle for the final passes
 // Final-pass particles with more than kFinalK pairs (piles) get their 27
-// per-cell partial sums computed in parallel before each pass (kOvfBlocks
-// workgroups), by block of 64 consecutive final-order positions: a block
+// per-cell partial sums computed in parallel before each pass (k_ovf_part),
+// by block of 64 consecutive final-order positions: a block
 // holding such a particle takes one of ovf_max slots (every block can have one
 // in a context; the allocation-free step has kStaticOvfSlots), and its
 // partials are stored slot by slot, cell by cell, 64 lanes a row.  A block
 // that finds no slot left sums its cells one after another in the pass.
-constexpr uint32_t kOvfBlocks = 2048;
 constexpr uint32_t kNoSlot = 0xFFFFFFFFu;       // oslot: no particle of the block overflowed (yet)
 constexpr uint32_t kPendingSlot = 0xFFFFFFFEu;  // oslot: being allocated (never seen across kernels)
 constexpr uint32_t kFullSlot = 0xFFFFFFFDu;     // oslot: no slot was left

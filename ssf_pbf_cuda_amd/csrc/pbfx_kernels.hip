@@ -1894,8 +1894,6 @@ __device__ __forceinline__ F3 xsph_pair(F3 self, F3 selfv, F3 pj, F3 vj, float i
 // The three final passes as (elements, pair term, support) for the particle
 // at slot g: the list walk, the direct sum, the per-cell partials and their
 // combination all evaluate a pass through these.
-// Blocks with overflowing positions up to which k_ovf_part sums their cells by rows.
-constexpr uint32_t kOvfRows = 20480;
 enum FinalPass : int { PASS_VORT = 0, PASS_CONF = 1, PASS_XSPH = 2 };
 
 template <int kPass>
@@ -2008,61 +2006,74 @@ __device__ __forceinline__ F3 pass_sum(const Bufs& b, const Grid& G, const Pass&
 }
 
 
-// Per-cell partials of pass kPass for the overflow slots.  A wave task is
-// (slot k, cell c, four consecutive positions of the slot's block): row r sums
-// cell c of the 27 around final-order position 64 * ovf[k] + 4 * sub + r, when
-// that position overflowed, in slot order (sum_cell_row) into
-// part[(k * 27 + c) * 64 + 4 * sub + r].  Consecutive tasks share a cell index,
-// so a workgroup's rows mostly scan the same cell, and the pass reads each row
-// of 64 whole.
+// Per-cell partials of pass kPass for the overflow slots, in one of two forms.
 //
-// A cell of a pile is one serial sum of thousands of terms, whose length set the
-// launch's time while the chip idled (a tenth of the VALU issue) when a thread
-// did it: 139 us a launch (vorticity) over the 40 chained steps of the 32k dam and
-// 1.49 ms over the first ten of the 1M dam; by rows 48 us and 0.40 ms.  Adding the
-// terms on every lane doubles the work, though: with more than kOvfRows blocks,
-// whose cells fill the chip a thread each, k_ovf_part_many does them.
+// Up to kOvfRows overflowing particles a wave task is (slot k, cell c, four consecutive positions
+// of the slot's block): row r sums cell c of the 27 around final-order position
+// 64 * ovf[k] + 4 * sub + r, when that position overflowed, in slot order
+// (sum_cell_row) into part[(k * 27 + c) * 64 + 4 * sub + r].  Consecutive tasks
+// share a cell index, so a workgroup's rows mostly scan the same cell, and the
+// pass reads each row of 64 whole.  A cell of a pile is one serial sum of
+// thousands of terms, whose length sets the time as long as few are under way
+// when a thread does it.
+//
+// Above, a wave task is (slot k, cell c), lane l summing the cell for position
+// 64 * ovf[k] + l: adding the terms on every lane doubles the work, which counts
+// once there are cells enough.  Few candidates of such piles are pairs, so the
+// terms take the IEEE root without asking whether the wave's pairs allow the short
+// one (143 against 153 ms for the three sums of a step of the 8M double dam, steps 30
+// to 35).
+//
+// The line was measured on every step of the chained 1M, 2M, 4M and 8M dams, time
+// of the rows over time of the threads by overflowing particles: 0.30 up to 50,000,
+// 0.45 up to 200,000, 0.67 up to 350,000, 0.87 up to 600,000, 0.98 up to 700,000, 1.17
+// up to 800,000, 1.3 up to 2,000,000, 1.7 above.  (By slots it is blurred: in a block
+// with few overflowing particles the threads idle and the rows do not.)
+//
+// The tasks differ by a thousand times, and the heavy ones lie together in ovf, so
+// the launch has many times the workgroups that fit the chip (ovf_blocks), which
+// the hardware hands out as others end.  With the 2,048 that fit, each wave going
+// round them in a fixed order, the three sums of a step took 652 ms on the 8M
+// double dam, steps 20 to 25, and 14.5 ms on the 1M dam, steps 80 to 100; with
+// 32,768 and 8,192 workgroups 419 and 12.0.
+constexpr uint32_t kOvfRows = 655360;
+
+// Positions of the step whose final list overflowed, from the statistics the list
+// builds left.
+__device__ __forceinline__ uint32_t overflowing(const uint32_t* __restrict__ ctr) {
+    static_assert(kStatRep == 64, "a lane reads a copy");
+    uint32_t v = ctr[CTR_NUM * (1u + lane_id()) + CTR_LISTOVF];
+    for (int d = 32; d > 0; d >>= 1) v += (uint32_t)__shfl_xor((int)v, d, 64);
+    return v;
+}
+
 template <bool kB, int kPass>
 __global__ __launch_bounds__(256) void k_ovf_part(Bufs b, Scenes<kB> SC) {
     const uint32_t ns = min(b.ctr[CTR_OVF], b.ovf_max);
-    if (ns == 0u || ns > kOvfRows) return;  // uniform over the grid
-    const uint32_t nl = b.offset[b.CT], lane = lane_id(), l = lane & 15u;
-    const bool any_big = big_cells(b);
-    const uint64_t ntask = (uint64_t)ns * (27u * 16u);
-    const uint32_t w0 = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-    const uint32_t nw = (gridDim.x * blockDim.x) >> 6;
-    for (uint64_t t = w0; t < ntask; t += nw) {
-        const uint32_t kc = (uint32_t)(t >> 4), k = kc / 27u, c = kc - k * 27u;
-        const uint32_t at = ((uint32_t)t & 15u) * 4u + (lane >> 4);  // position in the block
-        const uint32_t q = b.ovf[k] * 64u + at;
-        const bool active = q < nl && b.fcnt[q] == kFinalK + 1u;
-        if (!__any(active)) continue;
-        const uint32_t g = active ? b.cperm[q] : 0u;
-        by_scene<kB>((kB && active) ? b.sid[g] : 0u, active, [&](uint32_t sc) {
-            const PassTerms<kPass> ps(b, SC[sc].P, g);
-            const F3 cs = any_big ? sum_cell_row<true>(cell_view(b), SC[sc].G, ps, c, l)
-                                  : sum_cell_row<false>(cell_view(b), SC[sc].G, ps, c, l);
-            if (l == 0u) b.part[((size_t)k * 27u + c) * 64u + at] = make_float4(cs.x, cs.y, cs.z, 0.f);
-        });
-    }
-}
-
-// The same when more than kOvfRows blocks overflowed, a thread per (position,
-// cell): a wave task is (slot k, cell c), lane l summing the cell for position
-// 64 * ovf[k] + l.  Few candidates of such piles are pairs, so the terms take the
-// IEEE root without asking whether the wave's pairs allow the short one.  Chained
-// steps of the 8M double dam, 30 to 35 (2.0M particles overflow) 237 ms a step, by
-// rows 300, with the short root 261; steps 0 to 15 alike.  The 1M dam, which has at
-// most 16,384 blocks, is the slower for it (steps 0 to 60 10.5 ms against 8.1).
-template <bool kB, int kPass>
-__global__ __launch_bounds__(256) void k_ovf_part_many(Bufs b, Scenes<kB> SC) {
-    const uint32_t ns = min(b.ctr[CTR_OVF], b.ovf_max);
-    if (ns <= kOvfRows) return;  // uniform over the grid
+    if (ns == 0u) return;  // uniform over the grid
     const uint32_t nl = b.offset[b.CT], lane = lane_id();
     const bool any_big = big_cells(b);
-    const uint32_t ntask = ns * 27u;
     const uint32_t w0 = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
     const uint32_t nw = (gridDim.x * blockDim.x) >> 6;
+    if (ns <= kOvfRows / 64u || overflowing(b.ctr) <= kOvfRows) {
+        const uint32_t ntask = ns * (27u * 16u), l = lane & 15u;
+        for (uint32_t t = w0; t < ntask; t += nw) {
+            const uint32_t kc = t >> 4, k = kc / 27u, c = kc - k * 27u;
+            const uint32_t at = (t & 15u) * 4u + (lane >> 4);  // position in the block
+            const uint32_t q = b.ovf[k] * 64u + at;
+            const bool active = q < nl && b.fcnt[q] == kFinalK + 1u;
+            if (!__any(active)) continue;
+            const uint32_t g = active ? b.cperm[q] : 0u;
+            by_scene<kB>((kB && active) ? b.sid[g] : 0u, active, [&](uint32_t sc) {
+                const PassTerms<kPass> ps(b, SC[sc].P, g);
+                const F3 cs = any_big ? sum_cell_row<true>(cell_view(b), SC[sc].G, ps, c, l)
+                                      : sum_cell_row<false>(cell_view(b), SC[sc].G, ps, c, l);
+                if (l == 0u) b.part[((size_t)k * 27u + c) * 64u + at] = make_float4(cs.x, cs.y, cs.z, 0.f);
+            });
+        }
+        return;
+    }
+    const uint32_t ntask = ns * 27u;
     for (uint32_t t = w0; t < ntask; t += nw) {
         const uint32_t k = t / 27u, c = t - k * 27u;
         const uint32_t q = b.ovf[k] * 64u + lane;
@@ -2351,6 +2362,10 @@ void by_width(uint32_t cap, F&& f) {
 uint32_t stat_blocks(uint32_t n) { return std::min(64u, 1u + ceil_div(n, 4096u)); }
 // workgroups of the big-cell list builds (a loop over 32 particles each)
 dim3 big_grid(uint32_t n) { return dim3(std::min(4096u, ceil_div(n, kGroups))); }
+// Workgroups of k_ovf_part: at least what fills the chip, and one for every two
+// blocks of positions up to 32,768 (where no position overflows, a launch takes 4.6 us
+// with 2,048 or 8,192 workgroups and 8.3 with 32,768).
+uint32_t ovf_blocks(uint32_t n) { return std::min(32768u, std::max(2048u, n / 128u)); }
 // Tiles up to which a scan needs no launch for the tile totals (the last workgroup
 // then reads 8 x 4096 counts; a step of 10,000 particles over 8 tiles 97 us, with
 // the launch 101, of 960 over 4 tiles 150 and 155; the same at 16 tiles), and up to
@@ -2488,9 +2503,7 @@ hipError_t step_seq(const Bufs& b, const Scenes<kB>& SC, const Tuning& T, float*
     }
     // the overflow positions' per-cell partials, before each pass that adds them
     auto ovf_part = [&](auto pass) {
-        hipLaunchKernelGGL((k_ovf_part<kB, pass()>), dim3(kOvfBlocks), dim3(256), 0, s, b, SC);
-        if (std::min(ceil_div(n, 64u), b.ovf_max) > kOvfRows)
-            hipLaunchKernelGGL((k_ovf_part_many<kB, pass()>), dim3(kOvfBlocks), dim3(256), 0, s, b, SC);
+        hipLaunchKernelGGL((k_ovf_part<kB, pass()>), dim3(ovf_blocks(n)), dim3(256), 0, s, b, SC);
     };
     if (any_vort) {
         {
