@@ -875,13 +875,7 @@ __device__ void flush_tally(uint32_t* __restrict__ ctr_base, const Tally& t) {
 constexpr uint32_t kDeferred = 0xFFFFFFFFu;  // a group's count when it left its list to a wave
 
 // ------------------------------------------------- lists by groups of eight
-// Key of cell c (0..26, in z,y,x order) of the 27 around grid position gp.
-__device__ __forceinline__ uint32_t cell27(const int gp[3], uint32_t c, const Grid& G) {
-    const int dz = (int)(c / 9u) - 1, q = (int)(c % 9u);
-    return scene_key(gp[0] + (q % 3) - 1, gp[1] + (q / 3) - 1, gp[2] + dz, G);
-}
-
-// The same around the cell of key `key`.
+// Key of cell c (0..26, in z,y,x order) of the 27 around the cell of key `key`.
 __device__ __forceinline__ uint32_t key27(uint32_t key, uint32_t c, const Grid& G) {
     const uint32_t k = key - G.base, dz = c / 9u, q = c % 9u;
     const uint32_t x = (k + q % 3u - 1u) & (G.gx - 1u), y = ((k >> G.lgx) + q / 3u - 1u) & (G.gy - 1u),
@@ -1526,18 +1520,6 @@ __device__ __forceinline__ F3 sum_cell(CellView b, uint32_t key, F3 self, float 
     return cs;
 }
 
-// Direct sum over the 27 cells from global memory, for particles whose list
-// overflowed: the cells' partial sums added in z,y,x order.
-template <bool kBig, class ElemF, class TermF>
-__device__ __forceinline__ F3 sum27_global(const Grid& G, CellView b, F3 self, float cut2, ElemF&& elem,
-                                           TermF&& term) {
-    int gp[3];
-    grid_pos(self, G.cw, gp);
-    F3 sum = mk3(0.f, 0.f, 0.f);
-    for (uint32_t c = 0; c < 27u; ++c) acc(sum, sum_cell<kBig>(b, cell27(gp, c, G), self, cut2, elem, term));
-    return sum;
-}
-
 // Whether the final-cell run of slot g is too sparse for a unit (fewer than
 // kSparse particles).
 __device__ __forceinline__ bool sparse_run(const Bufs& b, uint32_t lgrun, uint32_t g) {
@@ -1933,12 +1915,12 @@ struct PassTerms {
 };
 
 // Partial sum of cell c (0..26) of the 27 around the pass particle's final
-// cell, by a row of 16 lanes: 16 candidates at a time, a lane each, and the
-// terms of those in range added in slot order by every lane (the others add
-// +0), as sum_cell adds them; the next candidates are loaded while one step is
-// added.  Called by all lanes of the row.
-template <bool kBig, class Pass>
-__device__ __forceinline__ F3 sum_cell_row(CellView b, const Grid& G, const Pass& ps, uint32_t c, uint32_t l) {
+// cell, by a group of L lanes (l: this lane): L candidates at a time, a lane
+// each, and the terms of those in range added in slot order by every lane (the
+// others add +0), as sum_cell adds them; the next candidates are loaded while one
+// step is added.  Called by all lanes of the group.
+template <bool kBig, int L, class Pass>
+__device__ __forceinline__ F3 sum_cell_lanes(CellView b, const Grid& G, const Pass& ps, uint32_t c, uint32_t l) {
     const uint32_t key = key27(ps.key, c, G);
     const uint32_t st = b.offset[key], n = b.offset[key + 1] - st;
     float cs[3] = {0.f, 0.f, 0.f};
@@ -1959,22 +1941,40 @@ __device__ __forceinline__ F3 sum_cell_row(CellView b, const Grid& G, const Pass
             return kBig && via ? b.aux[st + u] : st + u;
         };
         El2 el = ps.elem(slot(p0 + l));
-        uint32_t jn = slot(p0 + 16u + l);
-        for (uint32_t p = p0; p < p1; p += 16u) {
+        uint32_t jn = slot(p0 + (uint32_t)L + l);
+        for (uint32_t p = p0; p < p1; p += (uint32_t)L) {
             const El2 nx = ps.elem(jn);
-            jn = slot(p + 32u + l);
+            jn = slot(p + 2u * (uint32_t)L + l);
             const F3 d = f3of(el.p) - ps.self;
             const bool in = p + l < p1 && !(glm_dot(d, d) > ps.cut2);
             if (__builtin_amdgcn_ballot_w64(in)) {
                 F3 t = mk3(0.f, 0.f, 0.f);
                 if (in) t = ps.term(el);
                 const float v[3] = {t.x, t.y, t.z};
-                add_lanes<16>(cs, v);
+                add_lanes<L>(cs, v);
             }
             el = nx;
         }
     }
     return mk3(cs[0], cs[1], cs[2]);
+}
+
+// Direct sum over the 27 cells, for an overflowing position whose block has no
+// overflow slot (only in the allocation-free step, which has 64): the cells' partial
+// sums added in z,y,x order, each by the pass's own L lanes.  With every lane adding
+// the whole sum a static step of 12,000 particles in 3x3x3 cells took 6.2 ms (12,000
+// and 30,000 of about 30 a cell 0.65 and 0.68), now 1.6 (0.28 and 0.40).
+template <bool kBig, int L, class Pass>
+__device__ __forceinline__ F3 sum27(const Bufs& b, const Grid& G, const Pass& ps, uint32_t l) {
+    F3 sum = mk3(0.f, 0.f, 0.f);
+    for (uint32_t c = 0; c < 27u; ++c) {
+        if constexpr (L > 1)
+            acc(sum, sum_cell_lanes<kBig, L>(cell_view(b), G, ps, c, l));
+        else
+            acc(sum, sum_cell<kBig>(cell_view(b), key27(ps.key, c, G), ps.self, ps.cut2,
+                                    [&](uint32_t j) { return ps.elem(j); }, [&](const El2& e) { return ps.term(e); }));
+    }
+    return sum;
 }
 
 // The pass's sum for final-order position q with stored count n: the list
@@ -1997,8 +1997,7 @@ __device__ __forceinline__ F3 pass_sum(const Bufs& b, const Grid& G, const Pass&
     }
     const uint32_t k = b.oslot[q >> 6];
     if (k >= b.ovf_max)
-        return big_cells(b) ? sum27_global<true>(G, cell_view(b), ps.self, ps.cut2, elem, term)
-                            : sum27_global<false>(G, cell_view(b), ps.self, ps.cut2, elem, term);
+        return big_cells(b) ? sum27<true, L>(b, G, ps, l) : sum27<false, L>(b, G, ps, l);
     const float4* __restrict__ pk = b.part + (size_t)k * 27u * 64u + (q & 63u);
     F3 sum = mk3(0.f, 0.f, 0.f);
     for (uint32_t c = 0; c < 27u; ++c) acc(sum, f3of(pk[c * 64u]));
@@ -2011,7 +2010,7 @@ __device__ __forceinline__ F3 pass_sum(const Bufs& b, const Grid& G, const Pass&
 // Up to kOvfRows overflowing particles a wave task is (slot k, cell c, four consecutive positions
 // of the slot's block): row r sums cell c of the 27 around final-order position
 // 64 * ovf[k] + 4 * sub + r, when that position overflowed, in slot order
-// (sum_cell_row) into part[(k * 27 + c) * 64 + 4 * sub + r].  Consecutive tasks
+// (sum_cell_lanes) into part[(k * 27 + c) * 64 + 4 * sub + r].  Consecutive tasks
 // share a cell index, so a workgroup's rows mostly scan the same cell, and the
 // pass reads each row of 64 whole.  A cell of a pile is one serial sum of
 // thousands of terms, whose length sets the time as long as few are under way
@@ -2066,8 +2065,8 @@ __global__ __launch_bounds__(256) void k_ovf_part(Bufs b, Scenes<kB> SC) {
             const uint32_t g = active ? b.cperm[q] : 0u;
             by_scene<kB>((kB && active) ? b.sid[g] : 0u, active, [&](uint32_t sc) {
                 const PassTerms<kPass> ps(b, SC[sc].P, g);
-                const F3 cs = any_big ? sum_cell_row<true>(cell_view(b), SC[sc].G, ps, c, l)
-                                      : sum_cell_row<false>(cell_view(b), SC[sc].G, ps, c, l);
+                const F3 cs = any_big ? sum_cell_lanes<true, 16>(cell_view(b), SC[sc].G, ps, c, l)
+                                      : sum_cell_lanes<false, 16>(cell_view(b), SC[sc].G, ps, c, l);
                 if (l == 0u) b.part[((size_t)k * 27u + c) * 64u + at] = make_float4(cs.x, cs.y, cs.z, 0.f);
             });
         }
