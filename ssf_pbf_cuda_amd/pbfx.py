@@ -284,7 +284,7 @@ class Solver:
                                            pp.shape[0]), "pbfx_set_boundary")
 
     def autotune(self, x, v, num: int, lo, hi, iters: int, x_scratch, v_scratch, in_offsets=None, stream=None):
-        """Times each (tile_cap, unit_width) candidate on scratch copies of x, v and keeps the fastest."""
+        """Times each unit width on scratch copies of x, v and keeps the fastest; (tile_cap as set, unit width)."""
         t, w = ctypes.c_uint32(), ctypes.c_uint32()
         _check(self._lib.pbfx_autotune(self._ctx, _ptr(x), _ptr(v), int(num), _ptr(in_offsets), _f3(lo), _f3(hi),
                                        int(iters), _ptr(x_scratch), _ptr(v_scratch), ctypes.byref(t),
