@@ -427,8 +427,9 @@ __device__ __forceinline__ void sum_pairs(const uint32_t* __restrict__ nl, uint3
 // each.  q lies within 1.5 units in the last place of the quotient, so the
 // corrected value is off by at most 4 * 2^-25 units before it is rounded; the
 // quotients that lie that close to a midpoint (a 2^k - (2Q+1) s = N with
-// |N| <= 16, all 93 million pairs of significands) were compared with the IEEE
-// division one by one.  Valid while nothing underflows: div3_plain.
+// |N| <= 16, all 93 million pairs of significands) are compared with the IEEE
+// division one by one in tests/cpp/div_midpoints.cpp.  Valid while nothing
+// underflows: wave_plain_div.
 __device__ __forceinline__ F3 div3_inv(F3 a, float s, float inv) {
     const F3 q = mk3(a.x * inv, a.y * inv, a.z * inv);
     return mk3(__builtin_fmaf(__builtin_fmaf(-q.x, s, a.x), inv, q.x),
