@@ -124,6 +124,9 @@ enum Ctr : int {
 };
 constexpr uint32_t kStatRep = 64;                           // copies of the statistics counters
 constexpr uint32_t kCtrWords = CTR_NUM * (1 + kStatRep);    // ctr[0..CTR_NUM): allocation counters
+// Particles of the largest big cell (0: none), in a word of the first copy: the
+// allocation counters have no copies.
+constexpr uint32_t kCtrMostCell = CTR_NUM + CTR_BIGCELLS;
 
 // One scene's hash grid.  Scenes occupy consecutive ranges of one cell-key
 // space: cell (x, y, z) of a scene has key base + (z*gy + y)*gx + x.

@@ -669,10 +669,12 @@ __global__ __launch_bounds__(1024) void k_big_seg(Bufs b, Scenes<kB> SC) {
     __shared__ float red[16][8];
     const uint32_t lane = lane_id(), wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
     const uint32_t nb0 = b.ctr[CTR_BIGCELLS], nh = b.ctr[CTR_HUGECELLS];
+    uint32_t most = 0;
     for (uint32_t it = blockIdx.x; it < nh + nb0; it += gridDim.x) {
         uint32_t c;
         const uint32_t d = big_item(b, it, nh, c);
         const uint32_t o0 = b.offset[c], n = b.offset[c + 1] - o0;
+        most = max(most, n);
         const Grid G = SC[scene_index<kB>(b.kbase, b.nscenes, c)].G;
         for (uint32_t k = threadIdx.x; k < kCodes; k += blockDim.x) cnt[k] = 0u;
         __syncthreads();
@@ -743,6 +745,7 @@ __global__ __launch_bounds__(1024) void k_big_seg(Bufs b, Scenes<kB> SC) {
         if (threadIdx.x == 0) D.nseg = ns;
         __syncthreads();
     }
+    if (threadIdx.x == 0 && most) atomicMax(&b.ctr[kCtrMostCell], most);
 }
 
 // What a scan of big cell D (n particles) for a particle at `self` must
@@ -2007,43 +2010,47 @@ __device__ __forceinline__ F3 pass_sum(const Bufs& b, const Grid& G, const Pass&
 
 // Per-cell partials of pass kPass for the overflow slots, in one of two forms.
 //
-// Up to kOvfRows overflowing particles a wave task is (slot k, cell c, four consecutive positions
-// of the slot's block): row r sums cell c of the 27 around final-order position
+// By rows: a wave task is (slot k, cell c, four consecutive positions of the slot's
+// block), row r summing cell c of the 27 around final-order position
 // 64 * ovf[k] + 4 * sub + r, when that position overflowed, in slot order
 // (sum_cell_lanes) into part[(k * 27 + c) * 64 + 4 * sub + r].  Consecutive tasks
 // share a cell index, so a workgroup's rows mostly scan the same cell, and the
-// pass reads each row of 64 whole.  A cell of a pile is one serial sum of
-// thousands of terms, whose length sets the time as long as few are under way
-// when a thread does it.
+// pass reads each row of 64 whole.
 //
-// Above, a wave task is (slot k, cell c), lane l summing the cell for position
-// 64 * ovf[k] + l: adding the terms on every lane doubles the work, which counts
-// once there are cells enough.  Few candidates of such piles are pairs, so the
-// terms take the IEEE root without asking whether the wave's pairs allow the short
-// one (143 against 153 ms for the three sums of a step of the 8M double dam, steps 30
-// to 35).
+// By threads: a wave task is (slot k, cell c), lane l summing the cell for position
+// 64 * ovf[k] + l.  Few candidates of large piles are pairs, so the terms take the
+// IEEE root without asking whether the wave's pairs allow the short one (143 against
+// 153 ms for the three sums of a step of the 8M double dam, steps 30 to 35).
 //
-// The line was measured on every step of the chained 1M, 2M, 4M and 8M dams, time
-// of the rows over time of the threads by overflowing particles: 0.30 up to 50,000,
-// 0.45 up to 200,000, 0.67 up to 350,000, 0.87 up to 600,000, 0.98 up to 700,000, 1.17
-// up to 800,000, 1.3 up to 2,000,000, 1.7 above.  (By slots it is blurred: in a block
-// with few overflowing particles the threads idle and the rows do not.)
+// A cell of a pile is one serial sum of thousands of terms, which sets the time of the
+// threads until there are sums enough to hide it; by rows it is 16 times shorter, but
+// adding the terms on every lane doubles the work.  So the threads take over when the
+// overflowing particles are more than kOvfCell times the largest cell, or more than
+// kOvfRows.  Measured, time of the rows over time of the threads:
+//   fluid of 20 to 1,000 particles a cell throughout, by overflowing particles over
+//   the largest cell (64 at least): 0.8 at 25, 1.0 at 50, 1.15 at 100, 1.4 at 200, 2 at 2,000;
+//   a dam of 200,000 particles with a weak tensile term, falling together: 1.0 at 200, 1.2
+//   at 300; with a strong one (largest cells of 1,000): 0.45 at 25, 0.6 at 40;
+//   chained 1M to 8M dams (cells of 12,000 to 300,000: at most 41), by overflowing
+//   particles: 0.3 up to 50,000, 0.45 up to 200,000, 0.67 up to 350,000, 0.87 up to
+//   600,000, 0.98 up to 700,000, 1.17 up to 800,000, 1.3 up to 2,000,000, 1.7 above.
 //
-// The tasks differ by a thousand times, and the heavy ones lie together in ovf, so
-// the launch has many times the workgroups that fit the chip (ovf_blocks), which
-// the hardware hands out as others end.  With the 2,048 that fit, each wave going
-// round them in a fixed order, the three sums of a step took 652 ms on the 8M
-// double dam, steps 20 to 25, and 14.5 ms on the 1M dam, steps 80 to 100; with
-// 32,768 and 8,192 workgroups 419 and 12.0.
-constexpr uint32_t kOvfRows = 655360;
+// The tasks differ by a thousand times, so the launch has many times the workgroups
+// that fit the chip (ovf_blocks), which the hardware hands out as others end.  With the
+// 2,048 that fit, each wave going round the tasks in a fixed order, the three sums of a
+// step took 652 ms on the 8M double dam, steps 20 to 25, and 14.5 ms on the 1M dam, steps
+// 80 to 100; with 32,768 and 8,192 workgroups 419 and 12.0.
+constexpr uint32_t kOvfRows = 655360, kOvfCell = 64;
 
-// Positions of the step whose final list overflowed, from the statistics the list
-// builds left.
-__device__ __forceinline__ uint32_t overflowing(const uint32_t* __restrict__ ctr) {
+// Whether the ns slots' cells are summed by threads.  The overflowing positions come
+// from the statistics the list builds left.
+__device__ __forceinline__ bool ovf_by_threads(const uint32_t* __restrict__ ctr, uint32_t ns) {
     static_assert(kStatRep == 64, "a lane reads a copy");
+    const uint64_t line = min((uint64_t)kOvfRows, (uint64_t)kOvfCell * max(kSmallCell, ctr[kCtrMostCell]));
+    if (64ull * ns <= line) return false;
     uint32_t v = ctr[CTR_NUM * (1u + lane_id()) + CTR_LISTOVF];
     for (int d = 32; d > 0; d >>= 1) v += (uint32_t)__shfl_xor((int)v, d, 64);
-    return v;
+    return v > line;
 }
 
 template <bool kB, int kPass>
@@ -2054,7 +2061,7 @@ __global__ __launch_bounds__(256) void k_ovf_part(Bufs b, Scenes<kB> SC) {
     const bool any_big = big_cells(b);
     const uint32_t w0 = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
     const uint32_t nw = (gridDim.x * blockDim.x) >> 6;
-    if (ns <= kOvfRows / 64u || overflowing(b.ctr) <= kOvfRows) {
+    if (!ovf_by_threads(b.ctr, ns)) {
         const uint32_t ntask = ns * (27u * 16u), l = lane & 15u;
         for (uint32_t t = w0; t < ntask; t += nw) {
             const uint32_t kc = t >> 4, k = kc / 27u, c = kc - k * 27u;

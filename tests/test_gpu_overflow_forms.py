@@ -1,8 +1,8 @@
-"""The per-cell sums of blocks with overflowing final lists, on both sides of the
-655,360 overflowing particles at which k_ovf_part goes from rows of 16 lanes to a
-thread per cell: fewer particles than that in all, fewer overflowing ones in more than
-10,240 blocks, and more, without cells of more than 64 particles; and, in a batch, more
-with and without such cells.  Each state must equal the oracle's plain step."""
+"""The per-cell sums of blocks with overflowing final lists, by rows of 16 lanes or
+by threads, on both sides of the lines between the two (overflowing particles above 64
+times the largest cell, which counts as 64 at least, or above 655,360): without cells
+of more than 64 particles, with one, and in a batch.  Each state must equal the
+oracle's plain step."""
 from __future__ import annotations
 
 import dataclasses
@@ -34,26 +34,36 @@ def filled(per_cell, box, seed=3):
     return replace_params(sc, relaxation=1.0e9, scorr_k=1.0e-6)
 
 
-@pytest.mark.parametrize("per_cell,width", [(19, 3.2), (15, 6.4), (30, 3.2)])
-def test_both_forms_without_big_cells(per_cell, width):
-    sc = filled(per_cell, (width, 3.2, 3.2))
+# box, particles of one point, by threads
+CASES = {
+    "few": (30, (0.4, 0.4, 0.4), 0, False),
+    "small_cells": (30, (0.8, 0.8, 0.8), 0, True),
+    "one_larger_cell": (30, (0.8, 0.8, 0.8), 400, False),
+    "many_blocks": (15, (6.4, 3.2, 3.2), 7000, False),
+    "below_the_line": (19, (3.2, 3.2, 3.2), 10500, False),
+    "above_the_line": (30, (3.2, 3.2, 3.2), 16000, True),
+}
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_both_forms(name):
+    per_cell, box, point, threads = CASES[name]
+    sc = filled(per_cell, box)
+    sc.x[:point] = sc.x[0]
     got = gpu_run(sc, with_ns=True)
-    over = got["stats"]["list_overflow"]
-    print(f"{sc.n} particles, {over} overflowing", flush=True)
-    assert np.diff(got["cell_offset"][:-1].astype(np.int64)).max() <= 64
-    if per_cell == 19:
-        assert 0 < over <= sc.n < LINE
-    elif per_cell == 15:
-        assert sc.n > LINE * 1.4 and LINE // 4 < over < LINE
-    else:
-        assert over > LINE
+    over, most = got["stats"]["list_overflow"], np.diff(got["cell_offset"][:-1].astype(np.int64)).max()
+    print(f"{name}: {sc.n} particles, {over} overflowing, cells of up to {most}", flush=True)
+    assert over > 0 and (most > 64) == (point > 0)
+    assert (over > min(LINE, 64 * max(64, most))) == threads
+    if name == "many_blocks":
+        assert sc.n > LINE
     ref = oracle_run(sc)
     assert got["num"] == ref["num"]
     assert bit_mismatches(got["x"], ref["x"]) == 0 and bit_mismatches(got["v"], ref["v"]) == 0
 
 
 @pytest.mark.parametrize("point", [0, 300])
-def test_threads_per_cell_in_a_batch(point):
+def test_threads_in_a_batch(point):
     scs = [filled(30, (3.2, 3.2, 1.6), seed=s) for s in (5, 6)]
     scs.append(scenes.small_dam(12, 10, 8, iters=1))
     if point:
