@@ -276,10 +276,12 @@ typedef struct pbfx_stats {
 /* Statistics of the last step (synchronises `stream`). */
 pbfx_status pbfx_get_stats(pbfx_ctx* ctx, void* stream, pbfx_stats* out);
 
-/* Tuning knobs.  tile_cap: particles of a work unit's neighbourhood above
- * which a run of cells is split into narrower units, and a unit is counted as
- * slow (statistics; default 2048, max 4096); unit_width: cells per run along x
- * (power of two 1..32, default 16), by which the final passes group particles. */
+/* Tuning knobs; no result depends on them.  unit_width: cells per run along x
+ * (power of two 1..32, default 16), by which work units are listed; the final
+ * passes group particles by runs of as many cells, at most eight.  tile_cap
+ * (default 2048, max 4096) moves statistics only: a run whose neighbourhood,
+ * estimated from its mean density, passes three quarters of it is listed as narrower
+ * units, and a unit whose neighbourhood holds more than it is counted as slow. */
 pbfx_status pbfx_set_tuning(pbfx_ctx* ctx, uint32_t tile_cap, uint32_t unit_width);
 
 /* Autotuner: times one step of the given state for every candidate

@@ -282,7 +282,7 @@ __device__ __forceinline__ void for_T(const AdjBufs& a, const Grid& G, F3 p0, co
 }
 
 // Candidate counts of the final passes' sets and of the search cells;
-// particles above kAdjHeavy are flagged and listed for the heavy kernels
+// particles above kAdjHeavy are flagged and listed for the waves (for_roles)
 // (the reverse-list bit is set by k_adj_rev).  Also clears the per-particle
 // shares of the parameter gradients.
 __global__ __launch_bounds__(256) void k_adj_classify(StepTape t, AdjBufs a, Grid G) {
@@ -487,12 +487,10 @@ __global__ __launch_bounds__(256) void k_adj_xsph_own(StepTape t, AdjBufs a, Gri
             sumW += W;
             apos = apos - sc3(pd, gw * k.gamma * dot3(gi, e));
         });
-        if (W > 1) {
-            acc = gsum3<W>(acc);
-            sumW = gsum<W>(sumW);
-            apos = gsum3<W>(apos);
-            if (r.lane) return;
-        }
+        acc = gsum3<W>(acc);
+        sumW = gsum<W>(sumW);
+        apos = gsum3<W>(apos);
+        if (r.lane) return;
         const bool nan = isnan(acc.x) || isnan(acc.y) || isnan(acc.z);
         a.xnan[i] = nan ? 1u : 0u;
         if (nan) return;  // velocity kept: v_out = Vc
@@ -524,11 +522,9 @@ __global__ __launch_bounds__(256) void k_adj_xsph_rev(StepTape t, AdjBufs a, Gri
             avc = avc + sc3(gl, k.gamma * W);
             apos = apos + sc3(pd, gw * k.gamma * dot3(gl, vi - wid(vl)));
         });
-        if (W > 1) {
-            avc = gsum3<W>(avc);
-            apos = gsum3<W>(apos);
-            if (r.lane) return;
-        }
+        avc = gsum3<W>(avc);
+        apos = gsum3<W>(apos);
+        if (r.lane) return;
         st(a.aVc, i, ld(a.aVc, i) + avc);
         st(a.aP, i, ld(a.aP, i) + apos);
     });
@@ -552,10 +548,8 @@ __global__ __launch_bounds__(256) void k_adj_conf_own(StepTape t, AdjBufs a, Gri
             const D3 om = wid(t.OM4[j]);
             eta = eta + sc3(sd.f(), sqrt(dot3(om, om)));
         });
-        if (W > 1) {
-            eta = gsum3<W>(eta);
-            if (r.lane) return;
-        }
+        eta = gsum3<W>(eta);
+        if (r.lane) return;
         const D3 avc = ld(a.aVc, i);
         st(a.aV, i, avc);
         const double nr = sqrt(dot3(eta, eta));
@@ -580,7 +574,7 @@ __global__ __launch_bounds__(256) void k_adj_eta_own(StepTape t, AdjBufs a, Grid
         constexpr int W = decltype(width)::value;
         const uint32_t i = r.i;
         const D3 eb = ld(a.etab, i);
-        if (zero3(eb)) return;  // uniform over a heavy wave
+        if (zero3(eb)) return;  // uniform over the group
         const AdjConst k = adj_const(P);
         const F3 selff = f3of(t.PI[i]);
         const D3 self = wid3(selff);
@@ -591,10 +585,8 @@ __global__ __launch_bounds__(256) void k_adj_eta_own(StepTape t, AdjBufs a, Grid
             const D3 om = wid(t.OM4[j]);
             apos = apos - sc3(sd.H(eb), sqrt(dot3(om, om)));
         });
-        if (W > 1) {
-            apos = gsum3<W>(apos);
-            if (r.lane) return;
-        }
+        apos = gsum3<W>(apos);
+        if (r.lane) return;
         st(a.aP, i, ld(a.aP, i) + apos);
     });
 }
@@ -622,11 +614,9 @@ __global__ __launch_bounds__(256) void k_adj_eta_rev(StepTape t, AdjBufs a, Grid
             mb += dot3(el, sd.f());
             apos = apos + sc3(sd.H(el), wi);
         });
-        if (W > 1) {
-            mb = gsum<W>(mb);
-            apos = gsum3<W>(apos);
-            if (r.lane) return;
-        }
+        mb = gsum<W>(mb);
+        apos = gsum3<W>(apos);
+        if (r.lane) return;
         if (wi > 0.0) st(a.aOm, i, ld(a.aOm, i) + sc3(omi, mb / wi));
         st(a.aP, i, ld(a.aP, i) + apos);
     });
@@ -640,7 +630,7 @@ __global__ __launch_bounds__(256) void k_adj_vort_own(StepTape t, AdjBufs a, Gri
         constexpr int W = decltype(width)::value;
         const uint32_t i = r.i;
         const D3 ab = ld(a.aOm, i);
-        if (zero3(ab)) return;  // uniform over a heavy wave
+        if (zero3(ab)) return;  // uniform over the group
         const AdjConst k = adj_const(P);
         const F3 selff = f3of(t.PI[i]);
         const D3 self = wid3(selff);
@@ -654,11 +644,9 @@ __global__ __launch_bounds__(256) void k_adj_vort_own(StepTape t, AdjBufs a, Gri
             av = av - sc3(cross3(sd.f(), ab), k.beta);
             apos = apos - sd.H(sc3(cross3(ab, e), k.beta));
         });
-        if (W > 1) {
-            av = gsum3<W>(av);
-            apos = gsum3<W>(apos);
-            if (r.lane) return;
-        }
+        av = gsum3<W>(av);
+        apos = gsum3<W>(apos);
+        if (r.lane) return;
         st(a.aV, i, ld(a.aV, i) + av);
         st(a.aP, i, ld(a.aP, i) + apos);
     });
@@ -686,11 +674,9 @@ __global__ __launch_bounds__(256) void k_adj_vort_rev(StepTape t, AdjBufs a, Gri
             av = av + sc3(cross3(sd.f(), al), k.beta);
             apos = apos + sd.H(sc3(cross3(al, e), k.beta));
         });
-        if (W > 1) {
-            av = gsum3<W>(av);
-            apos = gsum3<W>(apos);
-            if (r.lane) return;
-        }
+        av = gsum3<W>(av);
+        apos = gsum3<W>(apos);
+        if (r.lane) return;
         st(a.aV, i, ld(a.aV, i) + av);
         st(a.aP, i, ld(a.aP, i) + apos);
     });
@@ -865,13 +851,11 @@ __global__ __launch_bounds__(256) void k_adj_lam(StepTape t, AdjBufs a, const fl
             const double Wb = -Ab * corr_dW(k, pa.W, sl, si);
             apos = apos - (sc3(pa.H(al), k.beta * A) + sc3(d, Wb * pa.gw));
         }
-        if (W > 1) {
-            sb = gsum<W>(sb);
-            kg2s = gsum<W>(kg2s);
-            kgs = gsum3<W>(kgs);
-            apos = gsum3<W>(apos);
-            if (r.lane) return;
-        }
+        sb = gsum<W>(sb);
+        kg2s = gsum<W>(kg2s);
+        kgs = gsum3<W>(kgs);
+        apos = gsum3<W>(apos);
+        if (r.lane) return;
         // s = C / D, C = beta sum W - 1, D = m2r2 (|sum kg|^2 + sum |kg|^2) + eps
         const double D = k.m2r2 * (dot3(kgs, kgs) + kg2s) + k.relax;
         const double ksb = k.beta * sb / D;
@@ -915,10 +899,8 @@ __global__ __launch_bounds__(256) void k_adj_pos(StepTape t, AdjBufs a, const fl
             if (!pair_adj(d, k, pa)) continue;
             apos = apos - (sc3(d, cl.x * pa.gw) + pa.H(md3(cl.y, cl.z, cl.w) + sc3(pa.kg, g2l)));
         }
-        if (W > 1) {
-            apos = gsum3<W>(apos);
-            if (r.lane) return;
-        }
+        apos = gsum3<W>(apos);
+        if (r.lane) return;
         st(a.aP, i, ld(a.aQ, i) + apos);
     });
 }

@@ -145,7 +145,8 @@ __device__ __forceinline__ uint32_t in_scene(uint32_t x) {
 
 // Runs f(s) for the active lanes, one scene at a time: s is uniform over the
 // wave (read from the first pending lane), so the scene's constants are scalar.
-// f must not use wave-wide operations.  As per-lane values the constants took up
+// Operations across lanes in f see the lanes of that scene only, so lanes that work
+// on one thing (a group of a particle) have to be of one scene.  As per-lane values the constants took up
 // to 70 vector registers a lane (vorticity 128 against 80 of a single scene,
 // XSPH 146 against 78), half the waves in flight: a step of 256 scenes 15.85 ms,
 // now 15.15.

@@ -183,8 +183,9 @@ __global__ __launch_bounds__(1024) void k_scan_tiles(const uint32_t* __restrict_
 // dam).  Listed by the wave that meets a run's first particle, as the reorder
 // and the regrouping's scatter did, it takes thousands, which one address
 // serialises: k_reorder took 101 us on the 1M dam and 756 us on the 8M double
-// dam at uw = 16, now 14 and 148; k_cur_scatter 22 and 338 us, now 15 and 97;
-// the two scans 18 us together, now 23.
+// dam at uw = 16, now 15 and 153; k_cur_scatter 24 and 329 us, now 14 and 138;
+// k_scan_cells 18 and 122 us in its two launches, now 22 and 122, of which the sum
+// before a tile replaces k_scan_tiles up to kPrefixTiles (7 us at 1M).
 enum EmitMode : int { EMIT_NONE = 0, EMIT_SEARCH, EMIT_FINAL };
 struct EmitArgs {
     uint32_t uw, lguw, lgrun, budget;  // lgrun: tile words per run
@@ -1395,10 +1396,12 @@ __global__ __launch_bounds__(256) void k_deltap(Bufs b, Scenes<kB> SC) {
 // the domain -- a corner pile of 7,000 particles on the 1M dam -- is not counted
 // through one contended line; key = run * 4 + copy.  Narrower runs keep
 // neighbours together in the lists and gathers of the final passes, fewer
-// counters are contended: cells per run / counters 16/8, 8/4, 4/4, 1/1 take 1051,
-// 1054, 1065, 1127 us for a step of the 1M dam, 9.09, 8.99, 8.95, 9.33 ms of the
-// 8M double dam, 37.5, 36.7, 35.9, 35.8 ms for ten steps of the wild 1M flow and
-// 16.7, 16.6, 16.4, 16.4 ms for a batch of 256 scenes.  The same
+// counters are contended: cells per run / counters 16/8, 8/4, 4/4, 1/1 take 1023,
+// 1030, 1041, 1102 us for a step of the 1M dam, 8.91, 8.84, 8.79, 9.17 ms of the
+// 8M double dam, 36.3, 35.9, 35.6, 35.7 ms for ten steps of the wild 1M flow and
+// 15.2, 15.0, 14.9, 14.8 ms for a batch of 256 scenes.  Particles sorted by cell inside
+// a run would make the three passes 2.09 ms at 8M instead of 2.20, and 0.14 in a sort of
+// its own for that takes it away again.  The same
 // pass packs each slot's record R = (x*, 0), (v, 0) with
 // v = inv_dt*(x* - x_sorted) (updateVelocityCUDA, pbf_update.cu:25-39), so
 // that a particle visited in run order costs one cache line.  Final cells
@@ -2277,8 +2280,7 @@ __global__ void k_scene_offsets(Bufs b, uint32_t* __restrict__ out) {
     if (s <= b.nscenes) out[s] = b.offset[b.kbase[s]];
 }
 
-// p[0..n) = value (grid-stride): clears counters and flags inside code that a
-// caller may capture in a graph, where memset nodes are avoided.
+// x / y, sqrt(x), fma(x, y, x) and floor(x / y) of each pair, as the device computes them.
 __global__ void k_selftest(const float* __restrict__ a, const float* __restrict__ bb, float* __restrict__ out,
                            uint32_t n) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
