@@ -2029,31 +2029,35 @@ __device__ __forceinline__ F3 pass_sum(const Bufs& b, const Grid& G, const Pass&
 // threads until there are sums enough to hide it; by rows it is 16 times shorter, but
 // adding the terms on every lane doubles the work.  So the threads take over when the
 // overflowing particles are more than kOvfCell times the largest cell, or more than
-// kOvfRows.  Measured, time of the rows over time of the threads:
+// kOvfFull times where their blocks are seven eighths full (in others the lanes of
+// the threads idle), or more than kOvfRows.  Measured, time of the rows over time of the
+// threads:
 //   fluid of 20 to 1,000 particles a cell throughout, by overflowing particles over
 //   the largest cell (64 at least): 0.8 at 25, 1.0 at 50, 1.15 at 100, 1.4 at 200, 2 at 2,000;
+//   full cells of 700 to 15,000 particles in a cube: 1.0 at 8, 1.1 to 1.4 from 24 to 60;
 //   a dam of 200,000 particles with a weak tensile term, falling together: 1.0 at 200, 1.2
-//   at 300; with a strong one (largest cells of 1,000): 0.45 at 25, 0.6 at 40;
-//   chained 1M to 8M dams (cells of 12,000 to 300,000: at most 41), by overflowing
-//   particles: 0.3 up to 50,000, 0.45 up to 200,000, 0.67 up to 350,000, 0.87 up to
-//   600,000, 0.98 up to 700,000, 1.17 up to 800,000, 1.3 up to 2,000,000, 1.7 above.
+//   at 300; with a strong one (blocks half full): 0.45 at 25, 0.6 at 40;
+//   chained 1M to 8M dams (cells of 12,000 to 300,000: at most 41; blocks seven eighths
+//   full: 1.0 to 1.3 at 35), by overflowing particles: 0.3 up to 50,000, 0.45 up to
+//   200,000, 0.67 up to 350,000, 0.87 up to 600,000, 0.98 up to 700,000, 1.17 up to
+//   800,000, 1.3 up to 2,000,000, 1.7 above.
 //
 // The tasks differ by a thousand times, so the launch has many times the workgroups
 // that fit the chip (ovf_blocks), which the hardware hands out as others end.  With the
 // 2,048 that fit, each wave going round the tasks in a fixed order, the three sums of a
 // step took 652 ms on the 8M double dam, steps 20 to 25, and 14.5 ms on the 1M dam, steps
 // 80 to 100; with 32,768 and 8,192 workgroups 419 and 12.0.
-constexpr uint32_t kOvfRows = 655360, kOvfCell = 64;
+constexpr uint32_t kOvfRows = 655360, kOvfCell = 64, kOvfFull = 24;
 
 // Whether the ns slots' cells are summed by threads.  The overflowing positions come
 // from the statistics the list builds left.
 __device__ __forceinline__ bool ovf_by_threads(const uint32_t* __restrict__ ctr, uint32_t ns) {
     static_assert(kStatRep == 64, "a lane reads a copy");
-    const uint64_t line = min((uint64_t)kOvfRows, (uint64_t)kOvfCell * max(kSmallCell, ctr[kCtrMostCell]));
-    if (64ull * ns <= line) return false;
+    const uint64_t cell = max(kSmallCell, ctr[kCtrMostCell]);
+    if (64ull * ns <= min((uint64_t)kOvfRows, kOvfFull * cell)) return false;
     uint32_t v = ctr[CTR_NUM * (1u + lane_id()) + CTR_LISTOVF];
     for (int d = 32; d > 0; d >>= 1) v += (uint32_t)__shfl_xor((int)v, d, 64);
-    return v > line;
+    return v > kOvfRows || v > kOvfCell * cell || (v > kOvfFull * cell && v > 56ull * ns);
 }
 
 template <bool kB, int kPass>

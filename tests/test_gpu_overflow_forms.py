@@ -1,8 +1,8 @@
 """The per-cell sums of blocks with overflowing final lists, by rows of 16 lanes or
 by threads, on both sides of the lines between the two (overflowing particles above 64
-times the largest cell, which counts as 64 at least, or above 655,360): without cells
-of more than 64 particles, with one, and in a batch.  Each state must equal the
-oracle's plain step."""
+times the largest cell, which counts as 64 at least, above 24 times where their blocks of
+64 are full, or above 655,360): without cells of more than 64 particles, with one, with
+full ones, and in a batch.  Each state must equal the oracle's plain step."""
 from __future__ import annotations
 
 import dataclasses
@@ -38,9 +38,11 @@ def filled(per_cell, box, seed=3):
 CASES = {
     "few": (30, (0.4, 0.4, 0.4), 0, False),
     "small_cells": (30, (0.8, 0.8, 0.8), 0, True),
-    "one_larger_cell": (30, (0.8, 0.8, 0.8), 400, False),
+    "one_larger_cell": (30, (0.8, 0.8, 0.8), 700, False),
+    "full_cells": (700, (0.4, 0.4, 0.4), 0, True),
+    "few_full_cells": (700, (0.4, 0.2, 0.2), 0, False),
     "many_blocks": (15, (6.4, 3.2, 3.2), 7000, False),
-    "below_the_line": (19, (3.2, 3.2, 3.2), 10500, False),
+    "below_the_line": (17, (3.2, 3.2, 3.2), 10500, False),
     "above_the_line": (30, (3.2, 3.2, 3.2), 16000, True),
 }
 
@@ -53,8 +55,12 @@ def test_both_forms(name):
     got = gpu_run(sc, with_ns=True)
     over, most = got["stats"]["list_overflow"], np.diff(got["cell_offset"][:-1].astype(np.int64)).max()
     print(f"{name}: {sc.n} particles, {over} overflowing, cells of up to {most}", flush=True)
-    assert over > 0 and (most > 64) == (point > 0)
-    assert (over > min(LINE, 64 * max(64, most))) == threads
+    assert over > 0 and (most > 64) == (point > 0 or per_cell > 64)
+    if name == "full_cells":
+        assert over == sc.n and 24 * most < over <= 64 * most
+    else:
+        assert (over > min(LINE, 64 * max(64, most))) == threads
+        assert threads or over < max(24 * max(64, most), 56 * (sc.n // 64))
     if name == "many_blocks":
         assert sc.n > LINE
     ref = oracle_run(sc)
